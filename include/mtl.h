@@ -274,6 +274,36 @@ int mtl_quant_dequant_sum_fp16(const float* const* parts, int32_t nparts, int64_
                                uint16_t* const* payloads, float* out, mtl_stream_t stream);
 
 /* ------------------------------------------------------------------------
+ * fp32 GEMM of a long prompt's projections on the f16 matrix cores:
+ *   Y[m][n] = sum_k x[m][k] W[n][k] (+ bias[n]),  nn.Linear on M token rows
+ * (model.py:197, 240, 339).  Every operand is split into two f16 parts under a
+ * power of two per row and each product takes three MFMAs with fp32
+ * accumulation: the error against exact arithmetic is below that of an fp32
+ * matrix product (csrc/gemm.hip).  Infinities and NaN come out as an fp32
+ * product gives them.
+ *   x: [M, K], row stride ldx; W: [N, K], row stride ldw; unit column stride.
+ *   y0: [M, N], row stride ldy0 < 2^21; with y1 (not NULL), columns [0,
+ *       n_split) go to y0 and the others to y1 (n_split a multiple of 32).
+ *   ws: mtl_linear_f32_ws_bytes(M, N, K) bytes (the split operands
+ *       and their exponents, about the bytes of x and W), 16-byte aligned.
+ * Outputs must not overlap the inputs or ws.
+ * ---------------------------------------------------------------------- */
+typedef struct {
+    const float* x;
+    const float* W;
+    const float* bias;       /* nullable */
+    float* y0;
+    float* y1;               /* nullable */
+    void* ws;
+    int64_t ws_bytes;
+    int64_t ldx, ldw, ldy0, ldy1;
+    int64_t n_split;
+    int64_t M, N, K;
+} mtl_linear_f32_args;
+int64_t mtl_linear_f32_ws_bytes(int64_t M, int64_t N, int64_t K);
+int mtl_linear_f32(const mtl_linear_f32_args* args, mtl_stream_t stream);
+
+/* ------------------------------------------------------------------------
  * Skinny fp32 GEMM on the matrix cores for the projections of a batched
  * decode step: y = x W^T (+ bias), nn.Linear on [b, K] with b <= 32 tokens --
  * in_proj (model.py:261), out_proj (model.py:293) and the tied lm_head

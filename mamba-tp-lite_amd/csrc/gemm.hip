@@ -1,0 +1,500 @@
+// fp32 GEMM for the projections of a long prompt on the f16 matrix cores
+// (gfx950):   Y[m, n] = sum_k X[m, k] W[n, k] (+ bias[n]),   fp32 in and out.
+//
+// The projections of a prefill (in_proj, out_proj: model.py:197, 240; the
+// tied lm_head: model.py:339) are compute-bound fp32 products, and the fp32
+// matrix instructions run at 1/16 of the f16 ones (154 against 1470 TFLOP/s
+// measured on 8192^3 library products).  Every fp32 value is therefore split
+// into two f16 parts,
+//   x 2^e = hi + lo,   hi = f16(x 2^e),  lo = f16(x 2^e - hi),
+// with one power of two 2^e per row (of X and of W) that puts the row's
+// largest magnitude in [2^14, 2^15).  hi + lo holds 22 significand bits of
+// every element down to 2^-17 of its row's largest, and an absolute 2^-40 of
+// that largest below it.  A product takes three MFMAs,
+//   x w = lo_x hi_w + hi_x lo_w + hi_x hi_w   (lo lo, under 2^-22 of the product, is left out),
+// all accumulated in fp32, and the epilogue multiplies by 2^-(e_x + e_w)
+// (exact).  The dropped and rounded parts are ~2^-24 of each product, as
+// fp32's own rounding is, and the fp32 accumulator is rounded 3 times per 16
+// columns in place of 16, so the result is closer to the exact product than
+// the fp32 matrix path's (tests/test_gpu_gemm.py).
+//
+// Operand layout (split_rows_kernel writes it): blocks of 64 rows, in them
+// 16-column panels,
+//   [rows / 64][K / 16][64][64 bytes],  a row's 64 bytes = hi of columns 0-7,
+//   lo of 0-7, hi of 8-15, lo of 8-15 of the panel (K padded to 32 columns
+//   with zeros; the rows past the last are never written and never used),
+// so a stage of the GEMM -- a panel or two of a tile's rows -- is a few
+// contiguous 4 KB runs, a tile's whole operand lies in one stretch of memory,
+// and a split row takes exactly the bytes of its fp32 values.
+//
+// A row that holds an infinity or NaN cannot be split; its exponent is
+// marked, and the outputs that touch it are computed from the fp32 operands
+// by plain fp32 sums in the epilogue, so infinities and NaN come out as an
+// fp32 product gives them.
+//
+// Measured (us; library fp32 GEMM -> this product, plus the splits of X / W):
+//   32768 x 3072 x 768 (mamba-130m in_proj, 32 x 1024 tokens)   1246 -> 449 + 44 / 7
+//   32768 x 768 x 1536 (its out_proj)                            554 -> 215 + 95 / 7
+//   1024 x 8192 x 2048 (mamba-1.4b in_proj, 1024 tokens)         240 -> 100 + 8 / 34
+//   1024 x 2048 x 4096 (its out_proj)                            119 -> 69 + 14 / 20
+//   999 x 50280 x 768 (the tied lm_head)                         700 -> 283 + 7 / 71
+// at 250 to 392 TFLOP/s of fp32 product, 3 MFMAs each: 0.75 to 1.18 PFLOP/s of
+// the 1.47 that the library reaches on an 8192^3 f16 product.  The relative
+// error against 64 bits (2-norm) falls from 5.0e-7 to 3.1e-7 at K = 768,
+// 8.1e-7 to 5.0e-7 at 2048 and 1.15e-6 to 7.1e-7 at 4096.  With the
+// conversion inside the product's loop (fp32 tiles in LDS, no split pass) the
+// 1024 x 8192 x 2048 product took 147 us in place of 100 + 42.
+
+#include "common.h"
+#include "gemm.h"
+
+namespace mtl {
+namespace {
+
+typedef _Float16 H8 __attribute__((ext_vector_type(8)));
+typedef float F16v __attribute__((ext_vector_type(16)));
+
+constexpr int kPanel = 16;                 // columns of a panel
+constexpr int kPanelBytes = 64;            // bytes of a row in it
+constexpr int kRowBlock = 64;              // rows of a block
+constexpr int kExpSpecial = 1 << 20;       // exponent mark of a row with infinities (kExpNan: with a NaN)
+constexpr int kExpNan = 1 << 21;
+
+// ------------------------------------------------------------------ splitting
+// One workgroup takes 16 rows: lane = (row of 16, 8-column block of 4), so a
+// wavefront reads whole 128-byte runs of 16 rows and writes 1 KB runs of two
+// panels; the wavefronts take 32-column units in turn.  Pass 1 finds each
+// row's largest |x| (bit patterns, so a NaN is the largest), pass 2 reads the
+// rows again (from L2) and writes the parts.  The mark of a row with
+// non-finite values is its largest bit pattern: above inf's it holds a NaN.
+constexpr int kSplitRows = 16;
+
+__device__ __forceinline__ void load8(const float* p, int n, bool vec, float* v) {
+    if (vec && n >= 8) {
+        const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = j < n ? p[j] : 0.f;
+    }
+}
+
+// the power of two of a row whose largest magnitude has the bits `mx`
+__device__ __forceinline__ int split_exp(uint32_t mx) {
+    if (mx >= 0x7f800000u) return mx > 0x7f800000u ? kExpNan : kExpSpecial;
+    // (a zero or subnormal row takes the largest scale, 2^126)
+    return min(14 - ((int)(mx >> 23) - 127), 126);
+}
+
+// 8 columns of a row into its hi and lo parts
+__device__ __forceinline__ void split8(const float* v, float scale, H8& hi, H8& lo) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float s = v[j] * scale;
+        hi[j] = (_Float16)s;
+        lo[j] = (_Float16)(s - (float)hi[j]);
+    }
+}
+
+struct SplitJob {
+    const float* x;
+    int64_t ld, rows;
+    int K, vec;                            // vec: 16-byte aligned rows
+    uint8_t* out;
+    int* exps;                             // [rows rounded up to 64]
+};
+
+// workgroups [0, nb0) take the first matrix, the others the second
+template <int NT>
+__global__ void __launch_bounds__(NT) split_rows_kernel(const SplitJob j0, const SplitJob j1, int nb0) {
+    const bool second = (int)blockIdx.x >= nb0;
+    const float* const x = second ? j1.x : j0.x;
+    const int64_t ld = second ? j1.ld : j0.ld, rows = second ? j1.rows : j0.rows;
+    const int K = second ? j1.K : j0.K;
+    const bool vec = second ? j1.vec : j0.vec;
+    uint8_t* const out = second ? j1.out : j0.out;
+    int* const exps = second ? j1.exps : j0.exps;
+    const int64_t block = (int)blockIdx.x - (second ? nb0 : 0);
+    constexpr int NW = NT / 64;
+    __shared__ uint32_t s_max[NW][kSplitRows];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane >> 2, blk = lane & 3;
+    const int64_t row = block * kSplitRows + r;
+    const float* p = x + min(row, rows - 1) * ld;
+    const int units = (K + 31) / 32;
+    uint32_t mx = 0;
+    for (int u = wave; u < units; u += NW) {
+        const int c = u * 32 + blk * 8;
+        float v[8];
+        load8(p + c, K - c, vec, v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mx = max(mx, abs_bits(v[j]));
+    }
+    mx = max(mx, dpp_mov_u<kDppXor1>(mx));
+    mx = max(mx, dpp_mov_u<kDppXor2>(mx));
+    if (blk == 0) s_max[wave][r] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) mx = max(mx, s_max[w][r]);
+    const int e = split_exp(mx);
+    if (wave == 0 && blk == 0) exps[row] = row < rows ? e : 0;     // exps is padded to whole row blocks
+    // a marked row's parts are never used: any finite values do
+    const float scale = e >= kExpSpecial ? 0.f : __uint_as_float((uint32_t)(e + 127) << 23);
+    const int np = 2 * units;
+    for (int u = wave; u < units; u += NW) {
+        const int c = u * 32 + blk * 8, pan = 2 * u + (blk >> 1);
+        float v[8];
+        load8(p + c, K - c, vec, v);
+        if (e >= kExpSpecial) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = 0.f;
+        }
+        H8 hi, lo;
+        split8(v, scale, hi, lo);
+        if (row < rows) {
+            uint8_t* q = out + (row / kRowBlock * np + pan) * (kRowBlock * kPanelBytes) +
+                         (row % kRowBlock) * kPanelBytes + (blk & 1) * 32;
+            *reinterpret_cast<H8*>(q) = hi;
+            *reinterpret_cast<H8*>(q + 16) = lo;
+        }
+    }
+}
+
+// ------------------------------------------------------------------ the product
+struct GemmArgs {
+    const uint8_t* xs; const int* ex;      // split X [M, K]
+    const uint8_t* ws; const int* ew;      // split W [N, K]
+    float* y0; float* y1;                  // columns [0, n_split) to y0, the others to y1
+    int64_t ldy0, ldy1;
+    const float* bias;
+    const float* x32; const float* w32;    // the fp32 operands, for rows that cannot be split
+    int64_t ldx, ldw;
+    int M, N, K, n_split;
+    int tm, tn;                            // tiles along M and N
+};
+
+// Mapping: a workgroup of 4 wavefronts takes a BM x BN tile of Y, each
+// wavefront WM x WN of it as 32 x 32 MFMA tiles; the K loop walks stages of PK
+// panels through an LDS ring of ST slots.
+//   * The copies (global_load_lds_dwordx4, 16 rows x 64 bytes each) put 16-byte
+//     chunk c of a row at position c ^ ((row >> 2) & 3): the fragment reads
+//     (ds_read_b128, 32 rows of one chunk) then meet no bank conflict
+//     (counted; with (row >> 1) & 3 half of the LDS cycles were conflicts).
+//   * One barrier per stage.  The next panel's fragments are read into a
+//     second register set, and the next stages' copies issued, between the
+//     MFMAs of the present panel; issued in one piece after the barrier, the
+//     copies held up the MFMAs behind them (32768 x 768 x 1536: 250 -> 218 us).
+//   * The three products run tile by tile in turn, so an accumulator is used
+//     again TI TJ MFMAs later.
+template <int BM, int BN, int WM, int WN, int PK, int ST, int OCC>
+__global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kernel(const GemmArgs a) {
+    constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN;
+    constexpr int TI = WM / 32, TJ = WN / 32;             // 32x32 MFMA tiles of a wavefront
+    constexpr int SROWS = BM + BN, STAGE = PK * SROWS * kPanelBytes;
+    constexpr int NI = PK * SROWS / 16 / NW;                   // 1 KB copies per wavefront and stage
+    static_assert(SROWS % (16 * NW) == 0, "copies divide over the wavefronts");
+    __shared__ __align__(1024) uint8_t ring[ST * STAGE];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave / NWN, wn = wave % NWN;
+
+    // XCD-aware tile order (workgroups are dealt to the 8 XCDs round robin):
+    // each XCD takes a contiguous range of tiles, ordered 8 row tiles by all
+    // column tiles, rows fastest, so the tiles resident on an XCD at one time
+    // share their operand rows in its L2
+    int t = blockIdx.x;
+    const int total = a.tm * a.tn;
+    {
+        const int per = total / 8, rem = total % 8, x = t % 8, i = t / 8;
+        t = x * per + min(x, rem) + i;
+    }
+    constexpr int GM = 8;
+    const int group = t / (GM * a.tn), g0 = group * GM, gm = min(GM, a.tm - g0);
+    const int in_g = t - group * GM * a.tn;
+    // (uniform, but the divisions run on the VALU: back to SGPRs)
+    const int m0 = __builtin_amdgcn_readfirstlane((g0 + in_g % gm) * BM);
+    const int n0 = __builtin_amdgcn_readfirstlane(in_g / gm * BN);
+
+    // copy lane: row 16 g + lane / 4 of the stage; position lane % 4 of a row
+    // takes 16-byte chunk (lane % 4) ^ ((row >> 1) & 3), so 8 consecutive rows'
+    // reads of one chunk hit distinct banks
+    const int np = (a.K + 31) / 32 * 2;                    // panels (K padded to 32)
+    const uint8_t* base[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int g = (wave * NI + i) % (SROWS / 16), pk = (wave * NI + i) / (SROWS / 16);
+        const int row = 16 * g + (lane >> 2);
+        const int c = (lane & 3) ^ ((row >> 2) & 3);
+        const bool isx = 16 * g < BM;                     // wavefront-uniform (BM a multiple of 16)
+        const int rr = isx ? min(m0 + row, a.M - 1) : min(n0 + row - BM, a.N - 1);
+        base[i] = (isx ? a.xs : a.ws) + ((int64_t)(rr / kRowBlock) * np + pk) * (kRowBlock * kPanelBytes) +
+                  rr % kRowBlock * kPanelBytes + c * 16;
+    }
+    // stage s's panels; a last stage past the panels re-reads the last ones (its products are skipped)
+    auto issue1 = [&](int i, int slot, int s) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        const uint32_t so = (uint32_t)s * (PK * kRowBlock * kPanelBytes);
+        __builtin_amdgcn_global_load_lds(base[i] + so, ring + slot * STAGE + (wave * NI + i) * 1024, 16, 0, 0);
+#else
+        (void)i; (void)slot; (void)s;
+#endif
+    };
+    auto issue = [&](int slot, int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) issue1(i, slot, s);
+    };
+
+    F16v acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+
+    const int r32 = lane & 31, g2 = lane >> 5;
+    // byte offsets of this lane's hi chunk in rows 32 i + r32 of a tile (the
+    // swizzle depends on r32 only, as 32 i is a multiple of 8)
+    const int sw = (r32 >> 2) & 3;
+    const uint32_t o_hi = r32 * kPanelBytes + ((2 * g2) ^ sw) * 16, o_lo = r32 * kPanelBytes + ((2 * g2 + 1) ^ sw) * 16;
+    struct Frag { H8 xh[TI], xl[TI], wh[TJ], wl[TJ]; };
+    constexpr int NR = 2 * (TI + TJ);                     // LDS reads of a fragment set
+    auto read1 = [&](Frag& f, int k, int slot, int pk) __attribute__((always_inline)) {
+        const uint8_t* p = ring + slot * STAGE + pk * SROWS * kPanelBytes;
+        const uint8_t* px = p + wm * WM * kPanelBytes;
+        const uint8_t* pw = p + (BM + wn * WN) * kPanelBytes;
+        // x lo and w hi first: the first product takes them
+        if (k < TI) f.xl[k] = *reinterpret_cast<const H8*>(px + k * 32 * kPanelBytes + o_lo);
+        else if (k < TI + TJ) f.wh[k - TI] = *reinterpret_cast<const H8*>(pw + (k - TI) * 32 * kPanelBytes + o_hi);
+        else if (k < 2 * TI + TJ) f.xh[k - TI - TJ] = *reinterpret_cast<const H8*>(px + (k - TI - TJ) * 32 * kPanelBytes + o_hi);
+        else f.wl[k - 2 * TI - TJ] = *reinterpret_cast<const H8*>(pw + (k - 2 * TI - TJ) * 32 * kPanelBytes + o_lo);
+    };
+    constexpr int MT = TI * TJ;                            // MFMAs of one of the three products
+    // MFMA t of the 3 MT of a panel: product t / MT (lo hi, hi lo, hi hi) of
+    // tile t % MT, so an accumulator is used again MT MFMAs later
+    auto mma1 = [&](const Frag& f, int t) __attribute__((always_inline)) {
+        const int p = t / MT, i = t % MT % TI, j = t % MT / TI;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(p == 0 ? f.xl[i] : f.xh[i], p == 1 ? f.wl[j] : f.wh[j],
+                                                           acc[i][j], 0, 0, 0);
+    };
+
+    const int ns = (np + PK - 1) / PK;                      // stages
+    int slot = 0;
+    // stage s + 1 of the ring is read into nxt while stage s (in cur) is multiplied
+    auto sync = [&](bool tail) __attribute__((always_inline)) {
+        if (tail)
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * NI) : "memory");
+    };
+    auto body = [&](Frag& cur, Frag& nxt, int s, int pk) __attribute__((always_inline)) {
+        int prev = slot;
+        bool load = false, rd = true;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) mma1(cur, t);
+        __builtin_amdgcn_sched_barrier(0);
+        if (pk + 1 == PK) {
+            rd = s + 1 < ns;
+            if (rd) {
+                sync(s + ST > ns);
+                slot = slot + 1 == ST ? 0 : slot + 1;
+                load = s + ST < ns;
+            }
+        }
+        const int npk = pk + 1 == PK ? 0 : pk + 1;
+        // the reads and then the copies go between the MFMAs of the other two products
+#pragma unroll
+        for (int t = 0; t < 2 * MT; ++t) {
+            mma1(cur, MT + t);
+            if (rd) {
+#pragma unroll
+                for (int k = t * NR / MT; k < (t + 1) * NR / MT && k < NR; ++k) read1(nxt, k, slot, npk);
+            }
+            if (t >= MT && load) {
+#pragma unroll
+                for (int k = (t - MT) * NI / MT; k < (t - MT + 1) * NI / MT; ++k) issue1(k, prev, s + ST);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < ST; ++s)
+        if (s < ns) issue(s, s);
+    Frag f0, f1;
+    if (ns >= ST)
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((ST - 1) * NI) : "memory");
+    else
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int k = 0; k < NR; ++k) read1(f0, k, 0, 0);
+    int s = 0;
+    if constexpr (PK == 1) {
+        for (; s + 1 < ns; s += 2) {
+            body(f0, f1, s, 0);
+            body(f1, f0, s + 1, 0);
+        }
+        if (s < ns) body(f0, f1, s, 0);
+    } else {
+        for (; s < ns; ++s) {
+            body(f0, f1, s, 0);
+            body(f1, f0, s, 1);
+        }
+    }
+
+    // D[i][j] of a tile: column j = lane % 32 (an output column n), row
+    // 8 (q / 4) + 4 (lane / 32) + q % 4 in register q (an output row m).  The
+    // stores go through buffer resources that end at this tile's last row of
+    // y; a lane past the last column gets an offset past the end, so neither
+    // needs a branch.
+    const int mw = m0 + wm * WM, mpad = (a.M + kRowBlock - 1) / kRowBlock * kRowBlock;
+    int en[TJ];
+    float bn[TJ];
+    bool special = false;
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+        const int n = n0 + wn * WN + 32 * j + r32, nc = min(n, a.N - 1);
+        en[j] = a.ew[nc];
+        bn[j] = a.bias ? a.bias[nc] : 0.f;
+        special |= en[j] >= kExpSpecial;
+    }
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+        int em[16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int4 v = *reinterpret_cast<const int4*>(a.ex + min(mw + 32 * i + 8 * q + 4 * g2, mpad - 4));
+            em[4 * q] = v.x; em[4 * q + 1] = v.y; em[4 * q + 2] = v.z; em[4 * q + 3] = v.w;
+            special |= max(max(v.x, v.y), max(v.z, v.w)) >= kExpSpecial;
+        }
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const int nt = n0 + wn * WN + 32 * j;            // n_split is a multiple of 32 (host-checked)
+            const bool first = nt < a.n_split;
+            const int64_t ldy = first ? a.ldy0 : a.ldy1;
+            const int n = nt + r32, col = first ? n : n - a.n_split;
+            float* yt = (first ? a.y0 : a.y1) + (int64_t)m0 * ldy;
+            const auto ry = __builtin_amdgcn_make_buffer_rsrc(yt, (short)0, (int)(min(BM, a.M - m0) * ldy * 4), 0x00020000);
+            const uint32_t vo = n < a.N ? (uint32_t)(col + 4 * g2 * ldy) * 4u : 0xfffffff0u;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int ml = wm * WM + 32 * i + 8 * (q >> 2) + (q & 3);
+                const float v = __builtin_amdgcn_ldexpf(acc[i][j][q], -(em[q] + en[j])) + bn[j];
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ry, (int)vo, (int)(ml * ldy * 4), 0);
+            }
+        }
+    }
+    // outputs of rows that could not be split, over the values stored above by the same lanes
+    if (__any(special)) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        for (int j = 0; j < TJ; ++j) {
+            const int n = n0 + wn * WN + 32 * j + r32;
+            for (int mi = 0; mi < 16 * TI; ++mi) {
+                const int q = mi & 15, m = mw + (mi >> 4) * 32 + 8 * (q >> 2) + 4 * g2 + (q & 3);
+                if (m >= a.M || n >= a.N || (a.ex[m] < kExpSpecial && a.ew[n] < kExpSpecial)) continue;
+                const float* x = a.x32 + m * a.ldx;
+                const float* w = a.w32 + n * a.ldw;
+                float v = 0.f;
+                for (int k = 0; k < a.K; ++k) v = fmaf(x[k], w[k], v);
+                if (a.bias) v += a.bias[n];
+                if (n < a.n_split) a.y0[m * a.ldy0 + n] = v;
+                else a.y1[m * a.ldy1 + n - a.n_split] = v;
+            }
+        }
+    }
+}
+
+template <int BM, int BN, int WM, int WN, int PK, int ST, int OCC>
+void launch_gemm(GemmArgs a, hipStream_t st) {
+    a.tm = (a.M + BM - 1) / BM;
+    a.tn = (a.N + BN - 1) / BN;
+    hipLaunchKernelGGL((gemm_split_kernel<BM, BN, WM, WN, PK, ST, OCC>), dim3((unsigned)(a.tm * a.tn)),
+                       dim3(BM / WM * (BN / WN) * 64), 0, st, a);
+}
+
+int64_t pad_to(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
+
+SplitJob split_job(const float* x, int64_t ld, int64_t rows, int64_t K, void* buf) {
+    SplitJob j{};
+    j.x = x; j.ld = ld; j.rows = rows; j.K = (int)K;
+    j.vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && ld % 4 == 0;
+    j.exps = static_cast<int*>(buf);
+    j.out = static_cast<uint8_t*>(buf) + pad_to(pad_to(rows, kRowBlock) * (int64_t)sizeof(int), 1024);
+    return j;
+}
+
+}  // namespace
+
+int64_t split_bytes(int64_t rows, int64_t K) {
+    return pad_to(pad_to(rows, kRowBlock) * (int64_t)sizeof(int), 1024) + pad_to(rows, kRowBlock) * pad_to(K, 32) * 4;
+}
+
+int split_rows(const float* x, int64_t ldx, int64_t M, const float* w, int64_t ldw, int64_t N, int64_t K, void* xbuf,
+               void* wbuf, hipStream_t st) {
+    const SplitJob jx = split_job(x ? x : w, x ? ldx : ldw, x ? M : N, K, x ? xbuf : wbuf);
+    const SplitJob jw = split_job(w ? w : x, w ? ldw : ldx, w ? N : M, K, w ? wbuf : xbuf);
+    const int64_t bx = x ? pad_to(M, kRowBlock) / kSplitRows : 0, bw = w ? pad_to(N, kRowBlock) / kSplitRows : 0;
+    hipLaunchKernelGGL((split_rows_kernel<512>), dim3((unsigned)(bx + bw)), dim3(512), 0, st, jx, jw, (int)bx);
+    return check_launch("split_rows");
+}
+
+int gemm_split(const SplitGemm& g, hipStream_t st) {
+    const SplitJob x = split_job(g.x, g.ldx, g.M, g.K, g.xbuf), w = split_job(g.w, g.ldw, g.N, g.K, g.wbuf);
+    GemmArgs a{};
+    a.xs = x.out; a.ex = x.exps; a.ws = w.out; a.ew = w.exps;
+    a.y0 = g.y0; a.ldy0 = g.ldy0; a.y1 = g.y1 ? g.y1 : g.y0; a.ldy1 = g.y1 ? g.ldy1 : g.ldy0;
+    a.n_split = (int)(g.y1 ? g.n_split : g.N);
+    a.bias = g.bias;
+    a.x32 = g.x; a.ldx = g.ldx; a.w32 = g.w; a.ldw = g.ldw;
+    a.M = (int)g.M; a.N = (int)g.N; a.K = (int)g.K;
+    // Tile by the number of tiles each gives (us at M x N x K; 256 x 128, 128 x
+    // 128, 64 x 64): 32768 x 3072 x 768 449 / 499 / 739, 512 x 50280 x 768 147 /
+    // 158 / 234 (786 large tiles); 768 x 8192 x 2048 100 / 90 / 103, 512 x 8192 x
+    // 2048 90 / 59 / 75 (256 middle tiles); 384 x 8192 x 2048 91 / 55 / 54, 999 x
+    // 3072 x 768 44 / 28 / 26 (192), 1024 x 2048 x 4096 154 / 92 / 69 (128).  A
+    // CU holds 2, 2 and 3 of these workgroups.
+    const int64_t large = ((g.M + 255) / 256) * ((g.N + 127) / 128), middle = ((g.M + 127) / 128) * ((g.N + 127) / 128);
+    if (large >= 512) launch_gemm<256, 128, 128, 64, 1, 3, 2>(a, st);
+    else if (middle >= 224) launch_gemm<128, 128, 64, 64, 2, 2, 2>(a, st);
+    else launch_gemm<64, 64, 32, 32, 2, 3, 3>(a, st);
+    return check_launch("gemm_split");
+}
+
+}  // namespace mtl
+
+extern "C" int64_t mtl_linear_f32_ws_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M < 1 || N < 1 || K < 1) return 0;
+    return mtl::pad_to(mtl::split_bytes(M, K), 1024) + mtl::split_bytes(N, K);
+}
+
+extern "C" int mtl_linear_f32(const mtl_linear_f32_args* g, mtl_stream_t stream) {
+    using namespace mtl;
+    clear_error();
+    MTL_REQUIRE(g, "null args");
+    MTL_REQUIRE(g->M >= 0 && g->N >= 0 && g->K >= 1, "M, N must be >= 0 and K >= 1");
+    if (g->M == 0 || g->N == 0) return MTL_OK;
+    MTL_REQUIRE(g->x && g->W && g->y0 && g->ws, "null x, W, y0 or ws");
+    // 2^30: tile counts, exponent indexes and 256 output rows' byte offsets stay in 32 bits
+    MTL_REQUIRE(g->M <= (int64_t(1) << 30) && g->N <= (int64_t(1) << 30) && g->K <= (int64_t(1) << 23),
+                "M, N must be <= 2^30 and K <= 2^23");
+    MTL_REQUIRE(((g->M + 63) / 64) * ((g->N + 63) / 64) < (int64_t(1) << 31), "too many output tiles");
+    MTL_REQUIRE(g->ldx >= g->K && g->ldw >= g->K, "ldx and ldw must be >= K");
+    const int64_t n0 = g->y1 ? g->n_split : g->N;
+    MTL_REQUIRE(!g->y1 || (g->n_split > 0 && g->n_split < g->N && g->n_split % 32 == 0),
+                "n_split must be a multiple of 32 inside (0, N)");
+    MTL_REQUIRE(g->ldy0 >= n0 && g->ldy0 < (int64_t(1) << 21) &&
+                (!g->y1 || (g->ldy1 >= g->N - n0 && g->ldy1 < (int64_t(1) << 21))),
+                "ldy must cover the output's columns and be below 2^21");
+    MTL_REQUIRE(g->ws_bytes >= mtl_linear_f32_ws_bytes(g->M, g->N, g->K), "ws is too small");
+    MTL_REQUIRE(reinterpret_cast<uintptr_t>(g->ws) % 16 == 0, "ws must be 16-byte aligned");
+    SplitGemm s{};
+    s.x = g->x; s.ldx = g->ldx; s.w = g->W; s.ldw = g->ldw; s.bias = g->bias;
+    s.y0 = g->y0; s.ldy0 = g->ldy0; s.y1 = g->y1; s.ldy1 = g->ldy1; s.n_split = g->n_split;
+    s.M = g->M; s.N = g->N; s.K = g->K;
+    s.xbuf = g->ws;
+    s.wbuf = static_cast<uint8_t*>(g->ws) + pad_to(split_bytes(g->M, g->K), 1024);
+    hipStream_t st = as_stream(stream);
+    const int rc = split_rows(s.x, s.ldx, s.M, s.w, s.ldw, s.N, s.K, s.xbuf, s.wbuf, st);
+    return rc ? rc : gemm_split(s, st);
+}

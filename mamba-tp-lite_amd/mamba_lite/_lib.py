@@ -84,6 +84,15 @@ class PrefillLongArgs(ctypes.Structure):
     ]
 
 
+class LinearF32Args(ctypes.Structure):
+    """mirror of mtl_linear_f32_args"""
+    _fields_ = [
+        ("x", _vp), ("W", _vp), ("bias", _vp), ("y0", _vp), ("y1", _vp), ("ws", _vp), ("ws_bytes", _i64),
+        ("ldx", _i64), ("ldw", _i64), ("ldy0", _i64), ("ldy1", _i64), ("n_split", _i64),
+        ("M", _i64), ("N", _i64), ("K", _i64),
+    ]
+
+
 class DecodeLayer(ctypes.Structure):
     """mirror of mtl_decode_layer"""
     _fields_ = [
@@ -148,6 +157,8 @@ SIGNATURES = {
                                      _fp, _i32, _i32, _i32, _i32, _i32, _i32, _vp]),
     "mtl_decode_gemv": (ctypes.c_int, [_fp, _fp, _fp, _fp, _fp, _i32, _i32, _i32, _vp]),
     "mtl_decode_gemv_parts": (ctypes.c_int, [_fp, _fp, _fp, _i32, _i32, _i32, _i32, _vp]),
+    "mtl_linear_f32_ws_bytes": (_i64, [_i64, _i64, _i64]),
+    "mtl_linear_f32": (ctypes.c_int, [ctypes.POINTER(LinearF32Args), _vp]),
     "mtl_linear_skinny": (ctypes.c_int, [_fp, _i64, _fp, _fp, _fp, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _vp]),
     "mtl_in_proj_conv_prefill": (ctypes.c_int, [_fp, _i64, _fp, _fp, _fp, _fp, _i32, _fp, _fp, _fp, _fp, _i64, _i64,
                                                 _i64, _i64, _vp]),

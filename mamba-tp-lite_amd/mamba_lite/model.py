@@ -220,6 +220,19 @@ def _skinny_rows(x: torch.Tensor, w: torch.Tensor, enabled: bool = True, bias=No
     return x2 if ops.linear_skinny_ok(x2, w, bias=bias) else None
 
 
+def _linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
+    """F.linear, on the split-f16 product (ops.linear_f32) where it is the faster one."""
+    return ops.linear_f32(x, w, bias) if ops.linear_f32_ok(x, w, bias) else F.linear(x, w, bias)
+
+
+def _linear_mod(mod, x: torch.Tensor) -> torch.Tensor:
+    """mod(x) of a projection; a plain nn.Linear without hooks may take ops.linear_f32."""
+    if type(mod) is nn.Linear and not mod._forward_hooks and not mod._forward_pre_hooks and \
+            ops.linear_f32_ok(x, mod.weight, mod.bias):
+        return ops.linear_f32(x, mod.weight, mod.bias)
+    return mod(x)
+
+
 def _skinny_split(K: int, most: int = 16) -> int:
     """The largest split of K into ranges of whole 128-column granules, at
     most `most` parts."""
@@ -354,12 +367,16 @@ class MambaMixer(nn.Module):
         elif split:
             # in_proj as two GEMMs (x rows, z rows) so the conv and the scan read
             # whole contiguous [b, l, D] rows rather than halves of [b, l, 2D] rows
+            # (one product that writes the halves apart where ops.linear_f32 takes it)
             w_in, b_in = self.in_proj.weight, self.in_proj.bias
-            xs = F.linear(x, w_in[:Dm], b_in[:Dm] if b_in is not None else None).transpose(1, 2)   # [b, D, l]
-            z = F.linear(x, w_in[Dm:], b_in[Dm:] if b_in is not None else None).transpose(1, 2)
+            if Dm % 32 == 0 and ops.linear_f32_ok(x, w_in, b_in):
+                xs, z = (t.transpose(1, 2) for t in ops.linear_f32(x, w_in, b_in, n_split=Dm))      # [b, D, l]
+            else:
+                xs = F.linear(x, w_in[:Dm], b_in[:Dm] if b_in is not None else None).transpose(1, 2)
+                z = F.linear(x, w_in[Dm:], b_in[Dm:] if b_in is not None else None).transpose(1, 2)
         else:
             xz = (ops.linear_skinny(x2, self.in_proj.weight, self.in_proj.bias).view(b, l, 2 * Dm) if x2 is not None
-                  else self.in_proj(x))                          # [b, l, 2D]
+                  else _linear_mod(self.in_proj, x))             # [b, l, 2D]
             xs = xz[..., :Dm].transpose(1, 2)                    # [b, D, l] view, D-stride 1
             z = xz[..., Dm:].transpose(1, 2)
         conv_in_state = cache.conv_state if cache is not None else None
@@ -425,7 +442,7 @@ class MambaMixer(nn.Module):
             if y2 is not None and Dm % (128 * SKINNY_OUT_SPLIT) == 0:
                 parts = ops.linear_skinny(y2, w_out, self.out_proj.bias, ksplit=SKINNY_OUT_SPLIT)
                 return _Parts(parts.view(SKINNY_OUT_SPLIT, b, l, -1)), conv_state, h
-        return self.out_proj(y_store), conv_state, h
+        return _linear_mod(self.out_proj, y_store), conv_state, h
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """No-cache forward (reference model.py:243-246)."""
@@ -565,7 +582,7 @@ class MambaLM(nn.Module):
         self.norm_f = RMSNorm(cfg.d_model, eps=cfg.layer_norm_epsilon)
 
     def lm_head(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.embedding.weight)
+        return _linear(x, self.embedding.weight)
 
     def _norm_weight(self, i: int) -> torch.Tensor:
         mod = self.layers[i].norm if i < len(self.layers) else self.norm_f

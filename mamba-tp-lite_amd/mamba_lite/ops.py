@@ -866,6 +866,68 @@ def decode_gemv(v, W, out, bias=None, x_in=None):
     return out
 
 
+def linear_f32_pays(M: int, N: int, K: int) -> bool:
+    """Where mtl_linear_f32 (the splits of x and W included) beats the library's
+    fp32 GEMM: the split of W is paid once per call, so the gain needs rows,
+    and few tiles leave CUs idle.  Measured, us, library / split + product:
+    999 x 3072 x 768 45 / 40, 768 x 3072 x 768 36 / 39; 768 x 2048 x 4096 107 /
+    96, 512 x 2048 x 4096 69 / 86; 384 x 8192 x 2048 112 / 96, 256 x 8192 x 2048
+    74 / 81; 256 x 50280 x 768 171 / 156, 192 x 50280 x 768 146 / 150; 999 x 768 x
+    1536 24 / 38."""
+    flops = 2.0 * M * N * K
+    return N >= 256 and K >= 128 and ((M >= 256 and flops >= 1.2e10) or (M >= 896 and flops >= 4.5e9))
+
+
+def linear_f32_ok(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
+    """Whether linear_f32 takes F.linear(x, W, bias) in its place: plain fp32
+    GPU tensors with unit column stride, sizes where it pays, and nothing of
+    torch's that a raw launch would bypass (autograd, autocast, subclasses)."""
+    if x.dtype != torch.float32 or W.dtype != torch.float32 or not x.is_cuda or W.device != x.device or \
+            x.dim() < 2 or W.dim() != 2 or not x.is_contiguous() or W.stride(1) != 1 or x.shape[-1] != W.shape[1]:
+        return False
+    if type(x) is not torch.Tensor or type(W) not in (torch.Tensor, torch.nn.Parameter):
+        return False
+    N, K = W.shape
+    if x.numel() == 0 or not linear_f32_pays(x.numel() // K, N, K) or N >= 1 << 21 or W.stride(0) < K:
+        return False
+    if bias is not None and (type(bias) not in (torch.Tensor, torch.nn.Parameter) or bias.dtype != torch.float32 or
+                             bias.device != x.device or not bias.is_contiguous() or tuple(bias.shape) != (N,)):
+        return False
+    if torch.is_autocast_enabled("cuda"):
+        return False
+    return not (torch.is_grad_enabled() and (x.requires_grad or W.requires_grad or
+                                             (bias is not None and bias.requires_grad)))
+
+
+def linear_f32(x, W, bias=None, n_split=None):
+    """F.linear(x, W, bias) of contiguous fp32 x [..., K] on the f16 matrix
+    cores (mtl_linear_f32).  With n_split (a multiple of 32), the output's
+    columns [0, n_split) and the others as two contiguous tensors."""
+    N, K = W.shape
+    if x.dtype != torch.float32 or W.dtype != torch.float32 or not x.is_contiguous() or x.shape[-1] != K or \
+            W.stride(1) != 1:
+        raise ValueError("linear_f32: x must be contiguous float32 [..., K] and W float32 [N, K] with unit column stride")
+    if bias is not None and (bias.dtype != torch.float32 or not bias.is_contiguous() or tuple(bias.shape) != (N,)):
+        raise ValueError(f"bias must be contiguous float32 [{N}]")
+    if n_split is not None and not (0 < n_split < N and n_split % 32 == 0):
+        raise ValueError("n_split must be a multiple of 32 inside (0, N)")
+    _same_device(x, W, bias)
+    lead, M = x.shape[:-1], x.numel() // K
+    lib = _lib.load()
+    a = _lib.LinearF32Args()
+    a.M, a.N, a.K, a.ldx, a.ldw = M, N, K, K, W.stride(0)
+    nb = lib.mtl_linear_f32_ws_bytes(M, N, K)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=x.device)
+    n0 = N if n_split is None else n_split
+    y0 = torch.empty(*lead, n0, dtype=torch.float32, device=x.device)
+    y1 = None if n_split is None else torch.empty(*lead, N - n0, dtype=torch.float32, device=x.device)
+    a.x, a.W, a.bias, a.y0, a.y1 = _ptr(x), _ptr(W), _ptr(bias), _ptr(y0), _ptr(y1)
+    a.ws, a.ws_bytes, a.ldy0, a.ldy1, a.n_split = _ptr(ws), nb, n0, N - n0, n0
+    with _dev_guard(x):
+        _lib.check(lib.mtl_linear_f32(ctypes.byref(a), _stream(x)), "linear_f32")
+    return y0 if y1 is None else (y0, y1)
+
+
 SKINNY_MAX_ROWS = 64     # mtl_linear_skinny: rows of x per launch chunk
 SKINNY_CHUNKED_MAX_ROWS = 64 * 65535   # rows of x over all chunks
 IN_CONV_MAX_ROWS = 32    # mtl_in_proj_conv_xproj: batch rows

@@ -1,0 +1,99 @@
+"""mtl_linear_f32: the fp32 product on split f16 operands against the float64
+product, at tile edges and remainders, and its handling of extreme rows."""
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from mamba_lite import ops
+
+pytestmark = pytest.mark.gpu
+
+# M, N, K: below, at and past the 64, 128 and 256 tiles, K not a multiple of 16 or 32, one and several K stages
+SHAPES = [(1, 1, 1), (63, 33, 15), (64, 64, 16), (65, 129, 33), (257, 96, 100), (100, 1000, 48), (999, 768, 1536),
+          (1500, 2500, 130), (4100, 8200, 64), (16500, 1100, 96)]
+
+
+def _inputs(M, N, K, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(M, K, device="cuda", generator=g)
+    w = torch.randn(N, K, device="cuda", generator=g) * 0.02
+    b = torch.randn(N, device="cuda", generator=g)
+    return x, w, b
+
+
+def _err(got, x, w, b=None):
+    ref = x.double() @ w.double().t()
+    if b is not None:
+        ref = ref + b.double()
+    return float((got.double() - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_product_matches_float64(M, N, K):
+    x, w, b = _inputs(M, N, K)
+    # operand parts: two roundings and the dropped lo.lo term, each under 2^-22 of a product; the fp32 sum of K
+    # products rounds 3 K / 16 times, a random walk: under 2^-24 sqrt(3 K / 16) of the result
+    tol = 3 * 2.0 ** -22 + 2.0 ** -24 * math.sqrt(3 * K / 16 + 4)
+    assert _err(ops.linear_f32(x, w), x, w) < tol
+    assert _err(ops.linear_f32(x, w, b), x, w, b) < tol
+
+
+@pytest.mark.parametrize("M,N,K", [(1024, 2048, 4096), (4096, 3072, 768), (512, 4096, 2048)])
+def test_error_not_above_the_fp32_product(M, N, K):
+    x, w, _ = _inputs(M, N, K)
+    assert _err(ops.linear_f32(x, w), x, w) <= _err(F.linear(x, w), x, w)
+
+
+def test_split_output_and_strided_weight():
+    x, w, b = _inputs(300, 192, 80)
+    y0, y1 = ops.linear_f32(x, w, b, n_split=96)
+    y = ops.linear_f32(x, w, b)
+    assert torch.equal(torch.cat([y0, y1], 1), y)
+    wide = torch.randn(192, 200, device="cuda")
+    sub = wide[:, 3:83]                       # rows off a 16-byte boundary
+    assert torch.equal(ops.linear_f32(x, sub, b), ops.linear_f32(x, sub.contiguous(), b))
+    with pytest.raises(ValueError):
+        ops.linear_f32(x, w, b, n_split=50)
+
+
+def test_rows_of_very_different_magnitude():
+    """Each row's split is relative to its own largest value: rows 1e-30 to 1e30 keep their relative error, and
+    values far below their row's largest keep an absolute one of 2^-38 of it."""
+    x, w, _ = _inputs(128, 96, 256)
+    s = torch.logspace(-30, 30, 128, device="cuda")[:, None]
+    a, b = ops.linear_f32(x * s, w).double() / s.double(), ops.linear_f32(x, w).double()
+    assert float((a - b).norm() / b.norm()) < 4 * 2.0 ** -24 * math.sqrt(256)
+    spread = x * torch.logspace(0, -12, 256, device="cuda")
+    assert _err(ops.linear_f32(spread, w), spread, w) < 1e-6
+    z = ops.linear_f32(torch.zeros(70, 64, device="cuda"), w[:, :64].contiguous())
+    assert torch.equal(z, torch.zeros_like(z))
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 90, 40), (300, 500, 64), (1300, 12800, 32)])
+def test_infinities_and_nan_as_in_fp32(M, N, K):
+    x, w, b = _inputs(M, N, K)
+    x[3, 5], x[17, 0], x[17, 2], x[-1, -1] = math.inf, math.inf, -math.inf, -math.inf
+    x[40, 1] = math.nan
+    w[7, 5], w[11, 3], w[-2, 0] = 0.0, math.inf, math.nan
+    got, ref = ops.linear_f32(x, w, b), (x.double() @ w.double().t() + b.double()).float()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.isinf(got), torch.isinf(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(got[inf], ref[inf])
+    ok = torch.isfinite(ref)
+    assert float((got[ok] - ref[ok]).norm() / ref[ok].norm()) < 1e-6
+
+
+def test_route_keeps_autograd_and_autocast():
+    x, w, _ = _inputs(1024, 4096, 768)
+    assert ops.linear_f32_ok(x, w)
+    wp = torch.nn.Parameter(w)
+    assert not ops.linear_f32_ok(x, wp)
+    with torch.no_grad():
+        assert ops.linear_f32_ok(x, wp)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert not ops.linear_f32_ok(x, wp)
+    assert not ops.linear_f32_ok(x.bfloat16(), w.bfloat16())
+    assert not ops.linear_f32_ok(x[:128], w)
