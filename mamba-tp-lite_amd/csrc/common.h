@@ -54,6 +54,23 @@ template <> struct Act<uint16_t> {  // bf16 storage
     __device__ __forceinline__ static void store(uint16_t* p, float v) { *p = f32_to_bf16(v); }
 };
 
+// 4 consecutive values as floats, one 16-byte (fp32) or 8-byte (bf16) access;
+// and a value rounded to the storage type.
+typedef float F4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ F4v ld4(const float* p) { return *reinterpret_cast<const F4v*>(p); }
+__device__ __forceinline__ F4v ld4(const uint16_t* p) {
+    const uint2 x = *reinterpret_cast<const uint2*>(p);
+    return F4v{__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u), __uint_as_float(x.y << 16),
+               __uint_as_float(x.y & 0xffff0000u)};
+}
+__device__ __forceinline__ void st4(float* p, F4v v) { *reinterpret_cast<F4v*>(p) = v; }
+__device__ __forceinline__ void st4(uint16_t* p, F4v v) {
+    *reinterpret_cast<uint2*>(p) = uint2{f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3])};
+}
+template <typename T> __device__ __forceinline__ float round_to(float v);
+template <> __device__ __forceinline__ float round_to<float>(float v) { return v; }
+template <> __device__ __forceinline__ float round_to<uint16_t>(float v) { return bf16_to_f32(f32_to_bf16(v)); }
+
 // exp(x) through the hardware base-2 exponential.
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 

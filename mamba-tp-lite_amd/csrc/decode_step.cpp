@@ -20,6 +20,7 @@
 #include <string>
 
 #include "common.h"
+#include "step_ops.h"
 
 extern "C" int mtl_decode_step(const mtl_decode_step_args* a, const mtl_decode_layer* layers, mtl_stream_t stream) {
     using namespace mtl;
@@ -105,10 +106,12 @@ extern "C" int mtl_decode_step(const mtl_decode_step_args* a, const mtl_decode_l
 
 // A batched step of the whole layer stack in one C call, for the row counts
 // the fused kernels above do not take (MambaLM.step at b <= 32, reference
-// model.py:343-353 over MambaBlock.step 308-311 and MambaMixer.step 249-294),
-// fp32.  The launches are the per-op ones the Python layer makes at these
+// model.py:343-353 over MambaBlock.step 308-311 and MambaMixer.step 249-294).
+// fp32: the launches are the per-op ones the Python layer makes at these
 // sizes, with the same tile choices, so the results are the same bits; what
-// goes away is launching ~5 ops per layer from Python.  Per layer:
+// goes away is launching ~5 ops per layer from Python.  bf16 (weights,
+// activations and conv history; fp32 residual, SSM state and partial sums):
+// the same launches on the bf16 matrix cores.  Per layer:
 //   in_proj + conv step (history updated in place) + the x_proj partials of
 //     each channel block (mtl_in_proj_conv_xproj; folded, from layer 1 on,
 //     its _normed form, which applies the norm to the dot products from the
@@ -133,6 +136,47 @@ int32_t step_resid_rows_per_block(int32_t b, int32_t M) {
     return (b > 16 && b <= 32 && M % 32 == 0 && M / 32 * kStepOutSplit >= 256) ? 32 : 16;
 }
 
+// the launches of every layer, the sizes and pointers checked by the caller
+template <typename T>
+int step_layers(const mtl_decode_step_batched_args* a, const mtl_decode_layer* layers, int32_t cpp, int32_t rpb_o,
+                int32_t rpb_r, mtl_stream_t stream) {
+    using namespace mtl;
+    const int32_t b = a->batch, M = a->d_model, D = a->d_inner, N = a->d_state, R = a->dt_rank, K = a->d_conv;
+    const int32_t J = R + 2 * N, nl = a->n_layers, tiles = M / rpb_r;
+    const bool fold = a->fold != 0;
+    auto t = [](const void* p) { return static_cast<const T*>(p); };
+    auto w = [](void* p) { return static_cast<T*>(p); };
+    T *inp = w(a->inp), *xn = w(a->xn), *xc = w(a->xc), *z = w(a->z), *y = w(a->y);
+    const int64_t bJ = (int64_t)b * J, bM = (int64_t)b * M;
+    int rc = add_rmsnorm<T>(a->h, nullptr, 0, nullptr, t(layers[0].norm_w), inp, b, M, layers[0].eps, stream);
+    if (rc) return rc;
+    for (int32_t i = 0; i < nl; ++i) {
+        const mtl_decode_layer& L = layers[i];
+        const bool last = i + 1 == nl, normed = fold && i > 0;
+        rc = in_proj_conv_xproj<T>(normed ? xn : inp, M, t(L.W_in), t(L.b_in), w(L.conv_state), t(L.conv_w),
+                                   t(L.conv_b), K, t(L.W_xT), J, xc, z, D, a->xpart, b, M, D, cpp,
+                                   normed ? a->sq : nullptr, normed ? tiles : 0, normed ? L.eps : 0.f, stream);
+        if (rc) return rc;
+        rc = mtl_sum_parts(a->xpart, D / cpp, bJ, a->x_dbl, stream);
+        if (rc) return rc;
+        rc = state_update<T>(L.ssm_state, xc, D, z, D, a->x_dbl, J, t(L.W_dt), t(L.dt_bias), t(L.A_log), t(L.Dv), y,
+                             D, b, D, N, R, stream);
+        if (rc) return rc;
+        if (fold && !last) {
+            rc = linear_residual<T>(y, D, t(L.W_out), t(L.b_out), a->parts, b, M, D, kStepOutSplit, rpb_r, a->h,
+                                    t(layers[i + 1].norm_w), xn, a->sq, a->counters + (int64_t)i * tiles, stream);
+            if (rc) return rc;
+            continue;
+        }
+        rc = linear_parts<T>(y, D, t(L.W_out), t(L.b_out), a->parts, M, bM, b, M, D, kStepOutSplit, rpb_o, stream);
+        if (rc) return rc;
+        rc = add_rmsnorm<T>(a->h, a->parts, kStepOutSplit, a->h, t(last ? a->norm_f : layers[i + 1].norm_w),
+                            last ? w(a->normed_out) : inp, b, M, last ? a->eps_f : layers[i + 1].eps, stream);
+        if (rc) return rc;
+    }
+    return MTL_OK;
+}
+
 }  // namespace
 
 extern "C" int mtl_decode_step_batched(const mtl_decode_step_batched_args* a, const mtl_decode_layer* layers,
@@ -146,7 +190,11 @@ extern "C" int mtl_decode_step_batched(const mtl_decode_step_batched_args* a, co
     MTL_REQUIRE(b >= 1 && b <= 32, "batch must be in [1, 32]");
     MTL_REQUIRE(nl >= 1, "n_layers must be >= 1");
     MTL_REQUIRE(M >= 256 && M % 128 == 0 && M <= 65536, "d_model must be a multiple of 128 in [256, 65536]");
-    MTL_REQUIRE(D >= 512 && D % 512 == 0 && D <= 65536, "d_inner must be a multiple of 512 in [512, 65536]");
+    MTL_REQUIRE((D >= 512 && D % 512 == 0 && D <= 65536) || a->dtype == MTL_BF16,
+                "d_inner must be a multiple of 512 in [512, 65536]");
+    MTL_REQUIRE(a->dtype == MTL_F32 || a->dtype == MTL_BF16, "dtype must be MTL_F32 or MTL_BF16");
+    MTL_REQUIRE(a->dtype == MTL_F32 || (M >= 512 && D >= 1024 && D % 256 == 0 && D <= 65536),
+                "bf16: d_model must be at least 512 and d_inner a multiple of 256 in [1024, 65536]");
     MTL_REQUIRE(N >= 1 && N <= 16 && R >= 1 && R <= 256, "d_state must be in [1, 16] and dt_rank in [1, 256]");
     MTL_REQUIRE(J <= 288, "dt_rank + 2 d_state must be at most 288");
     MTL_REQUIRE(K >= 2 && K <= 4, "d_conv must be 2, 3 or 4");
@@ -177,36 +225,6 @@ extern "C" int mtl_decode_step_batched(const mtl_decode_step_batched_args* a, co
                          "16-byte aligned");
         MTL_REQUIRE(L.eps >= 0.f, at + "eps must be >= 0 (not NaN)");
     }
-    const int64_t bJ = (int64_t)b * J, bM = (int64_t)b * M;
-    int rc = mtl_add_rmsnorm(a->h, nullptr, nullptr, layers[0].norm_w, a->inp, b, M, layers[0].eps, stream);
-    if (rc) return rc;
-    for (int32_t i = 0; i < nl; ++i) {
-        const mtl_decode_layer& L = layers[i];
-        const bool last = i + 1 == nl;
-        if (fold && i > 0)
-            rc = mtl_in_proj_conv_xproj_normed(a->xn, M, L.W_in, L.b_in, L.conv_state, L.conv_w, L.conv_b, K, L.W_xT,
-                                               J, a->xc, a->z, D, a->xpart, b, M, D, cpp, a->sq, tiles, L.eps, stream);
-        else
-            rc = mtl_in_proj_conv_xproj(a->inp, M, L.W_in, L.b_in, L.conv_state, L.conv_w, L.conv_b, K, L.W_xT, J,
-                                        a->xc, a->z, D, a->xpart, b, M, D, cpp, stream);
-        if (rc) return rc;
-        rc = mtl_sum_parts(a->xpart, D / cpp, bJ, a->x_dbl, stream);
-        if (rc) return rc;
-        rc = mtl_selective_state_update(L.ssm_state, a->xc, D, a->z, D, a->x_dbl, J, L.W_dt, L.dt_bias, L.A_log, L.Dv,
-                                        a->y, D, b, D, N, R, MTL_F32, 1, stream);
-        if (rc) return rc;
-        if (fold && !last) {
-            rc = mtl_linear_skinny_residual(a->y, D, L.W_out, L.b_out, a->parts, b, M, D, kStepOutSplit, rpb_r, a->h,
-                                            layers[i + 1].norm_w, a->xn, a->sq,
-                                            a->counters + (int64_t)i * tiles, stream);
-            if (rc) return rc;
-            continue;
-        }
-        rc = mtl_linear_skinny(a->y, D, L.W_out, L.b_out, a->parts, M, bM, b, M, D, kStepOutSplit, rpb_o, stream);
-        if (rc) return rc;
-        rc = mtl_add_rmsnorm_parts(a->h, a->parts, kStepOutSplit, a->h, last ? a->norm_f : layers[i + 1].norm_w,
-                                   last ? a->normed_out : a->inp, b, M, last ? a->eps_f : layers[i + 1].eps, stream);
-        if (rc) return rc;
-    }
-    return MTL_OK;
+    return a->dtype == MTL_BF16 ? step_layers<uint16_t>(a, layers, cpp, rpb_o, rpb_r, stream)
+                                : step_layers<float>(a, layers, cpp, rpb_o, rpb_r, stream);
 }

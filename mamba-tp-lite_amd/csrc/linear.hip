@@ -44,16 +44,22 @@
 // us (out_proj 16.7 / 12.6 / 10.0 us).
 
 #include "common.h"
+#include "step_ops.h"
 
 namespace mtl {
 namespace {
 
-typedef float F4v __attribute__((ext_vector_type(4)));
+typedef __bf16 B8v __attribute__((ext_vector_type(8)));
 
+// T: the storage type of x, W and the bias, float or bf16 (uint16_t).  A stage
+// row is 128 bytes either way: bf16 has 64 columns in it, and one
+// v_mfma_f32_16x16x32_bf16 takes the 16-byte chunks that four
+// v_mfma_f32_16x16x4_f32 take in fp32.
+template <typename T>
 struct LinArgs {
-    const float* x;        // [M, K], row stride x_rs
-    const float* W;        // [N, K] contiguous
-    const float* bias;     // [N] or null
+    const T* x;            // [M, K], row stride x_rs
+    const T* W;            // [N, K] contiguous
+    const T* bias;         // [N] or null
     float* y;              // [M, N] (row stride y_rs); split s at y + s * y_ks
     int64_t x_rs, y_rs, y_ks;
     int M, N, K, KS;
@@ -61,10 +67,9 @@ struct LinArgs {
 
 constexpr int kLinThreads = 256;
 constexpr int kLinWaves = kLinThreads / 64;
-constexpr int kKW = 32;                           // K columns per wavefront per stage
-constexpr int kKC = kLinWaves * kKW;              // K granule of a workgroup (128)
-
-__device__ __forceinline__ F4v ld4(const float* p) { return *reinterpret_cast<const F4v*>(p); }
+constexpr int kKW = 32;                           // 4-byte words of a stage row
+constexpr int kKC = kLinWaves * kKW;              // fp32 K granule of a workgroup (128)
+template <typename T> constexpr int kCols = kKW * 4 / (int)sizeof(T);   // columns of a stage row
 
 #define MTL_WAIT_VMCNT(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
 
@@ -73,8 +78,8 @@ __device__ __forceinline__ F4v ld4(const float* p) { return *reinterpret_cast<co
 // accumulators sit in s_acc = the ring's first RB MB 4 KB (after a barrier),
 // and tile_sum() adds them in wavefront order.  A kernel that calls it keeps
 // all of its LDS in the ring array (see in_conv_xproj_kernel).
-template <int RB, int MB, int D>
-__device__ __forceinline__ void skinny_tile(const LinArgs& a, float* ring, int n0, int ks) {
+template <int RB, int MB, int D, typename T>
+__device__ __forceinline__ void skinny_tile(const LinArgs<T>& a, float* ring, int n0, int ks) {
     constexpr int WR = 16 * RB, XR = 16 * MB, SROWS = WR + XR;   // rows of a stage: W then X
     constexpr int NI = SROWS / 8;                                 // copies per stage (8 rows each)
     constexpr int SLOT = SROWS * kKW;                             // floats per ring slot
@@ -83,19 +88,22 @@ __device__ __forceinline__ void skinny_tile(const LinArgs& a, float* ring, int n
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, kk = lane >> 4;
-    const int kper = a.K / a.KS;                       // a multiple of kKC (host-checked)
-    const int ns = kper / kKC;                         // stages per wavefront, >= D - 1 (host-checked)
-    const int kbeg = ks * kper + wave * (kper / kLinWaves);
+    // the stages of the split, dealt to the wavefronts in contiguous runs (the
+    // first ones take one more where they do not divide; fp32's always do)
+    constexpr int KW = kCols<T>, CE = 16 / (int)sizeof(T);
+    const int kper = a.K / a.KS, units = kper / KW;
+    const int ns = units / kLinWaves + (wave < units % kLinWaves ? 1 : 0);   // >= D - 1 (host-checked)
+    const int kbeg = ks * kper + (wave * (units / kLinWaves) + min(wave, units % kLinWaves)) * KW;
     float* myring = ring + wave * D * SLOT;
 
     // copy lane: row 8 i + lane / 8 of the stage, fetching chunk (lane % 8) ^ (row & 7)
     const int crow = lane >> 3, cch = (lane & 7) ^ crow;
-    const float* src[NI];
+    const T* src[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int row = 8 * i + crow;
-        src[i] = row < WR ? a.W + (int64_t)min(n0 + row, a.N - 1) * a.K + kbeg + 4 * cch
-                          : a.x + (int64_t)min(row - WR, a.M - 1) * a.x_rs + kbeg + 4 * cch;
+        src[i] = row < WR ? a.W + (int64_t)min(n0 + row, a.N - 1) * a.K + kbeg + CE * cch
+                          : a.x + (int64_t)min(row - WR, a.M - 1) * a.x_rs + kbeg + CE * cch;
     }
     auto issue = [&](int s) __attribute__((always_inline)) {
         float* dst = myring + (s % D) * SLOT;
@@ -104,7 +112,7 @@ __device__ __forceinline__ void skinny_tile(const LinArgs& a, float* ring, int n
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
         for (int i = 0; i < NI; ++i)
-            __builtin_amdgcn_global_load_lds(src[i] + s * kKW, dst + i * 256, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(src[i] + s * KW, dst + i * 256, 16, 0, 0);
 #else
         (void)dst;
 #endif
@@ -131,13 +139,23 @@ __device__ __forceinline__ void skinny_tile(const LinArgs& a, float* ring, int n
                 const int row = WR + 16 * mb + r;
                 xv[mb] = ld4(st + (row * 8 + (c ^ (row & 7))) * 4);
             }
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
+            if constexpr (sizeof(T) == 2) {
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb)
-                        acc[rb][mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[rb][q], xv[mb][q], acc[rb][mb], 0, 0, 0);
+                        acc[rb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(B8v, wv[rb]), __builtin_bit_cast(B8v, xv[mb]), acc[rb][mb], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                        for (int mb = 0; mb < MB; ++mb)
+                            acc[rb][mb] =
+                                __builtin_amdgcn_mfma_f32_16x16x4f32(wv[rb][q], xv[mb][q], acc[rb][mb], 0, 0, 0);
+            }
         }
     };
 
@@ -193,17 +211,17 @@ constexpr int ring_floats() { return kLinWaves * D * (16 * RB + 16 * MB) * kKW; 
 // workgroups are those of the z = 0 launch with x and y moved down, so the
 // n-tiles of every chunk share the tile order and land on the same XCD as
 // their z = 0 twins when the tiles per chunk are a multiple of 8.
-template <int RB, int MB, int D>
-__global__ void __launch_bounds__(kLinThreads) linear_skinny_kernel(const LinArgs a) {
+template <int RB, int MB, int D, typename T>
+__global__ void __launch_bounds__(kLinThreads) linear_skinny_kernel(const LinArgs<T> a) {
     __shared__ __align__(16) float ring[ring_floats<RB, MB, D>()];
     static_assert(sizeof(ring) >= sizeof(F4v) * kLinWaves * RB * MB * 64, "reduction space");
     const int n0 = blockIdx.x * 16 * RB, ks = blockIdx.y;
     const int r0 = blockIdx.z * 16 * MB;
-    LinArgs c = a;
+    LinArgs<T> c = a;
     c.x += (int64_t)r0 * a.x_rs;
     c.y += (int64_t)r0 * a.y_rs;
     c.M = min(16 * MB, a.M - r0);
-    skinny_tile<RB, MB, D>(c, ring, n0, ks);
+    skinny_tile<RB, MB, D, T>(c, ring, n0, ks);
     for (int t = threadIdx.x; t < RB * MB * 64; t += kLinThreads) {
         int m, nl;
         F4v sum = tile_sum<RB, MB>(ring, t, m, nl);
@@ -215,16 +233,20 @@ __global__ void __launch_bounds__(kLinThreads) linear_skinny_kernel(const LinArg
     }
 }
 
-template <int RB, int MB>
-void launch_linear(const LinArgs& a, hipStream_t st) {
+// whether every wavefront has the 2 stages a 3-slot ring needs
+template <typename T>
+bool deep_ring(const LinArgs<T>& a) { return a.K / a.KS / kCols<T> / kLinWaves >= 2; }
+
+template <int RB, int MB, typename T>
+void launch_linear(const LinArgs<T>& a, hipStream_t st) {
     dim3 grid((unsigned)((a.N + 16 * RB - 1) / (16 * RB)), (unsigned)a.KS, (unsigned)((a.M + 16 * MB - 1) / (16 * MB)));
     // 64 rows of x: a 2-stage ring (80 KB of LDS at 16 W rows, 96 KB at 32)
     if constexpr (MB > 2)
-        hipLaunchKernelGGL((linear_skinny_kernel<RB, MB, 2>), grid, dim3(kLinThreads), 0, st, a);
-    else if (a.K / a.KS >= 2 * kKC)
-        hipLaunchKernelGGL((linear_skinny_kernel<RB, MB, 3>), grid, dim3(kLinThreads), 0, st, a);
+        hipLaunchKernelGGL((linear_skinny_kernel<RB, MB, 2, T>), grid, dim3(kLinThreads), 0, st, a);
+    else if (deep_ring(a))
+        hipLaunchKernelGGL((linear_skinny_kernel<RB, MB, 3, T>), grid, dim3(kLinThreads), 0, st, a);
     else
-        hipLaunchKernelGGL((linear_skinny_kernel<RB, MB, 2>), grid, dim3(kLinThreads), 0, st, a);
+        hipLaunchKernelGGL((linear_skinny_kernel<RB, MB, 2, T>), grid, dim3(kLinThreads), 0, st, a);
 }
 
 // ------------------------------------------------------- out_proj + residual add + the next norm's inputs
@@ -254,10 +276,11 @@ void launch_linear(const LinArgs& a, hipStream_t st) {
 // every workgroup loads its pairs' h and w before it counts.  Counters start
 // at zero and each is taken by exactly KS workgroups of one launch; nothing
 // is reset, so a call needs its own zeroed counters.
+template <typename T>
 struct ResidArgs {
     float* h;          // [M, N] residual rows, in place
-    const float* w;    // [N] next RMSNorm's weight
-    float* xn;         // [M, N]
+    const T* w;        // [N] next RMSNorm's weight
+    T* xn;             // [M, N]
     float* sq;         // [N / (16 RB), M]
     unsigned* cnt;     // [N / (16 RB)], zero on entry
 };
@@ -276,8 +299,8 @@ __device__ __forceinline__ F4v load_coherent(const float* p) {
     return v;
 }
 
-template <int RB, int MB, int D>
-__global__ void __launch_bounds__(kLinThreads) linear_resid_kernel(const LinArgs a, const ResidArgs r) {
+template <int RB, int MB, int D, typename T>
+__global__ void __launch_bounds__(kLinThreads) linear_resid_kernel(const LinArgs<T> a, const ResidArgs<T> r) {
     constexpr int WR = 16 * RB, NPAIR = RB * MB * 64;
     __shared__ __align__(16) float ring[ring_floats<RB, MB, D>()];
     static_assert(sizeof(ring) >= sizeof(float) * (16 * MB * 4 * RB + 4), "epilogue space");
@@ -299,7 +322,7 @@ __global__ void __launch_bounds__(kLinThreads) linear_resid_kernel(const LinArgs
         hv = ld4(r.h + (int64_t)min(m, a.M - 1) * a.N + n0 + nl);
         wv = ld4(r.w + n0 + nl);
     }
-    skinny_tile<RB, MB, D>(a, ring, n0, ks);
+    skinny_tile<RB, MB, D, T>(a, ring, n0, ks);
     asm volatile("" : "+v"(bv), "+v"(hv), "+v"(wv));   // consumed after the product only
     F4v own = {0.f, 0.f, 0.f, 0.f};
     if (has_pair) {
@@ -330,7 +353,7 @@ __global__ void __launch_bounds__(kLinThreads) linear_resid_kernel(const LinArgs
         hv += t;
         const int64_t o = (int64_t)m * a.N + n0 + nl;
         *reinterpret_cast<F4v*>(r.h + o) = hv;
-        *reinterpret_cast<F4v*>(r.xn + o) = hv * wv;
+        st4(r.xn + o, hv * wv);
         float s = 0.f;
 #pragma unroll
         for (int q = 0; q < 4; ++q) s = fmaf(hv[q], hv[q], s);
@@ -345,13 +368,13 @@ __global__ void __launch_bounds__(kLinThreads) linear_resid_kernel(const LinArgs
     }
 }
 
-template <int RB, int MB>
-void launch_resid(const LinArgs& a, const ResidArgs& r, hipStream_t st) {
+template <int RB, int MB, typename T>
+void launch_resid(const LinArgs<T>& a, const ResidArgs<T>& r, hipStream_t st) {
     dim3 grid((unsigned)(a.N / (16 * RB)), (unsigned)a.KS);
-    if (a.K / a.KS >= 2 * kKC)
-        hipLaunchKernelGGL((linear_resid_kernel<RB, MB, 3>), grid, dim3(kLinThreads), 0, st, a, r);
+    if (deep_ring(a))
+        hipLaunchKernelGGL((linear_resid_kernel<RB, MB, 3, T>), grid, dim3(kLinThreads), 0, st, a, r);
     else
-        hipLaunchKernelGGL((linear_resid_kernel<RB, MB, 2>), grid, dim3(kLinThreads), 0, st, a, r);
+        hipLaunchKernelGGL((linear_resid_kernel<RB, MB, 2, T>), grid, dim3(kLinThreads), 0, st, a, r);
 }
 
 // ------------------------------------------------------- in_proj + conv step + x_proj partials
@@ -378,13 +401,14 @@ void launch_resid(const LinArgs& a, const ResidArgs& r, hipStream_t st) {
 // per-tile sums of h^2 of each row: the tile's in_proj outputs are scaled by
 // rsqrt(sum / d_model + eps) before the bias, which is in_proj applied to
 // RMSNorm(h) (model.py:130-135), the norm taken on the dot products.
+template <typename T>
 struct InConvArgs {
-    float* state;            // [b, D, K - 1], in place
-    const float* conv_w;     // [D, K]
-    const float* conv_b;     // [D] or null
-    const float* WxT;        // [D, J]
-    float* xc;               // [b, D]
-    float* z;                // [b, D] rows at stride z_rs
+    T* state;                // [b, D, K - 1], in place
+    const T* conv_w;         // [D, K]
+    const T* conv_b;         // [D] or null
+    const T* WxT;            // [D, J]
+    T* xc;                   // [b, D]
+    T* z;                    // [b, D] rows at stride z_rs
     float* xpart;            // [D / CB, b, J]
     const float* sq;         // [nsq, b] or null
     int64_t z_rs;
@@ -395,18 +419,22 @@ struct InConvArgs {
 constexpr int kIcMaxJ = 288;
 constexpr int kSqPerThread = 16;                 // nsq <= 8 kSqPerThread
 
-template <int RB, int MB, int D, int K, int NBJ>
-__global__ void __launch_bounds__(kLinThreads) in_conv_xproj_kernel(const LinArgs a, const InConvArgs c) {
+// bf16: the in_proj output and xc are rounded to bf16 where they are used
+// (the conv, the x_proj partial) as well as where they are stored, as the
+// separate bf16 ops round them; the partials and their sum stay fp32.
+template <int RB, int MB, int D, int K, int NBJ, typename T>
+__global__ void __launch_bounds__(kLinThreads) in_conv_xproj_kernel(const LinArgs<T> a, const InConvArgs<T> c) {
     constexpr int CB = 16 * RB, XR = 16 * MB;           // channels of a tile, rows of x
     constexpr int RING = ring_floats<RB, MB, D>();
-    constexpr int WXF = (CB * 16 * NBJ + 255) / 256 * 256;   // W_xT tile space, whole 1 KB copies
+    constexpr int EPC = 1024 / (int)sizeof(T);          // elements of a 1 KB copy
+    constexpr int WXF = (CB * 16 * NBJ + EPC - 1) / EPC * 256;   // W_xT tile space in floats, whole copies
     // All of the kernel's LDS is one array: with a second LDS array the
     // compiler can no longer tell the ring reads from the copies' LDS writes
     // and drains vmcnt to zero before every stage (1.4b width: 28.9 us
     // against 17 us for the plain product).
     __shared__ __align__(16) float lds[RING + WXF];
     float* ring = lds;
-    float* s_wx = lds + RING;                          // [CB][J]
+    T* s_wx = reinterpret_cast<T*>(lds + RING);        // [CB][J]
     constexpr int kAcc = kLinWaves * RB * MB * 64 * 4;  // floats of the reduction space
     static_assert(kAcc + XR * (CB + 1) + 8 * 32 <= RING, "epilogue space");
     static_assert(XR <= 32, "row scales for at most 32 rows");
@@ -421,12 +449,12 @@ __global__ void __launch_bounds__(kLinThreads) in_conv_xproj_kernel(const LinArg
     if (xtile) {
         // the tile's W_xT block, 1 KB per copy, copies dealt to the wavefronts;
         // lanes past the block re-read its last 16 bytes into the padding
-        const int nf = CB * J;                         // a multiple of 4
-        const float* src = c.WxT + (int64_t)n0 * J;
-        for (int ch = wave; ch * 256 < nf; ch += kLinWaves) {
-            const int f = min(ch * 256 + 4 * lane, nf - 4);
+        const int nf = CB * J;                         // a multiple of 16 bytes
+        const T* src = c.WxT + (int64_t)n0 * J;
+        for (int ch = wave; ch * EPC < nf; ch += kLinWaves) {
+            const int f = min(ch * EPC + EPC / 64 * lane, nf - EPC / 64);
 #if defined(__HIP_DEVICE_COMPILE__)
-            __builtin_amdgcn_global_load_lds(src + f, s_wx + ch * 256, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(src + f, s_wx + ch * EPC, 16, 0, 0);
 #else
             (void)f;
 #endif
@@ -445,7 +473,7 @@ __global__ void __launch_bounds__(kLinThreads) in_conv_xproj_kernel(const LinArg
         for (int i = 0; i < kSqPerThread; ++i) sv[i] = c.sq[(int64_t)min(sg + 8 * i, c.nsq - 1) * a.M + sm];
     }
 
-    skinny_tile<RB, MB, D>(a, ring, n0, 0);
+    skinny_tile<RB, MB, D, T>(a, ring, n0, 0);
 
     // every thread calls it (normed input only)
     auto row_scale = [&](int m) __attribute__((always_inline)) {
@@ -473,7 +501,7 @@ __global__ void __launch_bounds__(kLinThreads) in_conv_xproj_kernel(const LinArg
         if (c.sq) v *= row_scale(m);
         if (has_pair && m < a.M) {
             if (a.bias) v += ld4(a.bias + n0 + nl);
-            *reinterpret_cast<F4v*>(c.z + m * c.z_rs + (n0 + nl - c.D)) = v;
+            st4(c.z + m * c.z_rs + (n0 + nl - c.D), v);
         }
         return;
     }
@@ -489,12 +517,12 @@ __global__ void __launch_bounds__(kLinThreads) in_conv_xproj_kernel(const LinArg
         v = tile_sum<RB, MB>(ring, t, m, nl);
         ch = n0 + nl;
         const int mm = min(m, a.M - 1);
-        const F4v* sp = reinterpret_cast<const F4v*>(c.state + ((int64_t)mm * c.D + ch) * (K - 1));
+        const T* sp = c.state + ((int64_t)mm * c.D + ch) * (K - 1);
 #pragma unroll
-        for (int k = 0; k < K - 1; ++k) hist[k] = sp[k];
-        const F4v* wp = reinterpret_cast<const F4v*>(c.conv_w + (int64_t)ch * K);
+        for (int k = 0; k < K - 1; ++k) hist[k] = ld4(sp + 4 * k);
+        const T* wp = c.conv_w + (int64_t)ch * K;
 #pragma unroll
-        for (int k = 0; k < K; ++k) cw[k] = wp[k];
+        for (int k = 0; k < K; ++k) cw[k] = ld4(wp + 4 * k);
         if (c.conv_b) cb = ld4(c.conv_b + ch);
     }
     if (c.sq) v *= row_scale(m);
@@ -507,12 +535,12 @@ __global__ void __launch_bounds__(kLinThreads) in_conv_xproj_kernel(const LinArg
             float win[K];
 #pragma unroll
             for (int k = 0; k < K - 1; ++k) win[k] = hist[(q * (K - 1) + k) / 4][(q * (K - 1) + k) % 4];
-            win[K - 1] = v[q];
+            win[K - 1] = round_to<T>(v[q]);
             float acc = 0.f;
 #pragma unroll
             for (int k = 0; k < K; ++k) acc = fmaf(win[k], cw[(q * K + k) / 4][(q * K + k) % 4], acc);
             acc += cb[q];
-            xcv[q] = silu_f(acc);
+            xcv[q] = round_to<T>(silu_f(acc));
 #pragma unroll
             for (int k = 0; k < K - 1; ++k) nh[(q * (K - 1) + k) / 4][(q * (K - 1) + k) % 4] = win[k + 1];
         }
@@ -544,7 +572,7 @@ __global__ void __launch_bounds__(kLinThreads) in_conv_xproj_kernel(const LinArg
 #pragma unroll
         for (int i = 0; i < JPW; ++i) {
             const int jr = min(16 * (wave + kLinWaves * i) + r, J - 1);
-            const float bv = s_wx[(4 * s4 + kk) * J + jr];
+            const float bv = Act<T>::load(s_wx + (4 * s4 + kk) * J + jr);
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
                 acc[i][mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s4][mb], bv, acc[i][mb], 0, 0, 0);
@@ -564,10 +592,10 @@ __global__ void __launch_bounds__(kLinThreads) in_conv_xproj_kernel(const LinArg
         }
     }
     if (has_pair && m < a.M) {
-        F4v* spo = reinterpret_cast<F4v*>(c.state + ((int64_t)m * c.D + ch) * (K - 1));
+        T* spo = c.state + ((int64_t)m * c.D + ch) * (K - 1);
 #pragma unroll
-        for (int k = 0; k < K - 1; ++k) spo[k] = nh[k];
-        *reinterpret_cast<F4v*>(c.xc + (int64_t)m * c.D + ch) = xcv;
+        for (int k = 0; k < K - 1; ++k) st4(spo + 4 * k, nh[k]);
+        st4(c.xc + (int64_t)m * c.D + ch, xcv);
     }
 }
 
@@ -597,7 +625,7 @@ struct PrefillConvArgs {
 };
 
 template <int RB, int K>
-__global__ void __launch_bounds__(kLinThreads) in_conv_prefill_kernel(const LinArgs a, const PrefillConvArgs c) {
+__global__ void __launch_bounds__(kLinThreads) in_conv_prefill_kernel(const LinArgs<float> a, const PrefillConvArgs c) {
     constexpr int MB = 4, DEPTH = 2;
     constexpr int CB = 16 * RB, XR = 16 * MB;
     constexpr int RING = ring_floats<RB, MB, DEPTH>();
@@ -633,7 +661,7 @@ __global__ void __launch_bounds__(kLinThreads) in_conv_prefill_kernel(const LinA
         }
     }
 
-    skinny_tile<RB, MB, DEPTH>(a, ring, n0, 0);
+    skinny_tile<RB, MB, DEPTH, float>(a, ring, n0, 0);
 
     for (int t = tid; t < RB * MB * 64; t += kLinThreads) {
         int m, nl;
@@ -675,23 +703,23 @@ __global__ void __launch_bounds__(kLinThreads) in_conv_prefill_kernel(const LinA
     }
 }
 
-template <int RB, int MB, int K, int NBJ>
-void launch_in_conv(const LinArgs& a, const InConvArgs& c, hipStream_t st) {
-    hipLaunchKernelGGL((in_conv_xproj_kernel<RB, MB, 3, K, NBJ>), dim3((unsigned)(a.N / (16 * RB))),
+template <int RB, int MB, int K, int NBJ, typename T>
+void launch_in_conv(const LinArgs<T>& a, const InConvArgs<T>& c, hipStream_t st) {
+    hipLaunchKernelGGL((in_conv_xproj_kernel<RB, MB, 3, K, NBJ, T>), dim3((unsigned)(a.N / (16 * RB))),
                        dim3(kLinThreads), 0, st, a, c);
 }
 
 // NBJ = 16-column blocks of x_proj's output: the smallest of 2, 6, 10, 18 that covers J
-template <int RB, int MB, int K>
-void dispatch_in_conv_j(int J, const LinArgs& a, const InConvArgs& c, hipStream_t st) {
+template <int RB, int MB, int K, typename T>
+void dispatch_in_conv_j(int J, const LinArgs<T>& a, const InConvArgs<T>& c, hipStream_t st) {
     if (J <= 32) launch_in_conv<RB, MB, K, 2>(a, c, st);
     else if (J <= 96) launch_in_conv<RB, MB, K, 6>(a, c, st);
     else if (J <= 160) launch_in_conv<RB, MB, K, 10>(a, c, st);
     else launch_in_conv<RB, MB, K, 18>(a, c, st);
 }
 
-template <int RB, int MB>
-void dispatch_in_conv(int K, const LinArgs& a, const InConvArgs& c, hipStream_t st) {
+template <int RB, int MB, typename T>
+void dispatch_in_conv(int K, const LinArgs<T>& a, const InConvArgs<T>& c, hipStream_t st) {
     if (K == 2) dispatch_in_conv_j<RB, MB, 2>(c.J, a, c, st);
     else if (K == 3) dispatch_in_conv_j<RB, MB, 3>(c.J, a, c, st);
     else dispatch_in_conv_j<RB, MB, 4>(c.J, a, c, st);
@@ -702,23 +730,38 @@ void dispatch_in_conv(int K, const LinArgs& a, const InConvArgs& c, hipStream_t 
 
 using namespace mtl;
 
-extern "C" int mtl_linear_skinny(const float* x, int64_t x_rs, const float* W, const float* bias, float* y,
-                                 int64_t y_rs, int64_t y_ks, int64_t M, int64_t N, int64_t K, int32_t ksplit,
-                                 int32_t rows_per_block, mtl_stream_t stream) {
-    clear_error();
+namespace mtl {
+
+// K granules: fp32 deals whole 128-column granules to the four wavefronts,
+// bf16 its 64-column stages, at least one each
+template <typename T>
+bool k_ok(int64_t K, int64_t ksplit) {
+    return K >= 1 && K < (int64_t(1) << 31) &&
+           (sizeof(T) == 4 ? K % (int64_t(kKC) * ksplit) == 0
+                           : K % (int64_t(kCols<T>) * ksplit) == 0 && K / ksplit / kCols<T> >= kLinWaves);
+}
+template <typename T>
+constexpr const char* k_rule() {
+    return sizeof(T) == 4 ? "K must be a positive multiple of 128 * ksplit"
+                          : "K must be a multiple of 64 * ksplit, at least 256 * ksplit";
+}
+
+template <typename T>
+int linear_parts(const T* x, int64_t x_rs, const T* W, const T* bias, float* y, int64_t y_rs, int64_t y_ks, int64_t M,
+                 int64_t N, int64_t K, int32_t ksplit, int32_t rows_per_block, mtl_stream_t stream) {
     MTL_REQUIRE(x && W && y, "null pointer");
     MTL_REQUIRE(M >= 1 && M <= 64 * 65535, "M (rows of x) must be in [1, 4194240]");
     MTL_REQUIRE(N >= 1 && N % 4 == 0 && N < (int64_t(1) << 31), "N must be a positive multiple of 4");
     MTL_REQUIRE(ksplit >= 1 && ksplit <= 64, "ksplit must be in [1, 64]");
-    MTL_REQUIRE(K >= 1 && K % (int64_t(kKC) * ksplit) == 0 && K < (int64_t(1) << 31),
-                "K must be a positive multiple of 128 * ksplit");
+    MTL_REQUIRE(k_ok<T>(K, ksplit), k_rule<T>());
     MTL_REQUIRE(rows_per_block == 16 || rows_per_block == 32, "rows_per_block must be 16 or 32");
     MTL_REQUIRE(x_rs >= K && x_rs % 4 == 0 && y_rs >= N && y_rs % 4 == 0, "row strides must cover a row and be multiples of 4");
+    MTL_REQUIRE(x_rs * (int64_t)sizeof(T) % 16 == 0, "x rows must be 16-byte aligned");
     MTL_REQUIRE(ksplit == 1 || y_ks >= (M - 1) * y_rs + N, "split outputs must not overlap");
     MTL_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(y) |
                  reinterpret_cast<uintptr_t>(bias)) % 16 == 0, "x, W, y and bias must be 16-byte aligned");
     MTL_REQUIRE(y_ks % 4 == 0, "y_ks must be a multiple of 4");
-    LinArgs a{x, W, bias, y, x_rs, y_rs, y_ks, (int)M, (int)N, (int)K, (int)ksplit};
+    LinArgs<T> a{x, W, bias, y, x_rs, y_rs, y_ks, (int)M, (int)N, (int)K, (int)ksplit};
     hipStream_t st = as_stream(stream);
     // 16-row MFMA blocks of x: 1, 2 or 4
     if (rows_per_block == 32) {
@@ -731,6 +774,19 @@ extern "C" int mtl_linear_skinny(const float* x, int64_t x_rs, const float* W, c
         else launch_linear<1, 1>(a, st);
     }
     return check_launch("linear_skinny_kernel");
+}
+template int linear_parts<float>(const float*, int64_t, const float*, const float*, float*, int64_t, int64_t, int64_t,
+                                 int64_t, int64_t, int32_t, int32_t, mtl_stream_t);
+template int linear_parts<uint16_t>(const uint16_t*, int64_t, const uint16_t*, const uint16_t*, float*, int64_t,
+                                    int64_t, int64_t, int64_t, int64_t, int32_t, int32_t, mtl_stream_t);
+
+}  // namespace mtl
+
+extern "C" int mtl_linear_skinny(const float* x, int64_t x_rs, const float* W, const float* bias, float* y,
+                                 int64_t y_rs, int64_t y_ks, int64_t M, int64_t N, int64_t K, int32_t ksplit,
+                                 int32_t rows_per_block, mtl_stream_t stream) {
+    clear_error();
+    return linear_parts<float>(x, x_rs, W, bias, y, y_rs, y_ks, M, N, K, ksplit, rows_per_block, stream);
 }
 
 extern "C" int mtl_in_proj_conv_prefill(const float* x, int64_t x_rs, const float* W_in, const float* b_in,
@@ -750,7 +806,7 @@ extern "C" int mtl_in_proj_conv_prefill(const float* x, int64_t x_rs, const floa
                  reinterpret_cast<uintptr_t>(z)) % 16 == 0, "x, W_in, b_in and z must be 16-byte aligned");
     MTL_REQUIRE(conv_state_in != conv_state_out, "conv_state_out must not alias conv_state_in");
     const int64_t M = batch * seqlen;
-    LinArgs a{x, W_in, b_in, nullptr, x_rs, 0, 0, (int)M, (int)(2 * d_inner), (int)d_model, 1};
+    LinArgs<float> a{x, W_in, b_in, nullptr, x_rs, 0, 0, (int)M, (int)(2 * d_inner), (int)d_model, 1};
     const PrefillConvArgs c{conv_state_in, conv_state_out, conv_w, conv_b, u, z, (int)d_inner, (int)seqlen};
     const dim3 grid((unsigned)(2 * d_inner / 16));
     hipStream_t st = as_stream(stream);
@@ -760,27 +816,28 @@ extern "C" int mtl_in_proj_conv_prefill(const float* x, int64_t x_rs, const floa
     return check_launch("in_conv_prefill_kernel");
 }
 
-extern "C" int mtl_linear_skinny_residual(const float* x, int64_t x_rs, const float* W, const float* bias,
-                                          float* parts, int64_t M, int64_t N, int64_t K, int32_t ksplit,
-                                          int32_t rows_per_block, float* h, const float* w_next, float* x_next,
-                                          float* sq, uint32_t* counters, mtl_stream_t stream) {
-    clear_error();
+namespace mtl {
+
+template <typename T>
+int linear_residual(const T* x, int64_t x_rs, const T* W, const T* bias, float* parts, int64_t M, int64_t N, int64_t K,
+                    int32_t ksplit, int32_t rows_per_block, float* h, const T* w_next, T* x_next, float* sq,
+                    uint32_t* counters, mtl_stream_t stream) {
     MTL_REQUIRE(x && W && parts && h && w_next && x_next && sq && counters, "null required pointer");
     MTL_REQUIRE(M >= 1 && M <= 32, "M (rows of x) must be in [1, 32]");
     MTL_REQUIRE(rows_per_block == 16 || rows_per_block == 32, "rows_per_block must be 16 or 32");
     MTL_REQUIRE(N >= rows_per_block && N % rows_per_block == 0 && N < (int64_t(1) << 30),
                 "N must be a positive multiple of rows_per_block");
     MTL_REQUIRE(ksplit >= 1 && ksplit <= kResidMaxSplit, "ksplit must be in [1, 4]");
-    MTL_REQUIRE(K >= 1 && K % (int64_t(kKC) * ksplit) == 0 && K < (int64_t(1) << 31),
-                "K must be a positive multiple of 128 * ksplit");
+    MTL_REQUIRE(k_ok<T>(K, ksplit), k_rule<T>());
     MTL_REQUIRE(x_rs >= K && x_rs % 4 == 0, "x row stride must cover a row and be a multiple of 4");
+    MTL_REQUIRE(x_rs * (int64_t)sizeof(T) % 16 == 0, "x rows must be 16-byte aligned");
     MTL_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(bias) |
                  reinterpret_cast<uintptr_t>(parts) | reinterpret_cast<uintptr_t>(h) |
                  reinterpret_cast<uintptr_t>(w_next) | reinterpret_cast<uintptr_t>(x_next)) % 16 == 0,
                 "x, W, bias, parts, h, w_next and x_next must be 16-byte aligned");
-    MTL_REQUIRE(x_next != h, "x_next must not alias h");
-    LinArgs a{x, W, bias, parts, x_rs, N, M * N, (int)M, (int)N, (int)K, (int)ksplit};
-    const ResidArgs r{h, w_next, x_next, sq, counters};
+    MTL_REQUIRE(static_cast<const void*>(x_next) != static_cast<const void*>(h), "x_next must not alias h");
+    LinArgs<T> a{x, W, bias, parts, x_rs, N, M * N, (int)M, (int)N, (int)K, (int)ksplit};
+    const ResidArgs<T> r{h, w_next, x_next, sq, counters};
     hipStream_t st = as_stream(stream);
     if (rows_per_block == 32) {
         if (M > 16) launch_resid<2, 2>(a, r, st); else launch_resid<2, 1>(a, r, st);
@@ -789,16 +846,36 @@ extern "C" int mtl_linear_skinny_residual(const float* x, int64_t x_rs, const fl
     }
     return check_launch("linear_resid_kernel");
 }
+template int linear_residual<float>(const float*, int64_t, const float*, const float*, float*, int64_t, int64_t,
+                                    int64_t, int32_t, int32_t, float*, const float*, float*, float*, uint32_t*,
+                                    mtl_stream_t);
+template int linear_residual<uint16_t>(const uint16_t*, int64_t, const uint16_t*, const uint16_t*, float*, int64_t,
+                                       int64_t, int64_t, int32_t, int32_t, float*, const uint16_t*, uint16_t*, float*,
+                                       uint32_t*, mtl_stream_t);
 
-static int in_proj_conv_xproj(const float* x, int64_t x_rs, const float* W_in, const float* b_in, float* conv_state,
-                              const float* conv_w, const float* conv_b, int32_t d_conv, const float* W_xT, int32_t J,
-                              float* xc, float* z, int64_t z_rs, float* xpart, int64_t batch, int64_t d_model,
-                              int64_t d_inner, int32_t channels_per_part, const float* sq, int32_t sq_tiles, float eps,
-                              mtl_stream_t stream) {
+}  // namespace mtl
+
+extern "C" int mtl_linear_skinny_residual(const float* x, int64_t x_rs, const float* W, const float* bias,
+                                          float* parts, int64_t M, int64_t N, int64_t K, int32_t ksplit,
+                                          int32_t rows_per_block, float* h, const float* w_next, float* x_next,
+                                          float* sq, uint32_t* counters, mtl_stream_t stream) {
+    clear_error();
+    return linear_residual<float>(x, x_rs, W, bias, parts, M, N, K, ksplit, rows_per_block, h, w_next, x_next, sq,
+                                  counters, stream);
+}
+
+namespace mtl {
+
+template <typename T>
+int in_proj_conv_xproj(const T* x, int64_t x_rs, const T* W_in, const T* b_in, T* conv_state, const T* conv_w,
+                       const T* conv_b, int32_t d_conv, const T* W_xT, int32_t J, T* xc, T* z, int64_t z_rs,
+                       float* xpart, int64_t batch, int64_t d_model, int64_t d_inner, int32_t channels_per_part,
+                       const float* sq, int32_t sq_tiles, float eps, mtl_stream_t stream) {
     MTL_REQUIRE(x && W_in && conv_state && conv_w && W_xT && xc && z && xpart, "null required pointer");
     MTL_REQUIRE(batch >= 1 && batch <= 32, "batch must be in [1, 32]");
-    MTL_REQUIRE(d_model >= 2 * kKC && d_model % kKC == 0 && d_model < (int64_t(1) << 30),
-                "d_model must be a multiple of 128, at least 256");
+    MTL_REQUIRE(d_model >= 2 * kLinWaves * kCols<T> && d_model % kKC == 0 && d_model < (int64_t(1) << 30),
+                sizeof(T) == 4 ? "d_model must be a multiple of 128, at least 256"
+                               : "d_model must be a multiple of 128, at least 512");
     MTL_REQUIRE(channels_per_part == 16 || channels_per_part == 32, "channels_per_part must be 16 or 32");
     MTL_REQUIRE(d_inner >= channels_per_part && d_inner % channels_per_part == 0 && d_inner < (int64_t(1) << 29),
                 "d_inner must be a positive multiple of channels_per_part");
@@ -806,13 +883,14 @@ static int in_proj_conv_xproj(const float* x, int64_t x_rs, const float* W_in, c
     MTL_REQUIRE(J >= 1 && J <= kIcMaxJ, "J (x_proj rows) must be in [1, 288]");
     MTL_REQUIRE(x_rs >= d_model && x_rs % 4 == 0 && z_rs >= d_inner && z_rs % 4 == 0,
                 "row strides must cover a row and be multiples of 4");
+    MTL_REQUIRE(x_rs * (int64_t)sizeof(T) % 16 == 0, "x rows must be 16-byte aligned");
     MTL_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W_in) | reinterpret_cast<uintptr_t>(b_in) |
                  reinterpret_cast<uintptr_t>(conv_state) | reinterpret_cast<uintptr_t>(conv_w) |
                  reinterpret_cast<uintptr_t>(conv_b) | reinterpret_cast<uintptr_t>(xc) |
                  reinterpret_cast<uintptr_t>(z) | reinterpret_cast<uintptr_t>(W_xT)) % 16 == 0,
                 "x, W_in, b_in, conv_state, conv_w, conv_b, W_xT, xc and z must be 16-byte aligned");
-    LinArgs a{x, W_in, b_in, nullptr, x_rs, 0, 0, (int)batch, (int)(2 * d_inner), (int)d_model, 1};
-    InConvArgs c{conv_state, conv_w, conv_b, W_xT, xc, z, xpart, sq, z_rs, (int)d_inner, (int)J, (int)sq_tiles, eps};
+    LinArgs<T> a{x, W_in, b_in, nullptr, x_rs, 0, 0, (int)batch, (int)(2 * d_inner), (int)d_model, 1};
+    InConvArgs<T> c{conv_state, conv_w, conv_b, W_xT, xc, z, xpart, sq, z_rs, (int)d_inner, (int)J, (int)sq_tiles, eps};
     hipStream_t st = as_stream(stream);
     const bool two_m = batch > 16;
     if (channels_per_part == 32) {
@@ -822,6 +900,15 @@ static int in_proj_conv_xproj(const float* x, int64_t x_rs, const float* W_in, c
     }
     return check_launch("in_conv_xproj_kernel");
 }
+template int in_proj_conv_xproj<float>(const float*, int64_t, const float*, const float*, float*, const float*,
+                                       const float*, int32_t, const float*, int32_t, float*, float*, int64_t, float*,
+                                       int64_t, int64_t, int64_t, int32_t, const float*, int32_t, float, mtl_stream_t);
+template int in_proj_conv_xproj<uint16_t>(const uint16_t*, int64_t, const uint16_t*, const uint16_t*, uint16_t*,
+                                          const uint16_t*, const uint16_t*, int32_t, const uint16_t*, int32_t,
+                                          uint16_t*, uint16_t*, int64_t, float*, int64_t, int64_t, int64_t, int32_t,
+                                          const float*, int32_t, float, mtl_stream_t);
+
+}  // namespace mtl
 
 extern "C" int mtl_in_proj_conv_xproj(const float* x, int64_t x_rs, const float* W_in, const float* b_in,
                                       float* conv_state, const float* conv_w, const float* conv_b, int32_t d_conv,
@@ -829,7 +916,7 @@ extern "C" int mtl_in_proj_conv_xproj(const float* x, int64_t x_rs, const float*
                                       int64_t batch, int64_t d_model, int64_t d_inner, int32_t channels_per_part,
                                       mtl_stream_t stream) {
     clear_error();
-    return in_proj_conv_xproj(x, x_rs, W_in, b_in, conv_state, conv_w, conv_b, d_conv, W_xT, J, xc, z, z_rs, xpart,
+    return in_proj_conv_xproj<float>(x, x_rs, W_in, b_in, conv_state, conv_w, conv_b, d_conv, W_xT, J, xc, z, z_rs, xpart,
                               batch, d_model, d_inner, channels_per_part, nullptr, 0, 0.f, stream);
 }
 
@@ -843,6 +930,6 @@ extern "C" int mtl_in_proj_conv_xproj_normed(const float* x, int64_t x_rs, const
     MTL_REQUIRE(sq, "null sq");
     MTL_REQUIRE(sq_tiles >= 1 && sq_tiles <= 8 * kSqPerThread, "sq_tiles must be in [1, 128]");
     MTL_REQUIRE(eps >= 0.f, "eps must be >= 0");
-    return in_proj_conv_xproj(x, x_rs, W_in, b_in, conv_state, conv_w, conv_b, d_conv, W_xT, J, xc, z, z_rs, xpart,
+    return in_proj_conv_xproj<float>(x, x_rs, W_in, b_in, conv_state, conv_w, conv_b, d_conv, W_xT, J, xc, z, z_rs, xpart,
                               batch, d_model, d_inner, channels_per_part, sq, sq_tiles, eps, stream);
 }

@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "step_ops.h"
 
 namespace mtl {
 namespace {
@@ -27,11 +28,12 @@ constexpr int kChPerBlock = kStepThreads / kLanesPerChannel;
 // so W_dt, A, D and the biases are read once per BB rows.  The BB rows of
 // x_dbl and the block's x, z are staged in LDS by all threads; every other
 // operand is loaded up front with clamped addresses.
-template <typename T, int RQ, int BB>
+// T: x, z and y; X: x_dbl; P: the parameters (each float or bf16 as uint16_t).
+template <typename T, typename X, typename P, int RQ, int BB>
 __global__ void __launch_bounds__(kStepThreads)
 ssm_step_kernel(float* __restrict__ state, const T* __restrict__ x, int64_t x_sb, const T* __restrict__ z,
-                int64_t z_sb, const T* __restrict__ xdbl, int64_t xdbl_sb, const float* __restrict__ Wdt,
-                const float* __restrict__ bdt, const float* __restrict__ A, const float* __restrict__ Dv,
+                int64_t z_sb, const X* __restrict__ xdbl, int64_t xdbl_sb, const P* __restrict__ Wdt,
+                const P* __restrict__ bdt, const P* __restrict__ A, const P* __restrict__ Dv,
                 T* __restrict__ y, int64_t y_sb, int D, int N, int R, int batch, int a_is_log) {
     constexpr int kJMax = 16 * RQ + 2 * kLanesPerChannel;          // R + 2N <= 16 RQ + 32
     constexpr int kStage = (BB * kJMax + kStepThreads - 1) / kStepThreads;
@@ -47,10 +49,10 @@ ssm_step_kernel(float* __restrict__ state, const T* __restrict__ x, int64_t x_sb
 
     float wdt[RQ];
 #pragma unroll
-    for (int q = 0; q < RQ; ++q) wdt[q] = Wdt[(int64_t)cc * R + min(n + 16 * q, R - 1)];
-    float av = A[(int64_t)cc * N + nn];
-    const float bd = bdt[cc];
-    const float Dc = Dv ? Dv[cc] : 0.f;
+    for (int q = 0; q < RQ; ++q) wdt[q] = Act<P>::load(Wdt + (int64_t)cc * R + min(n + 16 * q, R - 1));
+    float av = Act<P>::load(A + (int64_t)cc * N + nn);
+    const float bd = Act<P>::load(bdt + cc);
+    const float Dc = Dv ? Act<P>::load(Dv + cc) : 0.f;
     float hs[BB];
 #pragma unroll
     for (int i = 0; i < BB; ++i) hs[i] = state[((int64_t)min(b0 + i, batch - 1) * D + cc) * N + nn];
@@ -60,7 +62,7 @@ ssm_step_kernel(float* __restrict__ state, const T* __restrict__ x, int64_t x_sb
     for (int q = 0; q < kStage; ++q) {
         const int e = min(tid + q * kStepThreads, BB * J - 1);
         const int i = e / J, j = e - i * J;
-        st[q] = Act<T>::load(xdbl + (int64_t)min(b0 + i, batch - 1) * xdbl_sb + j);
+        st[q] = Act<X>::load(xdbl + (int64_t)min(b0 + i, batch - 1) * xdbl_sb + j);
     }
     const bool xz_t = tid < BB * kChPerBlock;
     const int xi = min(tid / kChPerBlock, BB - 1), xch = tid % kChPerBlock;
@@ -284,10 +286,11 @@ constexpr int kNormThreads = 256;
 // y: NP parts (NP = 0: none) at stride yps, added to each other in part order
 // and then to x -- the split-K partial products of the out_proj before the
 // residual add
-template <int RUNS, int NP>
+// T: the weight and the output.
+template <int RUNS, int NP, typename T>
 __global__ void __launch_bounds__(kNormThreads)
 add_rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ y, int64_t yps, float* x_out,
-                   const float* __restrict__ w, float* __restrict__ normed, int cols, float eps) {
+                   const T* __restrict__ w, T* __restrict__ normed, int cols, float eps) {
     __shared__ float s_part[kNormThreads / 64];
     const int64_t row = blockIdx.x;
     const int tid = threadIdx.x;
@@ -297,7 +300,7 @@ add_rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ y, int
     for (int q = 0; q < RUNS; ++q) {
         const int i = min(tid + q * kNormThreads, cols - 1);
         v[q] = xr[i];
-        wv[q] = w[i];
+        wv[q] = Act<T>::load(w + i);
     }
     if constexpr (NP > 0) {
         float yv[NP][RUNS];
@@ -327,15 +330,16 @@ add_rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ y, int
         const int i = tid + q * kNormThreads;
         if (i < cols) {
             if (x_out) x_out[row * cols + i] = v[q];
-            normed[row * cols + i] = wv[q] * (v[q] * r);
+            Act<T>::store(normed + row * cols + i, wv[q] * (v[q] * r));
         }
     }
 }
 
 // rows longer than 256 * kMaxRuns
+template <typename T>
 __global__ void __launch_bounds__(kNormThreads)
 add_rmsnorm_long_kernel(const float* __restrict__ x, const float* __restrict__ y, int np, int64_t yps, float* x_out,
-                        const float* __restrict__ w, float* __restrict__ normed, int cols, float eps) {
+                        const T* __restrict__ w, T* __restrict__ normed, int cols, float eps) {
     __shared__ float s_part[kNormThreads / 64];
     const int64_t row = blockIdx.x;
     const float* xr = x + row * cols;
@@ -360,7 +364,7 @@ add_rmsnorm_long_kernel(const float* __restrict__ x, const float* __restrict__ y
         float v = xr[i];
         if (yr) v += ysum(i);
         if (x_out) x_out[row * cols + i] = v;
-        normed[row * cols + i] = w[i] * (v * r);
+        Act<T>::store(normed + row * cols + i, Act<T>::load(w + i) * (v * r));
     }
 }
 
@@ -398,14 +402,14 @@ constexpr int64_t kRowsMinBatch = MTL_ROWS_MIN_BATCH;   // the rows form from th
 #define MTL_ROWS_TILE 16
 #endif
 constexpr int kRowsTile = MTL_ROWS_TILE;                  // batch rows per workgroup (16 or 32)
-typedef float F4s __attribute__((ext_vector_type(4)));
+typedef F4v F4s;
 
-template <int KBW, int MB>   // KBW: 16-column blocks of dt_rank per wavefront (dt_rank <= 64 KBW); MB: 16-row blocks
+template <int KBW, int MB, typename T>   // T: x, z, y and the parameters; KBW: 16-column blocks of dt_rank per wavefront (dt_rank <= 64 KBW); MB: 16-row blocks
 __global__ void __launch_bounds__(kStepThreads)
-ssm_step_rows_kernel(float* __restrict__ state, const float* __restrict__ x, int64_t x_sb,
-                     const float* __restrict__ z, int64_t z_sb, const float* __restrict__ xdbl, int64_t xdbl_sb,
-                     const float* __restrict__ Wdt, const float* __restrict__ bdt, const float* __restrict__ A,
-                     const float* __restrict__ Dv, float* __restrict__ y, int64_t y_sb, int D, int R, int batch,
+ssm_step_rows_kernel(float* __restrict__ state, const T* __restrict__ x, int64_t x_sb,
+                     const T* __restrict__ z, int64_t z_sb, const float* __restrict__ xdbl, int64_t xdbl_sb,
+                     const T* __restrict__ Wdt, const T* __restrict__ bdt, const T* __restrict__ A,
+                     const T* __restrict__ Dv, T* __restrict__ y, int64_t y_sb, int D, int R, int batch,
                      int a_is_log) {
     constexpr int N = 16, TR = 16 * MB;               // rows per workgroup
     __shared__ __align__(16) F4s s_dt[kStepThreads / 64][MB][64];
@@ -417,7 +421,7 @@ ssm_step_rows_kernel(float* __restrict__ state, const float* __restrict__ x, int
     // ---- every independent load first
     const int r16 = lane & 15, kk = lane >> 4;
     const int nkb = R / 16;
-    const float* wrow = Wdt + (int64_t)min(c0 + r16, D - 1) * R + 4 * kk;
+    const T* wrow = Wdt + (int64_t)min(c0 + r16, D - 1) * R + 4 * kk;
     const float* xr[MB];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) xr[mb] = xdbl + (int64_t)min(b0 + 16 * mb + r16, batch - 1) * xdbl_sb + 4 * kk;
@@ -425,7 +429,7 @@ ssm_step_rows_kernel(float* __restrict__ state, const float* __restrict__ x, int
 #pragma unroll
     for (int j = 0; j < KBW; ++j) {
         const int kc = min(wave + 4 * j, nkb - 1) * 16;
-        wv[j] = *reinterpret_cast<const F4s*>(wrow + kc);
+        wv[j] = ld4(wrow + kc);
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) xo[j][mb] = *reinterpret_cast<const F4s*>(xr[mb] + kc);
     }
@@ -443,13 +447,13 @@ ssm_step_rows_kernel(float* __restrict__ state, const float* __restrict__ x, int
             const F4s v = sp[q];
             hs[u][4 * q] = v.x; hs[u][4 * q + 1] = v.y; hs[u][4 * q + 2] = v.z; hs[u][4 * q + 3] = v.w;
         }
-        xv[u] = x[brow[u] * x_sb + cg];
-        zv[u] = z ? z[brow[u] * z_sb + cg] : 0.f;
+        xv[u] = Act<T>::load(x + brow[u] * x_sb + cg);
+        zv[u] = z ? Act<T>::load(z + brow[u] * z_sb + cg) : 0.f;
     }
-    const float bd = bdt[cg];
-    const float Dc = Dv ? Dv[cg] : 0.f;
+    const float bd = Act<T>::load(bdt + cg);
+    const float Dc = Dv ? Act<T>::load(Dv + cg) : 0.f;
     // A of (channel tid / 16, state tid % 16), in log2 units
-    float av = A[(int64_t)min(c0 + (tid >> 4), D - 1) * N + (tid & 15)];
+    float av = Act<T>::load(A + (int64_t)min(c0 + (tid >> 4), D - 1) * N + (tid & 15));
     // B | C of row tid / 8, columns 4 (tid % 8) .. + 3
     const int bcr = tid >> 3, bcj = 4 * (tid & 7);
     const F4s bc = *reinterpret_cast<const F4s*>(xdbl + (int64_t)min(b0 + min(bcr, TR - 1), batch - 1) * xdbl_sb + R +
@@ -501,24 +505,23 @@ ssm_step_rows_kernel(float* __restrict__ state, const float* __restrict__ x, int
                 sp[q] = F4s{hs[u][4 * q], hs[u][4 * q + 1], hs[u][4 * q + 2], hs[u][4 * q + 3]};
             yv = fmaf(xv[u], Dc, yv);
             if (z) yv *= silu_f(zv[u]);
-            y[(int64_t)(b0 + r) * y_sb + c0 + pc] = yv;
+            Act<T>::store(y + (int64_t)(b0 + r) * y_sb + c0 + pc, yv);
         }
     }
 }
 
-template <typename T>
-void launch_ssm_step(float* state, const void* x, int64_t x_sb, const void* z, int64_t z_sb, const void* xdbl,
-                     int64_t xdbl_sb, const float* Wdt, const float* bdt, const float* A, const float* Dv, void* y,
-                     int64_t y_sb, int64_t batch, int D, int N, int R, int a_is_log, hipStream_t st) {
-    if constexpr (std::is_same<T, float>::value) {
+template <typename T, typename X, typename P>
+void launch_ssm_step(float* state, const T* x, int64_t x_sb, const T* z, int64_t z_sb, const X* xdbl, int64_t xdbl_sb,
+                     const P* Wdt, const P* bdt, const P* A, const P* Dv, T* y, int64_t y_sb, int64_t batch, int D,
+                     int N, int R, int a_is_log, hipStream_t st) {
+    if constexpr (std::is_same<X, float>::value && std::is_same<T, P>::value) {
         const bool aligned = ((uintptr_t)state | (uintptr_t)xdbl | (uintptr_t)Wdt) % 16 == 0 && xdbl_sb % 4 == 0;
         if (batch >= kRowsMinBatch && N == 16 && R % 16 == 0 && R <= 256 && aligned) {
             const int tr = kRowsTile;
             dim3 grid((unsigned)((D + kRowsCh - 1) / kRowsCh), (unsigned)((batch + tr - 1) / tr));
             const int kbw = (R / 16 + 3) / 4;
-#define MTL_ROWS(KB) hipLaunchKernelGGL((ssm_step_rows_kernel<KB, kRowsTile / 16>), grid, dim3(kStepThreads), 0, st, state, \
-        static_cast<const float*>(x), x_sb, static_cast<const float*>(z), z_sb, static_cast<const float*>(xdbl),      \
-        xdbl_sb, Wdt, bdt, A, Dv, static_cast<float*>(y), y_sb, D, R, (int)batch, a_is_log)
+#define MTL_ROWS(KB) hipLaunchKernelGGL((ssm_step_rows_kernel<KB, kRowsTile / 16, T>), grid, dim3(kStepThreads), 0, st, \
+        state, x, x_sb, z, z_sb, xdbl, xdbl_sb, Wdt, bdt, A, Dv, y, y_sb, D, R, (int)batch, a_is_log)
             if (kbw <= 1) MTL_ROWS(1);
             else if (kbw == 2) MTL_ROWS(2);
             else if (kbw == 3) MTL_ROWS(3);
@@ -530,13 +533,32 @@ void launch_ssm_step(float* state, const void* x, int64_t x_sb, const void* z, i
     const int bb = batch >= 8 ? 8 : batch >= 4 ? 4 : batch >= 2 ? 2 : 1;
     const int rq = round_runs((R + 15) / 16);
     dim3 grid((unsigned)((D + kChPerBlock - 1) / kChPerBlock), (unsigned)((batch + bb - 1) / bb));
-    MTL_DISPATCH_BB(bb, MTL_DISPATCH_RUNS(RQ, rq, hipLaunchKernelGGL((ssm_step_kernel<T, RQ, BB>), grid,
-        dim3(kStepThreads), 0, st, state, static_cast<const T*>(x), x_sb, static_cast<const T*>(z), z_sb,
-        static_cast<const T*>(xdbl), xdbl_sb, Wdt, bdt, A, Dv, static_cast<T*>(y), y_sb, D, N, R, (int)batch,
+    MTL_DISPATCH_BB(bb, MTL_DISPATCH_RUNS(RQ, rq, hipLaunchKernelGGL((ssm_step_kernel<T, X, P, RQ, BB>), grid,
+        dim3(kStepThreads), 0, st, state, x, x_sb, z, z_sb, xdbl, xdbl_sb, Wdt, bdt, A, Dv, y, y_sb, D, N, R, (int)batch,
         a_is_log)));
 }
 
 }  // namespace
+
+template <typename T>
+int state_update(float* ssm_state, const T* x, int64_t x_sb, const T* z, int64_t z_sb, const float* x_dbl,
+                 int64_t xdbl_sb, const T* W_dt, const T* b_dt, const T* A_log, const T* Dvec, T* y, int64_t y_sb,
+                 int64_t batch, int64_t dim, int64_t dstate, int64_t dt_rank, mtl_stream_t stream) {
+    MTL_REQUIRE(batch >= 1 && batch <= 65535 && dim >= 1 && dim < (int64_t(1) << 31), "size out of range");
+    MTL_REQUIRE(dstate >= 1 && dstate <= kLanesPerChannel && dt_rank >= 1 && dt_rank <= 16 * kMaxRuns,
+                "dstate must be in [1, 16] and dt_rank in [1, 256]");
+    MTL_REQUIRE(ssm_state && x && x_dbl && W_dt && b_dt && A_log && y, "null required pointer");
+    launch_ssm_step<T, float, T>(ssm_state, x, x_sb, z, z_sb, x_dbl, xdbl_sb, W_dt, b_dt, A_log, Dvec, y, y_sb, batch,
+                                 (int)dim, (int)dstate, (int)dt_rank, 1, as_stream(stream));
+    return check_launch("selective_state_update");
+}
+template int state_update<float>(float*, const float*, int64_t, const float*, int64_t, const float*, int64_t,
+                                 const float*, const float*, const float*, const float*, float*, int64_t, int64_t,
+                                 int64_t, int64_t, int64_t, mtl_stream_t);
+template int state_update<uint16_t>(float*, const uint16_t*, int64_t, const uint16_t*, int64_t, const float*, int64_t,
+                                    const uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*,
+                                    int64_t, int64_t, int64_t, int64_t, int64_t, mtl_stream_t);
+
 }  // namespace mtl
 
 extern "C" int mtl_selective_state_update(float* ssm_state, const void* x, int64_t x_sb, const void* z, int64_t z_sb,
@@ -555,26 +577,32 @@ extern "C" int mtl_selective_state_update(float* ssm_state, const void* x, int64
     MTL_REQUIRE(dt_rank >= 1 && dt_rank <= 16 * kMaxRuns, "dt_rank must be in [1, 256]");
     hipStream_t st = as_stream(stream);
     if (dtype == MTL_F32)
-        launch_ssm_step<float>(ssm_state, x, x_sb, z, z_sb, x_dbl, xdbl_sb, W_dt, b_dt, A, Dvec, y, y_sb, batch,
-                               (int)dim, (int)dstate, (int)dt_rank, a_is_log, st);
+        launch_ssm_step<float, float, float>(ssm_state, static_cast<const float*>(x), x_sb,
+                                             static_cast<const float*>(z), z_sb, static_cast<const float*>(x_dbl),
+                                             xdbl_sb, W_dt, b_dt, A, Dvec, static_cast<float*>(y), y_sb, batch,
+                                             (int)dim, (int)dstate, (int)dt_rank, a_is_log, st);
     else
-        launch_ssm_step<uint16_t>(ssm_state, x, x_sb, z, z_sb, x_dbl, xdbl_sb, W_dt, b_dt, A, Dvec, y, y_sb, batch,
-                                  (int)dim, (int)dstate, (int)dt_rank, a_is_log, st);
+        launch_ssm_step<uint16_t, uint16_t, float>(ssm_state, static_cast<const uint16_t*>(x), x_sb,
+                                                   static_cast<const uint16_t*>(z), z_sb,
+                                                   static_cast<const uint16_t*>(x_dbl), xdbl_sb, W_dt, b_dt, A, Dvec,
+                                                   static_cast<uint16_t*>(y), y_sb, batch, (int)dim, (int)dstate,
+                                                   (int)dt_rank, a_is_log, st);
     return check_launch("selective_state_update");
 }
 
 namespace mtl {
 namespace {
-int add_rmsnorm_launch(const float* x, const float* y, int32_t nparts, int64_t yps, float* x_out, const float* w,
-                       float* normed, int64_t rows, int64_t cols, float eps, hipStream_t st) {
+template <typename T>
+int add_rmsnorm_launch(const float* x, const float* y, int32_t nparts, int64_t yps, float* x_out, const T* w,
+                       T* normed, int64_t rows, int64_t cols, float eps, hipStream_t st) {
     const int runs = (int)((cols + kNormThreads - 1) / kNormThreads);
     const int np = y ? nparts : 0;
     if (runs > kMaxRuns || (np != 0 && np != 1 && np != 2 && np != 4)) {
-        hipLaunchKernelGGL(add_rmsnorm_long_kernel, dim3((unsigned)rows), dim3(kNormThreads), 0, st, x, y, np, yps,
+        hipLaunchKernelGGL((add_rmsnorm_long_kernel<T>), dim3((unsigned)rows), dim3(kNormThreads), 0, st, x, y, np, yps,
                            x_out, w, normed, (int)cols, eps);
     } else {
 #define MTL_NORM_NP(NPV)                                                                                             \
-    MTL_DISPATCH_RUNS(RUNS, round_runs(runs), hipLaunchKernelGGL((add_rmsnorm_kernel<RUNS, NPV>), dim3((unsigned)rows), \
+    MTL_DISPATCH_RUNS(RUNS, round_runs(runs), hipLaunchKernelGGL((add_rmsnorm_kernel<RUNS, NPV, T>), dim3((unsigned)rows), \
                                                                  dim3(kNormThreads), 0, st, x, y, yps, x_out, w,       \
                                                                  normed, (int)cols, eps))
         if (np == 0) { MTL_NORM_NP(0); }
@@ -586,6 +614,21 @@ int add_rmsnorm_launch(const float* x, const float* y, int32_t nparts, int64_t y
     return check_launch("add_rmsnorm");
 }
 }  // namespace
+
+template <typename T>
+int add_rmsnorm(const float* x, const float* parts, int32_t nparts, float* x_out, const T* w, T* normed, int64_t rows,
+                int64_t cols, float eps, mtl_stream_t stream) {
+    MTL_REQUIRE(rows >= 0 && cols >= 1 && cols < (int64_t(1) << 31), "size out of range");
+    MTL_REQUIRE(rows < (int64_t(1) << 31), "too many rows");
+    MTL_REQUIRE(nparts >= 0 && nparts <= 64 && (nparts == 0) == (parts == nullptr), "nparts must be in [0, 64]");
+    if (rows == 0) return MTL_OK;
+    MTL_REQUIRE(x && w && normed, "null required pointer");
+    return add_rmsnorm_launch<T>(x, parts, nparts, rows * cols, x_out, w, normed, rows, cols, eps, as_stream(stream));
+}
+template int add_rmsnorm<float>(const float*, const float*, int32_t, float*, const float*, float*, int64_t, int64_t,
+                                float, mtl_stream_t);
+template int add_rmsnorm<uint16_t>(const float*, const float*, int32_t, float*, const uint16_t*, uint16_t*, int64_t,
+                                   int64_t, float, mtl_stream_t);
 }  // namespace mtl
 
 extern "C" int mtl_add_rmsnorm(const float* x, const float* y, float* x_out, const float* w, float* normed,

@@ -120,7 +120,7 @@ class DecodeStepBatchedArgs(ctypes.Structure):
         ("h", _vp), ("normed_out", _vp), ("norm_f", _vp), ("inp", _vp), ("xn", _vp), ("xc", _vp), ("z", _vp),
         ("y", _vp), ("xpart", _vp), ("x_dbl", _vp), ("parts", _vp), ("sq", _vp), ("counters", _vp),
         ("eps_f", ctypes.c_float), ("n_layers", _i32), ("batch", _i32), ("d_model", _i32), ("d_inner", _i32),
-        ("d_state", _i32), ("dt_rank", _i32), ("d_conv", _i32), ("fold", _i32), ("reserved", _i32),
+        ("d_state", _i32), ("dt_rank", _i32), ("d_conv", _i32), ("fold", _i32), ("dtype", _i32),
     ]
 
 

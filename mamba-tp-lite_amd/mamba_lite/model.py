@@ -184,7 +184,11 @@ DECODE_STEP_NATIVE = True
 # runs its layer stack as one C call too (mtl_decode_step_batched) when
 # every layer takes the per-op path's in_proj + conv + x_proj launch and
 # split out_proj: the same launches with the same tile choices, so the same
-# bits, without the ~5 Python-launched ops per layer.
+# bits, without the ~5 Python-launched ops per layer.  A bfloat16 model takes
+# the call at any batch up to 32: the same launches on bf16 operands, in place
+# of library GEMMs, separate conv and SSM ops and a float copy of every small
+# parameter per step (8 layers at the mamba-1.4b width, batch 8, captured:
+# 663 -> 303 us per step).
 BATCHED_STEP_NATIVE = True
 
 # With DECODE_PERSIST, the batch-1 fused decode of a model that fits its
@@ -729,7 +733,9 @@ class MambaLM(nn.Module):
             got = self._batched_step_layers(x, cache, lt)
             if got is not None:
                 arr, fold = got
-                normed = ops.decode_step_batched(arr, x, self.norm_f.weight, self.norm_f.eps, self.cfg, fold)
+                h = x if x.dtype == torch.float32 else x.float()
+                normed = ops.decode_step_batched(arr, h, self.norm_f.weight, self.norm_f.eps, self.cfg, fold,
+                                                 dtype=x.dtype)
                 return self.lm_head(normed).unsqueeze(1)
         if self._fold_ok(x, cache):
             return self._step_folded(x, cache)
@@ -812,29 +818,32 @@ class MambaLM(nn.Module):
         this call's cache pointers, whether the residual add + norm fold),
         or None when some layer would not take the per-op path's in_proj +
         conv + x_proj launch and split out_proj, or a weight or cache tensor
-        is not a contiguous float32 tensor of its shape on x's device (the
-        step then runs op by op, with that path's checks and errors).  The
-        weights are checked when their addresses (or x_proj's version, which
+        is not a contiguous tensor of x's dtype (SSM states: float32) and its
+        shape on x's device (the step then runs op by op, with that path's
+        checks and errors).  The weights are checked when their addresses (or x_proj's version, which
         its transposed copy follows) change; the cache tensors every call.
         The fold follows _fold_ok's rule, which on these layers reduces to
         the row count and the out_proj tile."""
         cfg = self.cfg
         nl = len(self.layers)
-        if x.dim() != 2 or x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous() or \
+        act = x.dtype
+        if x.dim() != 2 or act not in (torch.float32, torch.bfloat16) or not x.is_cuda or not x.is_contiguous() or \
                 x.data_ptr() % 16 or len(cache.layers) != nl:
             return None
         b, dm = x.shape
         D, N, K, R = cfg.d_inner, cfg.d_state, cfg.d_conv, cfg.dt_rank
-        if not (1 <= b <= ops.IN_CONV_MAX_ROWS and dm >= 256 and dm % 128 == 0 and D % (128 * SKINNY_OUT_SPLIT) == 0
-                and N <= 16 and R <= 256 and 2 <= K <= 4 and R + 2 * N <= 288):
+        # bf16 stages hold 64 columns per wavefront, fp32 ones 32
+        fits = dm >= 256 and D % (128 * SKINNY_OUT_SPLIT) == 0 if act == torch.float32 else \
+            dm >= 512 and D >= 1024 and D % (64 * SKINNY_OUT_SPLIT) == 0
+        if not (1 <= b <= ops.IN_CONV_MAX_ROWS and fits and dm % 128 == 0 and N <= 16 and R <= 256 and 2 <= K <= 4 and R + 2 * N <= 288):
             return None
         dev = x.device
         lt = self._layer_tensors() if lt is None else lt
-        sig = (dev, dm, tuple(0 if t is None else t.data_ptr() for ts in lt for t in ts),
+        sig = (dev, dm, act, tuple(0 if t is None else t.data_ptr() for ts in lt for t in ts),
                tuple(ts[_LT_XPROJ]._version for ts in lt), self._norm_eps())
         cached = getattr(self, "_batched_tmpl", None)
         if cached is None or cached[0] != sig:
-            cached = (sig, self._batched_template(lt, dev, dm))
+            cached = (sig, self._batched_template(lt, dev, dm, act))
             self._batched_tmpl = cached
         tmpl = cached[1]
         if tmpl is None:
@@ -842,7 +851,7 @@ class MambaLM(nn.Module):
         cs_shape, hs_shape = (b, D, K - 1), (b, D, N)
         for lc in cache.layers:
             cs, hs = lc.conv_state, lc.ssm_state
-            if cs.dtype != torch.float32 or hs.dtype != torch.float32 or cs.shape != cs_shape or \
+            if cs.dtype != act or hs.dtype != torch.float32 or cs.shape != cs_shape or \
                     hs.shape != hs_shape or not cs.is_contiguous() or not hs.is_contiguous() or cs.device != dev or \
                     hs.device != dev or cs.data_ptr() % 16:
                 return None
@@ -854,18 +863,19 @@ class MambaLM(nn.Module):
             dm // rpb <= 128
         return arr, fold
 
-    def _batched_template(self, lt, dev, dm):
+    def _batched_template(self, lt, dev, dm, act):
         """The weight half of _batched_step_layers: mtl_decode_layer records
         (W_xT = x_proj transposed, conv weights as [D, K] views), or None when
-        a weight is not a contiguous float32 tensor of its shape on dev or one
+        a weight is not a contiguous `act` tensor of its shape on dev or one
         the library loads in 16-byte runs (norm, in_proj, conv, out_proj and
         their biases) is not 16-byte aligned."""
         cfg = self.cfg
         D, N, K, R = cfg.d_inner, cfg.d_state, cfg.d_conv, cfg.dt_rank
-        ok = lambda t, shape: t.device == dev and t.dtype == torch.float32 and t.is_contiguous() and \
-            tuple(t.shape) == shape
+        ok = lambda t, shape: t.device == dev and t.dtype == act and t.is_contiguous() and tuple(t.shape) == shape
         opt = lambda t, shape: t is None or ok(t, shape)
         tmpl = (_lib.DecodeLayer * len(lt))()
+        if not ok(self.norm_f.weight, (dm,)) and act != torch.float32:
+            return None
         for i, (ts, L) in enumerate(zip(lt, tmpl)):
             if not (ok(ts[_LT_NORM], (dm,)) and ok(ts[_LT_W_IN], (2 * D, dm)) and opt(ts[_LT_B_IN], (2 * D,))
                     and ok(ts[_LT_CONV_W], (D, 1, K)) and opt(ts[_LT_CONV_B], (D,))

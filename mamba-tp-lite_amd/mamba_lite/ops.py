@@ -655,20 +655,22 @@ def decode_step(layers, ids, emb, norm_f, eps_f, logits, xc, gz, y, xs, xpart, c
     return logits
 
 
-def decode_step_batched(layers, h, norm_f, eps_f, cfg, fold):
+def decode_step_batched(layers, h, norm_f, eps_f, cfg, fold, dtype=torch.float32):
     """mtl_decode_step_batched: a batched step of every layer in one call.
     `layers` is a ctypes array of _lib.DecodeLayer (weights with W_xT, and
     this call's cache pointers); h [b, d_model] float32 holds the step's
     embedding rows and is left holding the final residual stream.  Returns
-    norm_f of it [b, d_model], the tied lm_head's input.  The workspace is
+    norm_f of it [b, d_model], the tied lm_head's input.  dtype: the weights',
+    conv histories' and output's type, float32 or bfloat16.  The workspace is
     allocated here (one float32 tensor, and with fold the zeroed counters)."""
     _f32c(h, "h")
-    _f32c(norm_f, "norm_f")
+    if dtype not in _ACT_DTYPES or norm_f.dtype != dtype or not norm_f.is_contiguous():
+        raise ValueError(f"decode_step_batched: norm_f must be contiguous {dtype} (float32 or bfloat16)")
     if h.dim() != 2 or h.data_ptr() % 16 or h.shape[1] != cfg.d_model:
         raise ValueError(f"decode_step_batched: h must be a 16-byte aligned [b, {cfg.d_model}] tensor")
     b, M = h.shape
     if norm_f.numel() != M or norm_f.device != h.device:
-        raise ValueError(f"decode_step_batched: norm_f must hold {M} floats on {h.device}")
+        raise ValueError(f"decode_step_batched: norm_f must hold {M} values on {h.device}")
     D, J = cfg.d_inner, cfg.dt_rank + 2 * cfg.d_state
     nl = len(layers)
     pad = lambda n: -(-n // 64) * 64                      # 256-byte aligned slices
@@ -685,10 +687,10 @@ def decode_step_batched(layers, h, norm_f, eps_f, cfg, fold):
     a.counters = counters.data_ptr() if fold else None
     a.eps_f, a.n_layers, a.batch = float(eps_f), nl, b
     a.d_model, a.d_inner, a.d_state, a.dt_rank, a.d_conv = M, D, cfg.d_state, cfg.dt_rank, cfg.d_conv
-    a.fold = int(bool(fold))
+    a.fold, a.dtype = int(bool(fold)), _ACT_DTYPES[dtype]
     with _dev_guard(h):
         _lib.check(_lib.load().mtl_decode_step_batched(ctypes.byref(a), layers, _stream(h)), "decode_step_batched")
-    return ws[:b * M].view(b, M)
+    return ws.view(dtype)[:b * M].view(b, M)     # normed_out: the workspace's first slice
 
 
 def decode_persist_workspace(cfg, device) -> torch.Tensor:

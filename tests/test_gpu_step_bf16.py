@@ -1,0 +1,69 @@
+"""mtl_decode_step_batched on a bfloat16 model (weights, activations and conv
+history in bf16; fp32 residual, SSM state and partial sums): MambaLM.step
+(model.py:343-353) at 1-32 rows against the float64 oracle and the per-op
+step, and captured."""
+import numpy as np
+import pytest
+import torch
+
+import _golden as G
+from _util import assert_rel
+from mamba_lite import ops
+from mamba_lite.cuda_graph import GraphedStepper
+from mamba_lite.model import MambaCache, MambaConfig, MambaLM
+from oracle import mixer as om
+
+pytestmark = pytest.mark.gpu
+
+
+# d_model, d_inner / d_model, batch, d_conv, bias: fp32-ineligible widths too (d_inner 1280 and 1792, not a multiple
+# of 512; wavefronts with unequal stage counts), one row, fold edge (16 / 17 rows), 32 rows on 32-row tiles (d 2048)
+BF16_SHAPES = [(512, 2, 1, 4, False), (640, 2, 3, 4, True), (896, 2, 16, 3, False), (512, 3, 17, 2, True),
+               (768, 2, 32, 4, False), (2048, 2, 5, 4, False), (2048, 2, 32, 4, False)]
+
+
+@pytest.mark.parametrize("dm,expand,b,d_conv,bias", BF16_SHAPES)
+def test_bf16_one_call_step_matches_oracle_and_per_op(dm, expand, b, d_conv, bias, monkeypatch):
+    """A bfloat16 model's one-call step against the float64 oracle on the same
+    bf16-rounded weights and caches (1e-2, the bf16 gate), and no further
+    from it than twice the per-op step; graph replays equal eager."""
+    import mamba_lite.model as mm
+    torch.manual_seed(dm + b)
+    cfg = MambaConfig(d_model=dm, n_layer=2, vocab_size=200, d_state=16, d_conv=d_conv, expand=expand, bias=bias)
+    with torch.device("cuda"):
+        m = MambaLM(cfg).eval()
+    with torch.no_grad():
+        for blk in m.layers:
+            blk.mixer.dt_proj.bias.uniform_(-6.0, -2.0)
+    m = m.to(torch.bfloat16)
+    cache = MambaCache.allocate(cfg, b, "cuda", torch.bfloat16)
+    for lc in cache.layers:
+        lc.conv_state.normal_(0, 0.6)
+        lc.ssm_state.normal_(0, 0.1)
+    clone = lambda: MambaCache([type(lc)(lc.conv_state.clone(), lc.ssm_state.clone()) for lc in cache.layers])
+    ids = torch.randint(0, cfg.vocab_size, (b, 1), device="cuda")
+    calls = []
+    real = ops.decode_step_batched
+    monkeypatch.setattr(ops, "decode_step_batched", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    with torch.no_grad():
+        one, per_op = clone(), clone()
+        got = [m.step(ids, one) for _ in range(2)]
+        assert len(calls) == 2 and got[0].dtype == torch.bfloat16
+        monkeypatch.setattr(mm, "BATCHED_STEP_NATIVE", False)
+        old = [m.step(ids, per_op) for _ in range(2)]
+        monkeypatch.setattr(mm, "BATCHED_STEP_NATIVE", True)
+        W = G.oracle_lm_dict({k: v.double().cpu().numpy() for k, v in m.state_dict().items()}, cfg.n_layer)
+        f64 = lambda t: t.double().cpu().numpy()
+        oc = [(f64(lc.conv_state), f64(lc.ssm_state)) for lc in cache.layers]
+        for g, o in zip(got, old):
+            ref = om.lm_step(W, ids.cpu().numpy(), oc, dtype=np.float64)
+            assert_rel(f64(g), ref, 1e-2, "one call vs oracle")
+            e_g, e_o = np.linalg.norm(f64(g) - ref), np.linalg.norm(f64(o) - ref)
+            assert e_g <= 2 * e_o, (e_g, e_o)
+        for a_, b_ in zip(one.layers, per_op.layers):
+            assert_rel(f64(a_.ssm_state), f64(b_.ssm_state), 1e-2, "ssm_state")
+            assert_rel(f64(a_.conv_state), f64(b_.conv_state), 2e-2, "conv_state")
+        st = GraphedStepper(m, clone(), b, "cuda")
+        st.capture()
+        for g in got:
+            assert torch.equal(st.replay(ids), g)
