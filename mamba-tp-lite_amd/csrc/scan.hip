@@ -19,8 +19,15 @@
 //   * Each wavefront writes its partial y_t (sum over its states) to LDS;
 //     the loader threads add the 4 partials in a fixed order (deterministic),
 //     apply (y + D*u) * silu(z) and store y coalesced.
-// Per (channel, t, state) the inner loop costs one v_exp_f32 and four VALU
-// ops (mul, mul, fma, fma).  dt is staged in log2 units (dt * log2 e, which
+// Per (channel, t, state) the inner loop costs one v_exp_f32, three VALU ops
+// (dt * A, the decay of h, the C fma) and a quarter of a matrix instruction:
+// the injection of dt u B is, for 64 channels and a wavefront's 4 states, 16
+// rank-1 products of 4 channels by 4 states, which v_mfma_f32_4x4x1 adds to
+// the decayed states in place of 4 multiplies and 4 fused adds.  It issues
+// alone on the SIMD for its 8 cycles, so the gain is that of 4 VALU
+// instructions for 2: [32, 2048, 2048] bf16 with its conv 544 -> 534 us, fp32
+// [32, 1536, 1024] 208.2 -> 206.2 us, the error against float64 unchanged
+// (2.0e-7 / 2.1e-7).  dt is staged in log2 units (dt * log2 e, which
 // softplus_l2_f returns directly), so exp(dt * A) is exp2(dt_l2 * A); the
 // injection dt * u * B then takes its ln 2 from B, scaled where B is staged.
 
@@ -263,7 +270,10 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
 
     // scan registers: states [wave*SPW, wave*SPW + SPW) of channel c0 + lane
     const bool lane_ok = c0 + lane < D;
-    float h[SPW], a2[SPW];
+    // (state k in h[k / 4][k % 4])
+    constexpr bool MF = SPW % 4 == 0;
+    F4v h[(SPW + 3) / 4];
+    float a2[SPW];
 #pragma unroll
     for (int k = 0; k < SPW; ++k) {
         const int n = wave * SPW + k;
@@ -271,7 +281,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
         float av = ok ? a.A[(int64_t)(c0 + lane) * N + n] : 0.f;
         if (ok && a.a_is_log) av = -expf(av);
         a2[k] = av;
-        h[k] = (ok && a.h0) ? a.h0[((int64_t)b * D + c0 + lane) * N + n] : 0.f;
+        h[k / 4][k % 4] = (ok && a.h0) ? a.h0[((int64_t)b * D + c0 + lane) * N + n] : 0.f;
     }
 
     // The lambdas below are forced inline: an outlined one takes the state
@@ -424,13 +434,16 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
         // the B / C broadcasts of step st are read two steps before their use
         // (at 8 states per wavefront the registers for that would spill)
         constexpr int PRE = SPW <= 4 ? 2 : 0;
-        float bq[TT][SPW], cq[TT][SPW];
+        constexpr int NB = MF ? SPW / 4 : SPW;         // B registers of a step
+        float bq[TT][NB], cq[TT][SPW];
+        auto read_b = [&](int st, int k) __attribute__((always_inline)) {
+            return s_B[kc * TT + st][wave * SPW + (MF ? 4 * k + (lane & 3) : k)];
+        };
         auto read_bc = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
-            for (int k = 0; k < SPW; ++k) {
-                bq[st][k] = s_B[kc * TT + st][wave * SPW + k];
-                cq[st][k] = s_C[kc * TT + st][wave * SPW + k];
-            }
+            for (int k = 0; k < NB; ++k) bq[st][k] = read_b(st, k);
+#pragma unroll
+            for (int k = 0; k < SPW; ++k) cq[st][k] = s_C[kc * TT + st][wave * SPW + k];
         };
 #pragma unroll
         for (int st = 0; st < PRE; ++st) read_bc(st);
@@ -446,12 +459,25 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
                 const int st = tt + q;
                 if (PRE > 0 && st + PRE < TT) read_bc(st + PRE);
                 float acc = 0.f;
+                auto ck = [&](int k) __attribute__((always_inline)) {
+                    return PRE > 0 ? cq[st][k] : s_C[kc * TT + st][wave * SPW + k];
+                };
+                if constexpr (MF) {
 #pragma unroll
-                for (int k = 0; k < SPW; ++k) {
-                    const float bk = PRE > 0 ? bq[st][k] : s_B[kc * TT + st][wave * SPW + k];
-                    const float ck = PRE > 0 ? cq[st][k] : s_C[kc * TT + st][wave * SPW + k];
-                    h[k] = fmaf(__builtin_amdgcn_exp2f(dts[q] * a2[k]), h[k], dxs[q] * bk);
-                    acc = fmaf(h[k], ck, acc);
+                    for (int k = 0; k < SPW; ++k) h[k / 4][k % 4] *= __builtin_amdgcn_exp2f(dts[q] * a2[k]);
+#pragma unroll
+                    for (int g = 0; g < SPW / 4; ++g)
+                        h[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(PRE > 0 ? bq[st][g] : read_b(st, g), dxs[q], h[g],
+                                                                  0, 0, 0);
+#pragma unroll
+                    for (int k = 0; k < SPW; ++k) acc = fmaf(h[k / 4][k % 4], ck(k), acc);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < SPW; ++k) {
+                        const float bk = PRE > 0 ? bq[st][k] : read_b(st, k);
+                        h[k / 4][k % 4] = fmaf(__builtin_amdgcn_exp2f(dts[q] * a2[k]), h[k / 4][k % 4], dxs[q] * bk);
+                        acc = fmaf(h[k / 4][k % 4], ck(k), acc);
+                    }
                 }
                 yq[q] = acc;
             }
@@ -590,7 +616,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
 #pragma unroll
         for (int k = 0; k < SPW; ++k) {
             const int n = wave * SPW + k;
-            if (lane_ok && n < N) a.h_out[((int64_t)b * D + c0 + lane) * N + n] = h[k];
+            if (lane_ok && n < N) a.h_out[((int64_t)b * D + c0 + lane) * N + n] = h[k / 4][k % 4];
         }
     }
 }

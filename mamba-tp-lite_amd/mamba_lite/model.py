@@ -863,7 +863,7 @@ class MambaLM(nn.Module):
             dm // rpb <= 128
         return arr, fold
 
-    def _batched_template(self, lt, dev, dm, act):
+    def _batched_template(self, lt, dev, dm, act=torch.float32):
         """The weight half of _batched_step_layers: mtl_decode_layer records
         (W_xT = x_proj transposed, conv weights as [D, K] views), or None when
         a weight is not a contiguous `act` tensor of its shape on dev or one
