@@ -96,6 +96,16 @@ typedef struct {
 } mtl_scan_params;
 
 int mtl_selective_scan_fwd(const mtl_scan_params* p, mtl_stream_t stream);
+/* The same with a workspace.  Where the grid of the step-by-step kernel would
+ * leave the GPU mostly idle, the sequence is cut into segments that run in
+ * parallel, in two launches: each segment's decay and end state from zero,
+ * then every segment from the states its predecessors' summaries give.  The
+ * summaries need mtl_selective_scan_ws_bytes(...) bytes (0: the scan does not
+ * run in segments); with less, or ws NULL, or algo != 0, the call is
+ * mtl_selective_scan_fwd. */
+int64_t mtl_selective_scan_ws_bytes(int64_t batch, int64_t dim, int64_t dstate, int64_t seqlen);
+int mtl_selective_scan_fwd_ws(const mtl_scan_params* params, void* ws, int64_t ws_bytes, mtl_stream_t stream);
+
 
 /* ------------------------------------------------------------------------
  * Causal depthwise conv1d (+ optional SiLU), prefill.

@@ -249,7 +249,8 @@ extern "C" int mtl_prefill_long(const mtl_prefill_long_args* a, const mtl_prefil
         p.A = L.A_log; p.D = L.Dv; p.delta_bias = L.dt_bias; p.h0 = L.h0; p.h_out = L.h_out;
         p.batch = b; p.seqlen = l; p.dim = D; p.dstate = N;
         p.dtype = MTL_F32; p.delta_softplus = 1; p.a_is_log = 1; p.algo = 0;
-        rc = mtl_selective_scan_fwd(&p, stream);
+        // (the GEMM workspace is free here: segments of the sequence run in parallel where the grid is small)
+        rc = mtl_selective_scan_fwd_ws(&p, a->blas_ws, a->blas_ws_bytes, stream);
         if (rc) return rc;
         const bool last = i + 1 == a->n_layers;
         const float* w_next = last ? a->norm_f : layers[i + 1].norm_w;

@@ -49,6 +49,12 @@ struct ScanArgs {
     int64_t y_sb, y_sd, y_sl;
     int L, D, N;
     int softplus, a_is_log;
+    // sequence in segments (scan_fwd_kernel's PASS 1 and 2): steps of a
+    // segment, and per (segment, batch row, channel) the sum of dt (log2
+    // units) and the states a segment reaches from zero
+    int seg_len;
+    float* seg_dt;           // [segments, batch, D]
+    float* seg_h;            // [segments, batch, D, N]
 };
 
 // E contiguous activations <-> floats (E a multiple of 4; 16-byte (fp32) or
@@ -174,8 +180,25 @@ template <> struct Buf4<uint16_t> {
 // token-major ones fit 128 VGPRs, so 4 workgroups share a CU.
 // GEN: softplus and the z gate follow the runtime flags; without it both are
 // on (the mixer's case), and the staging has no per-element selects for them.
-template <typename T, int NW, int SPW, int TT, bool CM, bool VEC, bool GEN>
-__global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const ScanArgs a) {
+// PASS 0: the whole sequence.  PASS 1, 2: blockIdx.z is a segment of it.
+// Pass 1 runs each segment from zero states and leaves the states it reaches
+// and its sum of dt (the product of its decays is exp(A sum dt)); z, C and y
+// are left out.  Pass 2 folds the earlier segments' summaries, in order, into
+// its first states and runs the segment in full.
+template <typename T, int NW, int SPW, int TT, bool CM, bool VEC, bool GEN, int PASS>
+__global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const ScanArgs args) {
+    ScanArgs a = args;
+    if constexpr (PASS != 0) {
+        const int64_t t0 = (int64_t)blockIdx.z * a.seg_len;
+        auto at = [&](const void* p, int64_t sl) { return static_cast<const T*>(p) + t0 * sl; };
+        a.u = at(a.u, a.u_sl);
+        a.delta = at(a.delta, a.d_sl);
+        if (a.z) a.z = at(a.z, a.z_sl);
+        a.B = at(a.B, a.B_sl);
+        a.C = at(a.C, a.C_sl);
+        a.y = static_cast<T*>(a.y) + t0 * a.y_sl;
+        a.L = min(a.seg_len, a.L - (int)t0);
+    }
     constexpr int NT = NW * 64;
     constexpr int E = TT * 64 / NT;            // consecutive steps one thread stages per sub-tile
     constexpr int KC = CM ? 2 : 1;             // sub-tiles per load tile
@@ -281,7 +304,22 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
         float av = ok ? a.A[(int64_t)(c0 + lane) * N + n] : 0.f;
         if (ok && a.a_is_log) av = -expf(av);
         a2[k] = av;
-        h[k / 4][k % 4] = (ok && a.h0) ? a.h0[((int64_t)b * D + c0 + lane) * N + n] : 0.f;
+        h[k / 4][k % 4] = (PASS != 1 && ok && a.h0) ? a.h0[((int64_t)b * D + c0 + lane) * N + n] : 0.f;
+    }
+    [[maybe_unused]] float dt_sum = 0.f;
+    if constexpr (PASS == 2) {
+        const int64_t nb = gridDim.y;
+#pragma unroll 4
+        for (int sg = 0; sg < (int)blockIdx.z; ++sg) {
+            const int64_t row = (sg * nb + b) * D + min(c0 + lane, D - 1);
+            const float sd = a.seg_dt[row];
+#pragma unroll
+            for (int k = 0; k < SPW; ++k) {
+                const int n = wave * SPW + k;
+                const float e = a.seg_h[row * N + min(n, N - 1)];
+                h[k / 4][k % 4] = fmaf(__builtin_amdgcn_exp2f(sd * a2[k]), h[k / 4][k % 4], n < N ? e : 0.f);
+            }
+        }
     }
 
     // The lambdas below are forced inline: an outlined one takes the state
@@ -334,19 +372,19 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
                 for (int q = 0; q < E / 4; ++q) {
                     Buf4<T>::load(ru_cm, vo_u + vs + q * 4 * sizeof(T), so, &r.u[kc][4 * q]);
                     Buf4<T>::load(rd_cm, vo_d + vs + q * 4 * sizeof(T), so, &r.d[kc][4 * q]);
-                    Buf4<T>::load(rz_cm, vo_z + vs + q * 4 * sizeof(T), so, &r.z[kc][4 * q]);
+                    if constexpr (PASS != 1) Buf4<T>::load(rz_cm, vo_z + vs + q * 4 * sizeof(T), so, &r.z[kc][4 * q]);
                 }
             } else if constexpr (CM && F) {
                 load_run<T, E, VEC>(up + t0, r.u[kc]);
                 load_run<T, E, VEC>(dp + t0, r.d[kc]);
-                load_run<T, E, VEC>(zp + t0, r.z[kc]);
+                if constexpr (PASS != 1) load_run<T, E, VEC>(zp + t0, r.z[kc]);
             } else if constexpr (CM) {
 #pragma unroll
                 for (int j = 0; j < E; ++j) {
                     const int t = F ? t0 + j : min(t0 + j, L - 1);
                     r.u[kc][j] = Act<T>::load(up + t);
                     r.d[kc][j] = Act<T>::load(dp + t);
-                    r.z[kc][j] = Act<T>::load(zp + t);
+                    if constexpr (PASS != 1) r.z[kc][j] = Act<T>::load(zp + t);
                 }
             } else {
                 // token-major: one buffer resource per tensor over the E rows of
@@ -361,7 +399,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
                     const uint32_t dj = (uint32_t)((F ? tw + j : min(tw + j, L - 1)) - t0c);
                     r.u[kc][j] = BufAct<T>::load(ru, ch_bytes, dj * sl_bytes_u);
                     r.d[kc][j] = BufAct<T>::load(rd, ch_bytes, dj * sl_bytes_d);
-                    r.z[kc][j] = BufAct<T>::load(rz, ch_bytes, dj * sl_bytes_z);
+                    if constexpr (PASS != 1) r.z[kc][j] = BufAct<T>::load(rz, ch_bytes, dj * sl_bytes_z);
                 }
             }
         }
@@ -375,14 +413,14 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
 #pragma unroll
             for (int k = 0; k < BCE; ++k) {
                 r.B[k] = Act<T>::load(at_bytes(Bt, b_bytes[k]));
-                r.C[k] = Act<T>::load(at_bytes(Ct, c_bytes[k]));
+                if constexpr (PASS != 1) r.C[k] = Act<T>::load(at_bytes(Ct, c_bytes[k]));
             }
         } else {
 #pragma unroll
             for (int k = 0; k < BCE; ++k) {
                 const int t = min(tb + bc_t[k], L - 1);
                 r.B[k] = Act<T>::load(Bp + bc_off[k] * a.B_sn + (int64_t)t * a.B_sl);
-                r.C[k] = Act<T>::load(Cp + bc_off[k] * a.C_sn + (int64_t)t * a.C_sl);
+                if constexpr (PASS != 1) r.C[k] = Act<T>::load(Cp + bc_off[k] * a.C_sn + (int64_t)t * a.C_sl);
             }
         }
     };
@@ -407,7 +445,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
             vdt[j] = dt;
             vdx[j] = dt * uv;
             du[j] = uv;                         // D * u is folded into the output fma
-            gz[j] = has_z ? silu_f(r.z[kc][j]) : 1.f;
+            if constexpr (PASS != 1) gz[j] = has_z ? silu_f(r.z[kc][j]) : 1.f;
         }
 #pragma unroll
         for (int q = 0; q < E / 4; ++q) {
@@ -422,7 +460,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
                 if (bc_slot[k] >= 0) {
                     const bool ok = bc_ok[k] && (F || tb + bc_t[k] < L);
                     (&s_B[0][0])[bc_slot[k]] = ok ? r.B[k] * kLn2 : 0.f;
-                    (&s_C[0][0])[bc_slot[k]] = ok ? r.C[k] : 0.f;
+                    if constexpr (PASS != 1) (&s_C[0][0])[bc_slot[k]] = ok ? r.C[k] : 0.f;
                 }
             }
         }
@@ -443,7 +481,8 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
 #pragma unroll
             for (int k = 0; k < NB; ++k) bq[st][k] = read_b(st, k);
 #pragma unroll
-            for (int k = 0; k < SPW; ++k) cq[st][k] = s_C[kc * TT + st][wave * SPW + k];
+            for (int k = 0; k < SPW; ++k)
+                if constexpr (PASS != 1) cq[st][k] = s_C[kc * TT + st][wave * SPW + k];
         };
 #pragma unroll
         for (int st = 0; st < PRE; ++st) read_bc(st);
@@ -458,6 +497,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
             for (int q = 0; q < 4; ++q) {
                 const int st = tt + q;
                 if (PRE > 0 && st + PRE < TT) read_bc(st + PRE);
+                if constexpr (PASS == 1) dt_sum += dts[q];
                 float acc = 0.f;
                 auto ck = [&](int k) __attribute__((always_inline)) {
                     return PRE > 0 ? cq[st][k] : s_C[kc * TT + st][wave * SPW + k];
@@ -470,18 +510,20 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
                         h[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(PRE > 0 ? bq[st][g] : read_b(st, g), dxs[q], h[g],
                                                                   0, 0, 0);
 #pragma unroll
-                    for (int k = 0; k < SPW; ++k) acc = fmaf(h[k / 4][k % 4], ck(k), acc);
+                    for (int k = 0; k < SPW; ++k)
+                        if constexpr (PASS != 1) acc = fmaf(h[k / 4][k % 4], ck(k), acc);
                 } else {
 #pragma unroll
                     for (int k = 0; k < SPW; ++k) {
                         const float bk = PRE > 0 ? bq[st][k] : read_b(st, k);
                         h[k / 4][k % 4] = fmaf(__builtin_amdgcn_exp2f(dts[q] * a2[k]), h[k / 4][k % 4], dxs[q] * bk);
-                        acc = fmaf(h[k / 4][k % 4], ck(k), acc);
+                        if constexpr (PASS != 1) acc = fmaf(h[k / 4][k % 4], ck(k), acc);
                     }
                 }
                 yq[q] = acc;
             }
-            *reinterpret_cast<float4*>(&s_y[wave][lane][tt]) = make_float4(yq[0], yq[1], yq[2], yq[3]);
+            if constexpr (PASS != 1)
+                *reinterpret_cast<float4*>(&s_y[wave][lane][tt]) = make_float4(yq[0], yq[1], yq[2], yq[3]);
         }
     };
 
@@ -543,7 +585,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
             refill(kc);
             scan_tile(kc);
             __syncthreads();
-            finish_tile(tb, kc, full);
+            if constexpr (PASS != 1) finish_tile(tb, kc, full);
         }
     };
 
@@ -612,11 +654,18 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
         run_subtiles(r0, tb, Full<false>{}, [](int) {});
     }
 
-    if (a.h_out) {
+    float* ho = a.h_out;
+    if constexpr (PASS == 1) {
+        ho = a.seg_h + (int64_t)blockIdx.z * gridDim.y * D * N;
+        if (wave == 0 && lane_ok) a.seg_dt[((int64_t)blockIdx.z * gridDim.y + b) * D + c0 + lane] = dt_sum;
+    } else if constexpr (PASS == 2) {
+        if (blockIdx.z + 1 < gridDim.z) ho = nullptr;
+    }
+    if (ho) {
 #pragma unroll
         for (int k = 0; k < SPW; ++k) {
             const int n = wave * SPW + k;
-            if (lane_ok && n < N) a.h_out[((int64_t)b * D + c0 + lane) * N + n] = h[k / 4][k % 4];
+            if (lane_ok && n < N) ho[((int64_t)b * D + c0 + lane) * N + n] = h[k / 4][k % 4];
         }
     }
 }
@@ -624,10 +673,20 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
 template <typename T, int NW, int SPW, int TT, bool CM, bool VEC>
 void launch_scan(const ScanArgs& a, int64_t batch, hipStream_t st) {
     dim3 grid((unsigned)((a.D + 63) / 64), (unsigned)batch);
-    if (a.softplus && a.z != nullptr)
-        hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, false>), grid, dim3(NW * 64), 0, st, a);
-    else
-        hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, true>), grid, dim3(NW * 64), 0, st, a);
+    const bool plain = a.softplus && a.z != nullptr;
+    if (a.seg_len > 0) {
+        // (the last segment's summary is not used: pass 1 leaves it out)
+        const int nseg = (a.L + a.seg_len - 1) / a.seg_len;
+        dim3 g1(grid.x, grid.y, (unsigned)(nseg - 1)), g2(grid.x, grid.y, (unsigned)nseg);
+        if (a.softplus) hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, false, 1>), g1, dim3(NW * 64), 0, st, a);
+        else hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, true, 1>), g1, dim3(NW * 64), 0, st, a);
+        if (plain) hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, false, 2>), g2, dim3(NW * 64), 0, st, a);
+        else hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, true, 2>), g2, dim3(NW * 64), 0, st, a);
+    } else if (plain) {
+        hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, false, 0>), grid, dim3(NW * 64), 0, st, a);
+    } else {
+        hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, true, 0>), grid, dim3(NW * 64), 0, st, a);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1087,7 +1146,33 @@ bool rows_aligned(const ScanArgs& a, int64_t batch) {
 }  // namespace
 }  // namespace mtl
 
+// Segment length of a scan that has room for the summaries, 0 for none.  The
+// tiled kernel runs w = batch ceil(D / 64) workgroups, and its time is the
+// sequence times a step's latency until about 3 of them share a CU; segments
+// cost a second pass (0.7 of the first) and two launches' lead-in.  Measured,
+// us, mixer layout, fp32, this rule against the chunked or tiled kernel:
+// 72 workgroups 333 steps 26.1 / 33.7, 64 x 1024 45.4 / 58.7, 128 x 512 41.7 /
+// 57.8, 192 x 512 49.7 / 58.0; level or behind at 24 x 1024 33.6 / 29.1, 64 x
+// 256 20.8 / 19.3 and 256 x 500 59.4 / 59.4 (bf16 alike).
+static int scan_segment_len(int64_t batch, int64_t dim, int64_t seqlen) {
+    const int64_t w = batch * ((dim + 63) / 64);
+    if (w < 48 || w >= 256 || seqlen < 320) return 0;
+    const int64_t segs = ((w <= 128 ? 512 : 768) + w - 1) / w;
+    const int64_t len = ((seqlen + segs - 1) / segs + 31) / 32 * 32;    // whole load tiles
+    return len < seqlen ? (int)len : 0;
+}
+
+extern "C" int64_t mtl_selective_scan_ws_bytes(int64_t batch, int64_t dim, int64_t dstate, int64_t seqlen) {
+    if (batch < 1 || dim < 1 || dstate < 1 || seqlen < 1) return 0;
+    const int64_t len = scan_segment_len(batch, dim, seqlen);
+    return len ? (seqlen + len - 1) / len * batch * dim * (dstate + 1) * (int64_t)sizeof(float) : 0;
+}
+
 extern "C" int mtl_selective_scan_fwd(const mtl_scan_params* p, mtl_stream_t stream) {
+    return mtl_selective_scan_fwd_ws(p, nullptr, 0, stream);
+}
+
+extern "C" int mtl_selective_scan_fwd_ws(const mtl_scan_params* p, void* ws, int64_t ws_bytes, mtl_stream_t stream) {
     using namespace mtl;
     clear_error();
     MTL_REQUIRE(p != nullptr, "null params");
@@ -1109,7 +1194,7 @@ extern "C" int mtl_selective_scan_fwd(const mtl_scan_params* p, mtl_stream_t str
     MTL_REQUIRE(cm || tm || p->seqlen <= 1,
                 "u/delta/z/y must all be channel-major (stride_l == 1) or all token-major (stride_d == 1)");
 
-    ScanArgs a;
+    ScanArgs a{};
     a.u = p->u; a.delta = p->delta; a.z = p->z; a.B = p->B; a.C = p->C; a.y = p->y;
     a.A = p->A; a.Dv = p->D; a.dbias = p->delta_bias; a.h0 = p->h0; a.h_out = p->h_out;
     a.u_sb = p->u_sb; a.u_sd = p->u_sd; a.u_sl = p->u_sl;
@@ -1141,8 +1226,15 @@ extern "C" int mtl_selective_scan_fwd(const mtl_scan_params* p, mtl_stream_t str
 
     MTL_REQUIRE(p->algo >= 0 && p->algo <= 2, "algo must be 0 (auto), 1 (tiled) or 2 (chunked)");
     hipStream_t st = as_stream(stream);
+    const int seg_len = p->seqlen && p->algo == 0 ? scan_segment_len(p->batch, p->dim, p->seqlen) : 0;
     if (p->seqlen == 0) {
         // no steps: h_out = h0 (or zeros); the tiled kernel's path carries it
+    } else if (seg_len && ws && ws_bytes >= mtl_selective_scan_ws_bytes(p->batch, p->dim, p->dstate, p->seqlen)) {
+        MTL_REQUIRE(reinterpret_cast<uintptr_t>(ws) % 4 == 0, "ws must be 4-byte aligned");
+        const int64_t rows = (p->seqlen + seg_len - 1) / seg_len * p->batch * p->dim;
+        a.seg_len = seg_len;
+        a.seg_dt = static_cast<float*>(ws);
+        a.seg_h = a.seg_dt + rows;
     } else if (p->algo == 2 || (p->algo == 0 && p->batch * ((p->dim + 63) / 64) < kChunkedBelowWorkgroups &&
                                 p->seqlen > kChunkedMinSteps)) {
         MTL_REQUIRE(p->batch * ((p->dim + kLaneChannels - 1) / kLaneChannels) < (int64_t(1) << 31), "grid too large");

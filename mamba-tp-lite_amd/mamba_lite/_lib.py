@@ -129,6 +129,8 @@ SIGNATURES = {
     "mtl_last_error": (ctypes.c_char_p, []),
     "mtl_abi_version": (ctypes.c_int, []),
     "mtl_selective_scan_fwd": (ctypes.c_int, [ctypes.POINTER(ScanParams), _vp]),
+    "mtl_selective_scan_ws_bytes": (_i64, [_i64, _i64, _i64, _i64]),
+    "mtl_selective_scan_fwd_ws": (ctypes.c_int, [ctypes.POINTER(ScanParams), _vp, _i64, _vp]),
     "mtl_causal_conv1d_fwd": (ctypes.c_int, [ctypes.POINTER(ConvParams), _vp]),
     "mtl_conv_step": (ctypes.c_int, [_vp, _vp, _i64, _fp, _fp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _vp]),
     "mtl_selective_state_update": (ctypes.c_int, [_fp, _vp, _i64, _vp, _i64, _vp, _i64, _fp, _fp, _fp, _fp,

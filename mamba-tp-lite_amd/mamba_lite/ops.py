@@ -173,8 +173,11 @@ def selective_scan(u, delta, A, B, C, D=None, z=None, delta_bias=None, h0=None, 
     p.batch, p.seqlen, p.dim, p.dstate = b, L, Dm, N
     p.dtype, p.delta_softplus, p.a_is_log = code, int(bool(delta_softplus)), int(bool(a_is_log))
     p.algo = SCAN_ALGOS[algo]
+    lib = _lib.load()
+    nb = lib.mtl_selective_scan_ws_bytes(b, Dm, N, L) if p.algo == 0 else 0
+    ws = torch.empty(nb // 4, device=u.device, dtype=torch.float32) if nb else None
     with _dev_guard(u):
-        _lib.check(_lib.load().mtl_selective_scan_fwd(ctypes.byref(p), _stream(u)), "selective_scan_fwd")
+        _lib.check(lib.mtl_selective_scan_fwd_ws(ctypes.byref(p), _ptr(ws), nb, _stream(u)), "selective_scan_fwd")
     return y, h_out
 
 

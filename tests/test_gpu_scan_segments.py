@@ -1,0 +1,47 @@
+"""Scans that run in parallel segments (mtl_selective_scan_fwd_ws) against the
+step-by-step kernel on the same inputs: segment boundaries, remainders,
+layouts, state counts, h0, types and the optional operands."""
+import pytest
+import torch
+
+from mamba_lite import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(b, D, L, N, dtype, cm, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    r = lambda *s, k=1.0: (k * torch.randn(*s, device="cuda", generator=g)).to(dtype)
+    lay = (lambda t: t) if cm else (lambda t: t.transpose(1, 2).contiguous().transpose(1, 2))
+    return dict(u=lay(r(b, D, L)), delta=lay(r(b, D, L, k=0.5)), z=lay(r(b, D, L)), B=r(b, N, L), C=r(b, N, L),
+                A=-torch.arange(1, N + 1, device="cuda", dtype=torch.float32).repeat(D, 1).contiguous(),
+                D=torch.ones(D, device="cuda"), bias=-2 - 3 * torch.rand(D, device="cuda", generator=g),
+                h0=torch.randn(b, D, N, device="cuda", generator=g))
+
+
+# b, D, L, N: the smallest segmented length, one step past whole segments, a last segment of 1 step, tail channels,
+# the fewest and most workgroups of the range, 1-32 states
+SHAPES = [(1, 3072, 320, 16), (3, 1536, 333, 16), (1, 4096, 1025, 16), (2, 4090, 385, 5), (3, 5000, 500, 1),
+          (2, 2048, 640, 32), (1, 3080, 2000, 8)]
+
+
+@pytest.mark.parametrize("b,D,L,N", SHAPES)
+@pytest.mark.parametrize("dtype,cm", [(torch.float32, True), (torch.float32, False), (torch.bfloat16, False)])
+def test_segments_match_the_sequential_scan(b, D, L, N, dtype, cm):
+    assert _lib.load().mtl_selective_scan_ws_bytes(b, D, N, L) > 0
+    c = _case(b, D, L, N, dtype, cm)
+    # fp32: the decay over a segment is exp(A sum dt) for a product of exps, and the carried state is rounded once more
+    # per segment: some 2^-23; bf16 y: one rounding of the output, 2^-9
+    tol = 1e-6 if dtype == torch.float32 else 2.0 ** -8
+    rel = lambda a, r: float((a.double() - r.double()).norm() / r.double().norm())
+    for kw in (dict(z=c["z"], h0=c["h0"], delta_bias=c["bias"], D=c["D"]), dict(delta_bias=c["bias"]),
+               dict(z=c["z"], delta_softplus=False, delta_bias=None)):
+        d = c["delta"] if kw.get("delta_softplus", True) else 0.01 * c["delta"].abs()
+        y, h = ops.selective_scan(c["u"], d, c["A"], c["B"], c["C"], **kw)
+        yr, hr = ops.selective_scan(c["u"], d, c["A"], c["B"], c["C"], algo="tiled", **kw)
+        assert rel(y, yr) < tol and rel(h, hr) < 1e-6
+
+
+def test_outside_the_rule_nothing_changes():
+    ws = _lib.load().mtl_selective_scan_ws_bytes
+    assert ws(1, 1536, 16, 1024) == 0 and ws(32, 1536, 16, 1024) == 0 and ws(1, 4096, 16, 300) == 0
