@@ -311,6 +311,8 @@ typedef struct {
     int64_t M, N, K;
 } mtl_linear_f32_args;
 int64_t mtl_linear_f32_ws_bytes(int64_t M, int64_t N, int64_t K);
+/* 1 where it is faster than the library's fp32 GEMM (by measurement), else 0 */
+int mtl_linear_f32_pays(int64_t M, int64_t N, int64_t K);
 int mtl_linear_f32(const mtl_linear_f32_args* args, mtl_stream_t stream);
 
 /* ------------------------------------------------------------------------

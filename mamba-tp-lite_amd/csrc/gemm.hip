@@ -105,17 +105,14 @@ struct SplitJob {
     int* exps;                             // [rows rounded up to 64]
 };
 
-// workgroups [0, nb0) take the first matrix, the others the second
 template <int NT>
-__global__ void __launch_bounds__(NT) split_rows_kernel(const SplitJob j0, const SplitJob j1, int nb0) {
-    const bool second = (int)blockIdx.x >= nb0;
-    const float* const x = second ? j1.x : j0.x;
-    const int64_t ld = second ? j1.ld : j0.ld, rows = second ? j1.rows : j0.rows;
-    const int K = second ? j1.K : j0.K;
-    const bool vec = second ? j1.vec : j0.vec;
-    uint8_t* const out = second ? j1.out : j0.out;
-    int* const exps = second ? j1.exps : j0.exps;
-    const int64_t block = (int)blockIdx.x - (second ? nb0 : 0);
+__device__ __forceinline__ void split_block(const SplitJob& j, int64_t block) {
+    const float* const x = j.x;
+    const int64_t ld = j.ld, rows = j.rows;
+    const int K = j.K;
+    const bool vec = j.vec;
+    uint8_t* const out = j.out;
+    int* const exps = j.exps;
     constexpr int NW = NT / 64;
     __shared__ uint32_t s_max[NW][kSplitRows];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -158,6 +155,103 @@ __global__ void __launch_bounds__(NT) split_rows_kernel(const SplitJob j0, const
             *reinterpret_cast<H8*>(q) = hi;
             *reinterpret_cast<H8*>(q + 16) = lo;
         }
+    }
+}
+
+// workgroups [0, nb0) take the first matrix, the others the second
+template <int NT>
+__global__ void __launch_bounds__(NT) split_rows_kernel(const SplitJob j0, const SplitJob j1, int nb0) {
+    const bool second = (int)blockIdx.x >= nb0;
+    split_block<NT>(second ? j1 : j0, (int)blockIdx.x - (second ? nb0 : 0));
+}
+
+// The residual add and RMSNorm in front of an in_proj (model.py:306, 130-135)
+// with the split of its output, and the split of the in_proj's weight, in one
+// launch: the first nbn workgroups take 8 rows each (a wavefront a row, 8
+// columns per lane and run, all loaded up front), the others 16 weight rows.
+// Separate launches of the norm and the two splits took 5.5 + 6.8 + 7 us at
+// 999 x 768, each of them mostly its launch and first round trip.
+struct NormArgs {
+    const float* x; const float* y;        // h, and the mixer output to add (null: none)
+    float* x_out;                          // x + y (null: not stored)
+    const float* w;
+    float* normed;                         // the norm's output in fp32
+    float eps;
+};
+constexpr int kNsThreads = 512, kNsRows = kNsThreads / 64;
+
+template <int RU>                          // 512-column runs of a row
+__global__ void __launch_bounds__(kNsThreads) norm_split_kernel(const NormArgs n, const SplitJob jx, const SplitJob jw,
+                                                                int nbn) {
+    if ((int)blockIdx.x >= nbn) {
+        split_block<kNsThreads>(jw, (int)blockIdx.x - nbn);
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * kNsRows + (threadIdx.x >> 6);
+    const int cols = jx.K;                 // a multiple of 32
+    if (row >= jx.rows) {                  // whole wavefronts: the row block's padding
+        if (lane == 0) jx.exps[row] = 0;
+        return;
+    }
+    float v[RU][8], wv[RU][8];
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+        const int c = min(u * 512 + lane * 8, cols - 8);
+        load8(n.x + row * cols + c, 8, true, v[u]);
+        load8(n.w + c, 8, true, wv[u]);
+    }
+    if (n.y) {
+        float yv[RU][8];
+#pragma unroll
+        for (int u = 0; u < RU; ++u) load8(n.y + row * cols + min(u * 512 + lane * 8, cols - 8), 8, true, yv[u]);
+#pragma unroll
+        for (int u = 0; u < RU; ++u)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[u][j] += yv[u][j];
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < RU; ++u)
+        if (u * 512 + lane * 8 < cols) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) ss = fmaf(v[u][j], v[u][j], ss);
+        }
+    const float r = rsqrtf(group_sum<64>(ss) / (float)cols + n.eps);
+    uint32_t mx = 0;
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+        const int c = u * 512 + lane * 8;
+        if (c >= cols) continue;
+        if (n.x_out) {
+            float4* p = reinterpret_cast<float4*>(n.x_out + row * cols + c);
+            p[0] = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
+            p[1] = make_float4(v[u][4], v[u][5], v[u][6], v[u][7]);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            v[u][j] = wv[u][j] * (v[u][j] * r);
+            mx = max(mx, abs_bits(v[u][j]));
+        }
+        float4* p = reinterpret_cast<float4*>(n.normed + row * cols + c);
+        p[0] = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
+        p[1] = make_float4(v[u][4], v[u][5], v[u][6], v[u][7]);
+    }
+    const int e = split_exp(group_umax<64>(mx));
+    if (lane == 0) jx.exps[row] = e;
+    if (e >= kExpSpecial) return;          // a marked row's parts are never used
+    const float scale = __uint_as_float((uint32_t)(e + 127) << 23);
+    const int np = cols / kPanel;
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+        const int c = u * 512 + lane * 8;
+        if (c >= cols) continue;
+        H8 hi, lo;
+        split8(v[u], scale, hi, lo);
+        uint8_t* q = jx.out + (row / kRowBlock * np + c / kPanel) * (kRowBlock * kPanelBytes) +
+                     (row % kRowBlock) * kPanelBytes + (c / 8 % 2) * 32;
+        *reinterpret_cast<H8*>(q) = hi;
+        *reinterpret_cast<H8*>(q + 16) = lo;
     }
 }
 
@@ -439,6 +533,35 @@ int split_rows(const float* x, int64_t ldx, int64_t M, const float* w, int64_t l
     return check_launch("split_rows");
 }
 
+int norm_split(const float* x, const float* y, float* x_out, const float* w, float eps, float* normed, int64_t M,
+               int64_t K, const float* wmat, int64_t ldw, int64_t N, void* xbuf, void* wbuf, hipStream_t st) {
+    const NormArgs n{x, y, x_out, w, normed, eps};
+    const SplitJob jx = split_job(normed, K, M, K, xbuf), jw = split_job(wmat, ldw, N, K, wbuf);
+    const int64_t bn = pad_to(M, kRowBlock) / kNsRows, bw = pad_to(N, kRowBlock) / kSplitRows;
+    const dim3 grid((unsigned)(bn + bw)), nt(kNsThreads);
+    if (K <= 512) hipLaunchKernelGGL((norm_split_kernel<1>), grid, nt, 0, st, n, jx, jw, (int)bn);
+    else if (K <= 1024) hipLaunchKernelGGL((norm_split_kernel<2>), grid, nt, 0, st, n, jx, jw, (int)bn);
+    else hipLaunchKernelGGL((norm_split_kernel<4>), grid, nt, 0, st, n, jx, jw, (int)bn);
+    return check_launch("norm_split");
+}
+
+bool norm_split_ok(const float* x, const float* y, const float* w, const float* normed, int64_t K) {
+    return K % 32 == 0 && K <= 2048 &&
+           (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(w) |
+            reinterpret_cast<uintptr_t>(normed)) % 16 == 0;
+}
+
+// Where the product with the splits of x and W beats the library's fp32 GEMM:
+// the split of W is paid once per call, so the gain needs rows, and few tiles
+// leave CUs idle.  Measured, us, library / split + product: 999 x 3072 x 768
+// 45 / 40, 768 x 3072 x 768 36 / 39; 768 x 2048 x 4096 107 / 96, 512 x 2048 x
+// 4096 69 / 86; 384 x 8192 x 2048 112 / 96, 256 x 8192 x 2048 74 / 81; 256 x
+// 50280 x 768 171 / 156, 192 x 50280 x 768 146 / 150; 999 x 768 x 1536 24 / 38.
+bool split_pays(int64_t M, int64_t N, int64_t K) {
+    const double flops = 2.0 * (double)M * (double)N * (double)K;
+    return N >= 256 && K >= 128 && ((M >= 256 && flops >= 1.2e10) || (M >= 896 && flops >= 4.5e9));
+}
+
 int gemm_split(const SplitGemm& g, hipStream_t st) {
     const SplitJob x = split_job(g.x, g.ldx, g.M, g.K, g.xbuf), w = split_job(g.w, g.ldw, g.N, g.K, g.wbuf);
     GemmArgs a{};
@@ -462,6 +585,8 @@ int gemm_split(const SplitGemm& g, hipStream_t st) {
 }
 
 }  // namespace mtl
+
+extern "C" int mtl_linear_f32_pays(int64_t M, int64_t N, int64_t K) { return mtl::split_pays(M, N, K) ? 1 : 0; }
 
 extern "C" int64_t mtl_linear_f32_ws_bytes(int64_t M, int64_t N, int64_t K) {
     if (M < 1 || N < 1 || K < 1) return 0;

@@ -26,7 +26,11 @@
 // conv over more than 64 rows crosses the in_proj tiles.  The parts live in
 // blas_ws, which the skinny form does not otherwise use.
 //
-// The GEMMs are hipBLASLt matmuls, fp32 in and out, fp32 compute.  For each
+// An in_proj or out_proj with enough rows runs as the split-f16 product of
+// gemm.hip (split_pays), its operands split in blas_ws; the norm before such
+// an in_proj writes the split too (norm_split).
+//
+// The other GEMMs are hipBLASLt matmuls, fp32 in and out, fp32 compute.  For each
 // shape the heuristic's first algorithm is looked up once per device and
 // kept (descriptors and algorithm), so a call costs the launches only; the
 // workspace is the caller's, so the call allocates no device memory and can
@@ -44,6 +48,7 @@
 #include <tuple>
 
 #include "common.h"
+#include "gemm.h"
 
 namespace {
 
@@ -55,6 +60,8 @@ struct GemmPlan {
 
 // (device, n, rows, k, ldw, ldx, ldy, bias, workspace bytes)
 using GemmKey = std::tuple<int, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, bool, size_t>;
+
+constexpr int64_t kBlasWs = 32 << 20;             // a larger workspace serves the split products, not hipBLASLt
 
 std::mutex g_mu;                                  // guards the handles, the plans and every call's launches
 std::map<int, hipblasLtHandle_t> g_handles;
@@ -193,6 +200,18 @@ extern "C" int mtl_prefill_long(const mtl_prefill_long_args* a, const mtl_prefil
         const mtl_prefill_layer& L = layers[i];
         skinny = al16(L.W_in) && al16(L.b_in) && al16(L.W_x) && al16(L.W_out) && al16(L.b_out);
     }
+    // The products that the split-f16 GEMM takes, where it is the faster one
+    // and the workspace holds the split operands.  The in_proj's x is then
+    // split where the norm before it writes it, together with the split of
+    // that layer's weight: the region is taken first and nothing else of the
+    // call may use it between that norm and the in_proj.
+    const int64_t xb = (split_bytes(rows, M) + 1023) / 1024 * 1024, in_bytes = xb + split_bytes(2 * D, M);
+    const int64_t yb = (split_bytes(rows, D) + 1023) / 1024 * 1024, out_bytes = yb + split_bytes(M, D);
+    bool split_in = !skinny && split_pays(rows, 2 * D, M) && in_bytes <= a->blas_ws_bytes && al16(a->blas_ws) &&
+                    norm_split_ok(a->h, a->out, nullptr, a->xn, M);
+    for (int32_t i = 0; split_in && i < a->n_layers; ++i) split_in = al16(layers[i].norm_w);
+    const bool split_out = !skinny && split_pays(rows, M, D) && out_bytes <= a->blas_ws_bytes && al16(a->blas_ws);
+    uint8_t* sws = static_cast<uint8_t*>(a->blas_ws);
     float* x_parts = static_cast<float*>(a->blas_ws);                 // [xs, rows, J]
     float* y_parts = x_parts + (int64_t)xs * rows * J;                 // [4, rows, M]
     hipStream_t st = as_stream(stream);
@@ -203,15 +222,28 @@ extern "C" int mtl_prefill_long(const mtl_prefill_long_args* a, const mtl_prefil
     }
     std::lock_guard<std::mutex> lock(g_mu);
     void* ws = a->blas_ws;
-    const size_t wsb = (size_t)a->blas_ws_bytes;
-    int rc = mtl_add_rmsnorm(a->h, nullptr, nullptr, layers[0].norm_w, a->xn, rows, M, layers[0].eps, stream);
+    const size_t wsb = (size_t)std::min<int64_t>(a->blas_ws_bytes, kBlasWs);
+    // norm i's output feeds layer i's in_proj
+    auto norm = [&](int32_t i, const float* y) {
+        const mtl_prefill_layer& L = layers[i];
+        if (split_in)
+            return norm_split(a->h, y, y ? a->h : nullptr, L.norm_w, L.eps, a->xn, rows, M, L.W_in, M, 2 * D, sws,
+                              sws + xb, st);
+        return mtl_add_rmsnorm(a->h, y, y ? a->h : nullptr, L.norm_w, a->xn, rows, M, L.eps, stream);
+    };
+    int rc = norm(0, nullptr);
     if (rc) return rc;
     for (int32_t i = 0; i < a->n_layers; ++i) {
         const mtl_prefill_layer& L = layers[i];
         if (skinny)
             rc = mtl_linear_skinny(a->xn, M, L.W_in, L.b_in, a->xz, 2 * D, 0, rows, 2 * D, M, 1,
                                    rows_per_block_of(rows, 2 * D, 1), stream);
-        else
+        else if (split_in) {
+            SplitGemm g{};
+            g.x = a->xn; g.ldx = M; g.w = L.W_in; g.ldw = M; g.bias = L.b_in; g.y0 = a->xz; g.ldy0 = 2 * D;
+            g.M = rows; g.N = 2 * D; g.K = M; g.xbuf = sws; g.wbuf = sws + xb;
+            rc = gemm_split(g, st);
+        } else
             rc = gemm(dev, L.W_in, M, a->xn, M, a->xz, 2 * D, L.b_in, 2 * D, rows, M, ws, wsb, st);
         if (rc) return rc;
         // [b, D, l] views of the [b l, 2D] and [b l, D] buffers
@@ -262,9 +294,18 @@ extern "C" int mtl_prefill_long(const mtl_prefill_long_args* a, const mtl_prefil
             if (rc) return rc;
             rc = mtl_add_rmsnorm_parts(a->h, y_parts, kOutSplit, a->h, w_next, normed, rows, M, eps, stream);
         } else {
-            rc = gemm(dev, L.W_out, D, a->y, D, a->out, M, L.b_out, M, rows, D, ws, wsb, st);
+            if (split_out) {
+                SplitGemm g{};
+                g.x = a->y; g.ldx = D; g.w = L.W_out; g.ldw = D; g.bias = L.b_out; g.y0 = a->out; g.ldy0 = M;
+                g.M = rows; g.N = M; g.K = D; g.xbuf = sws; g.wbuf = sws + yb;
+                rc = split_rows(g.x, D, rows, g.w, D, M, D, g.xbuf, g.wbuf, st);
+                if (rc) return rc;
+                rc = gemm_split(g, st);
+            } else {
+                rc = gemm(dev, L.W_out, D, a->y, D, a->out, M, L.b_out, M, rows, D, ws, wsb, st);
+            }
             if (rc) return rc;
-            rc = mtl_add_rmsnorm(a->h, a->out, a->h, w_next, normed, rows, M, eps, stream);
+            rc = last ? mtl_add_rmsnorm(a->h, a->out, a->h, w_next, normed, rows, M, eps, stream) : norm(i + 1, a->out);
         }
         if (rc) return rc;
     }

@@ -150,18 +150,17 @@ _SKINNY_PREFILL = True
 SHORT_PREFILL_NATIVE = True
 
 # Longer prompts on an fp32 model run as one C call too (mtl_prefill_long),
-# with the projections as hipBLASLt GEMMs launched from C++, up to
-# LONG_PREFILL_MAX_ELEMS token-channels (b l d_inner): below it an eager
-# per-op prefill is bound by its ~160 us of Python per layer.  Measured per
-# prompt, one call against the per-op path: mamba-130m width 65 tokens 1.62
-# against 3.94 ms, 256 tokens 1.70 against 3.91 ms, 1024 tokens 3.55 against
-# 3.92 ms; mamba-1.4b width 128 tokens 4.82 against 8.10 ms, 512 tokens 12.87
-# against 12.85 ms.  Past it the GPU time dominates and the per-op path keeps
-# torch's GEMMs (and any tuned GEMM table: 1.4b 1024 tokens 23.4 against 23.9
-# ms with it).  The C call's GEMM picks differ from torch's, so its logits
-# differ from the per-op path's by float rounding.
+# up to LONG_PREFILL_MAX_ELEMS token-channels (b l d_inner): an eager per-op
+# prefill costs ~160 us of Python per layer, and the one call writes the split
+# operands of a large in_proj from the norm before it.  Measured per layer,
+# per-op path against the one call: mamba-130m width 1024 tokens 165 / 109 us,
+# 4096 tokens 238 / 235; mamba-1.4b width 1024 tokens 338 / 330, 2048 tokens 545
+# / 523.  Far past that the two are level, and from SPLIT_PROJ_MIN_TOKENS the
+# per-op path lays the in_proj's halves out apart for the scan.  The C call's
+# library GEMM picks differ from torch's, so its logits differ from the per-op
+# path's by float rounding.
 LONG_PREFILL_NATIVE = True
-LONG_PREFILL_MAX_ELEMS = 1 << 21
+LONG_PREFILL_MAX_ELEMS = 1 << 23
 # Up to LONG_PREFILL_SKINNY_ROWS token rows, at widths up to
 # LONG_PREFILL_SKINNY_MAX_D_MODEL, the one-call long prefill runs its
 # projections on the library's skinny GEMM (64-row chunks) instead of

@@ -581,7 +581,7 @@ def check_step_shape(d_state, dt_rank) -> None:
                          f"{STEP_MAX_D_STATE} and dt_rank <= {STEP_MAX_DT_RANK}")
 
 
-PREFILL_LONG_BLAS_WS = 32 << 20     # bytes of hipBLASLt workspace per mtl_prefill_long call
+PREFILL_LONG_BLAS_WS = 32 << 20     # bytes of hipBLASLt workspace per mtl_prefill_long call (it takes no more)
 
 
 def prefill_long_ok(b, l, d_model, d_inner, d_state, dt_rank, d_conv) -> bool:
@@ -596,8 +596,9 @@ def prefill_long_ok(b, l, d_model, d_inner, d_state, dt_rank, d_conv) -> bool:
 
 def prefill_long(h, layers, norm_f, eps_f, d_inner, d_state, dt_rank, d_conv, skinny_rows=0):
     """mtl_prefill_long: a prompt's whole layer stack in one call (any
-    length, the projections on hipBLASLt; up to skinny_rows token rows on
-    the library's skinny GEMM where the shapes fit it).  h [b, l, d_model]
+    length; the projections on hipBLASLt, up to skinny_rows token rows on
+    the library's skinny GEMM where the shapes fit it, and from enough rows
+    on the in_proj and out_proj on the split-f16 product).  h [b, l, d_model]
     float32 holds the embedded tokens and is overwritten with the final
     residual stream; `layers` is a ctypes array of _lib.PrefillLayer
     (weights plus this call's cache pointers).  Returns norm_f(h)
@@ -608,9 +609,13 @@ def prefill_long(h, layers, norm_f, eps_f, d_inner, d_state, dt_rank, d_conv, sk
     rows, J = b * l, dt_rank + 2 * d_state
     if norm_f.numel() != M or norm_f.device != h.device:
         raise ValueError(f"prefill_long: norm_f must hold {M} floats on {h.device}")
-    # one workspace, every buffer on a 256-byte boundary
+    # one workspace, every buffer on a 256-byte boundary; the last serves the
+    # GEMM library or, where those products are split, their operands
+    lib = _lib.load()
+    blas_ws = max([PREFILL_LONG_BLAS_WS] + [lib.mtl_linear_f32_ws_bytes(rows, n, k)
+                                            for n, k in ((2 * d_inner, M), (M, d_inner)) if linear_f32_pays(rows, n, k)])
     sizes = [rows * M, rows * 2 * d_inner, rows * d_inner, rows * J, rows * d_inner, rows * d_inner, rows * M,
-             PREFILL_LONG_BLAS_WS // 4]
+             -(-blas_ws // 4)]
     offs, n = [], 0
     for sz in sizes:
         offs.append(n)
@@ -621,12 +626,12 @@ def prefill_long(h, layers, norm_f, eps_f, d_inner, d_state, dt_rank, d_conv, sk
     a = _lib.PrefillLongArgs()
     a.h = h.data_ptr()
     a.xn, a.xz, a.u, a.x_dbl, a.dt, a.y, a.out, a.blas_ws = [base + 4 * o for o in offs]
-    a.blas_ws_bytes = PREFILL_LONG_BLAS_WS
+    a.blas_ws_bytes = blas_ws
     a.norm_f, a.normed_out, a.eps_f = norm_f.data_ptr(), normed.data_ptr(), float(eps_f)
     a.d_conv, a.n_layers, a.skinny_rows = d_conv, len(layers), int(skinny_rows)
     a.batch, a.seqlen, a.d_model, a.d_inner, a.d_state, a.dt_rank = b, l, M, d_inner, d_state, dt_rank
     with _dev_guard(h):
-        _lib.check(_lib.load().mtl_prefill_long(ctypes.byref(a), layers, _stream(h)), "prefill_long")
+        _lib.check(lib.mtl_prefill_long(ctypes.byref(a), layers, _stream(h)), "prefill_long")
     return normed
 
 
@@ -872,15 +877,8 @@ def decode_gemv(v, W, out, bias=None, x_in=None):
 
 
 def linear_f32_pays(M: int, N: int, K: int) -> bool:
-    """Where mtl_linear_f32 (the splits of x and W included) beats the library's
-    fp32 GEMM: the split of W is paid once per call, so the gain needs rows,
-    and few tiles leave CUs idle.  Measured, us, library / split + product:
-    999 x 3072 x 768 45 / 40, 768 x 3072 x 768 36 / 39; 768 x 2048 x 4096 107 /
-    96, 512 x 2048 x 4096 69 / 86; 384 x 8192 x 2048 112 / 96, 256 x 8192 x 2048
-    74 / 81; 256 x 50280 x 768 171 / 156, 192 x 50280 x 768 146 / 150; 999 x 768 x
-    1536 24 / 38."""
-    flops = 2.0 * M * N * K
-    return N >= 256 and K >= 128 and ((M >= 256 and flops >= 1.2e10) or (M >= 896 and flops >= 4.5e9))
+    """Where mtl_linear_f32 (the splits of x and W included) beats the library's fp32 GEMM."""
+    return bool(_lib.load().mtl_linear_f32_pays(M, N, K))
 
 
 def linear_f32_ok(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:

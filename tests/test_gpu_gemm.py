@@ -97,3 +97,29 @@ def test_route_keeps_autograd_and_autocast():
             assert not ops.linear_f32_ok(x, wp)
     assert not ops.linear_f32_ok(x.bfloat16(), w.bfloat16())
     assert not ops.linear_f32_ok(x[:128], w)
+
+
+@pytest.mark.parametrize("d_model,b,l,kw", [(768, 3, 333, dict(bias=True)), (768, 1, 2000, {}), (2048, 1, 420, {}),
+                                            (1000, 1, 1100, {})])
+def test_one_call_prefill_with_split_projections(d_model, b, l, kw, monkeypatch):
+    """A one-call prefill whose in_proj (and, from 1909 rows at d_model 768,
+    out_proj) run split, the in_proj's operand written by the norm before it
+    (d_model 1000 is no multiple of 32: library GEMM there), against the
+    per-op path: the two differ by fp32 rounding only (1e-5, the bound the
+    long prefill's other forms are held to)."""
+    import mamba_lite.model as mm
+    from mamba_lite.model import MambaConfig, MambaLM
+    torch.manual_seed(l)
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=d_model, n_layer=2, vocab_size=300, **kw)).eval()
+    ids = torch.randint(0, 300, (b, l), device="cuda")
+    assert lm._native_prefill_kind(b, l) == "long"
+    with torch.no_grad():
+        got, cache = lm.prefill(ids)
+        monkeypatch.setattr(mm, "LONG_PREFILL_NATIVE", False)
+        monkeypatch.setattr(ops, "linear_f32_ok", lambda *a, **k: False)
+        ref, rcache = lm.prefill(ids)
+    rel = lambda a, r: float((a.double() - r.double()).norm() / r.double().norm())
+    assert rel(got, ref) < 1e-5
+    for a, r in zip(cache.layers, rcache.layers):
+        assert rel(a.ssm_state, r.ssm_state) < 1e-5 and rel(a.conv_state, r.conv_state) < 1e-5
