@@ -316,6 +316,18 @@ int mtl_linear_f32_pays(int64_t M, int64_t N, int64_t K);
 int mtl_linear_f32(const mtl_linear_f32_args* args, mtl_stream_t stream);
 
 /* ------------------------------------------------------------------------
+ * The tied lm_head of few rows (model.py:326, 353): y [M, N] = x [M, K] W
+ * [N, K]^T, all contiguous, 16-byte aligned and of `dtype` (fp32 sums), W
+ * streamed once with x held in registers.  M <= 16; N a multiple of 4 below
+ * 2^27; K a multiple of 128 from 1024 to 2048 (bf16: of 256 from 2048 to
+ * 4096).  mtl_lm_head_ok: 1 where these sizes hold and N is large enough
+ * (32768) for it to be the faster one.
+ * ---------------------------------------------------------------------- */
+int mtl_lm_head_ok(int64_t M, int64_t N, int64_t K, int32_t dtype);
+int mtl_lm_head(const void* x, const void* W, void* y, int64_t M, int64_t N, int64_t K, int32_t dtype,
+                mtl_stream_t stream);
+
+/* ------------------------------------------------------------------------
  * Skinny fp32 GEMM on the matrix cores for the projections of a batched
  * decode step: y = x W^T (+ bias), nn.Linear on [b, K] with b <= 32 tokens --
  * in_proj (model.py:261), out_proj (model.py:293) and the tied lm_head

@@ -159,6 +159,8 @@ SIGNATURES = {
                                      _fp, _i32, _i32, _i32, _i32, _i32, _i32, _vp]),
     "mtl_decode_gemv": (ctypes.c_int, [_fp, _fp, _fp, _fp, _fp, _i32, _i32, _i32, _vp]),
     "mtl_decode_gemv_parts": (ctypes.c_int, [_fp, _fp, _fp, _i32, _i32, _i32, _i32, _vp]),
+    "mtl_lm_head_ok": (ctypes.c_int, [_i64, _i64, _i64, _i32]),
+    "mtl_lm_head": (ctypes.c_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp]),
     "mtl_linear_f32_pays": (ctypes.c_int, [_i64, _i64, _i64]),
     "mtl_linear_f32_ws_bytes": (_i64, [_i64, _i64, _i64]),
     "mtl_linear_f32": (ctypes.c_int, [ctypes.POINTER(LinearF32Args), _vp]),

@@ -585,7 +585,8 @@ class MambaLM(nn.Module):
         self.norm_f = RMSNorm(cfg.d_model, eps=cfg.layer_norm_epsilon)
 
     def lm_head(self, x: torch.Tensor) -> torch.Tensor:
-        return _linear(x, self.embedding.weight)
+        w = self.embedding.weight
+        return ops.lm_head(x, w) if ops.lm_head_ok(x, w) else _linear(x, w)
 
     def _norm_weight(self, i: int) -> torch.Tensor:
         mod = self.layers[i].norm if i < len(self.layers) else self.norm_f

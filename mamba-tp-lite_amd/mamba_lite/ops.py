@@ -888,18 +888,46 @@ def linear_f32_ok(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
     if x.dtype != torch.float32 or W.dtype != torch.float32 or not x.is_cuda or W.device != x.device or \
             x.dim() < 2 or W.dim() != 2 or not x.is_contiguous() or W.stride(1) != 1 or x.shape[-1] != W.shape[1]:
         return False
-    if type(x) is not torch.Tensor or type(W) not in (torch.Tensor, torch.nn.Parameter):
-        return False
     N, K = W.shape
     if x.numel() == 0 or not linear_f32_pays(x.numel() // K, N, K) or N >= 1 << 21 or W.stride(0) < K:
         return False
-    if bias is not None and (type(bias) not in (torch.Tensor, torch.nn.Parameter) or bias.dtype != torch.float32 or
-                             bias.device != x.device or not bias.is_contiguous() or tuple(bias.shape) != (N,)):
+    if bias is not None and (bias.dtype != torch.float32 or bias.device != x.device or not bias.is_contiguous() or
+                             tuple(bias.shape) != (N,)):
         return False
-    if torch.is_autocast_enabled("cuda"):
+    return _plain_forward(x, W) if bias is None else _plain_forward(x, W, bias)
+
+
+def _plain_forward(*ts) -> bool:
+    """Nothing of torch's between these tensors and a raw launch: no autograd, autocast or tensor subclass."""
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts) and \
+        not torch.is_autocast_enabled("cuda") and \
+        not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+
+
+def lm_head_ok(x: torch.Tensor, W: torch.Tensor) -> bool:
+    """Whether lm_head takes F.linear(x, W) in its place: a decode step's rows
+    against a wide, contiguous vocabulary matrix of x's type."""
+    if x.dtype not in _ACT_DTYPES or W.dtype != x.dtype or not x.is_cuda or W.device != x.device or x.dim() < 2 or \
+            W.dim() != 2 or x.shape[-1] != W.shape[1] or not x.is_contiguous() or not W.is_contiguous():
         return False
-    return not (torch.is_grad_enabled() and (x.requires_grad or W.requires_grad or
-                                             (bias is not None and bias.requires_grad)))
+    N, K = W.shape
+    M = x.numel() // K if K else 0
+    return M <= 16 and _plain_forward(x, W) and aligned16(x, W) and \
+        bool(_lib.load().mtl_lm_head_ok(M, N, K, _ACT_DTYPES[x.dtype]))
+
+
+def lm_head(x, W):
+    """F.linear(x, W) for at most 16 rows of x against a wide W (mtl_lm_head)."""
+    N, K = W.shape
+    if W.dtype != x.dtype or not x.is_contiguous() or not W.is_contiguous() or x.shape[-1] != K:
+        raise ValueError("lm_head: x [..., K] and W [N, K] must be contiguous and of one type")
+    code = _act_code(x, W)
+    _same_device(x, W)
+    y = torch.empty(*x.shape[:-1], N, device=x.device, dtype=x.dtype)
+    with _dev_guard(x):
+        _lib.check(_lib.load().mtl_lm_head(_ptr(x), _ptr(W), _ptr(y), x.numel() // K, N, K, code, _stream(x)),
+                   "lm_head")
+    return y
 
 
 def linear_f32(x, W, bias=None, n_split=None):
