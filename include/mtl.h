@@ -32,7 +32,12 @@ extern "C" {
 #endif
 
 enum mtl_status { MTL_OK = 0, MTL_EINVAL = 1, MTL_EHIP = 2, MTL_EUNSUPPORTED = 3 };
-enum mtl_dtype { MTL_F32 = 0, MTL_BF16 = 1 };
+enum mtl_dtype {
+    MTL_F32 = 0,
+    MTL_BF16 = 1,
+    MTL_BF16_PARAMS = 2   /* scan and causal conv only: bf16 activations and bf16 parameters
+                             (A, D, delta_bias; w 8-byte aligned, bias) in place of float ones */
+};
 
 typedef void* mtl_stream_t; /* hipStream_t */
 

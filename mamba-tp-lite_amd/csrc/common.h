@@ -54,6 +54,11 @@ template <> struct Act<uint16_t> {  // bf16 storage
     __device__ __forceinline__ static void store(uint16_t* p, float v) { *p = f32_to_bf16(v); }
 };
 
+// Parameter i of a float array, or of a bf16 one (bf uniform).
+__device__ __forceinline__ float load_param(const void* p, int64_t i, bool bf) {
+    return bf ? bf16_to_f32(static_cast<const uint16_t*>(p)[i]) : static_cast<const float*>(p)[i];
+}
+
 // 4 consecutive values as floats, one 16-byte (fp32) or 8-byte (bf16) access;
 // and a value rounded to the storage type.
 typedef float F4v __attribute__((ext_vector_type(4)));

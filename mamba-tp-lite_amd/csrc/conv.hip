@@ -27,10 +27,11 @@ constexpr int kTC = 16;      // timesteps per thread
 constexpr int kMaxK = 8;
 
 struct ConvArgs {
-    const void* x; void* out; const float* w; const float* bias;
+    const void* x; void* out;
+    const void* w; const void* bias;     // float, or bf16 with par_bf (bf16 activations only)
     const void* st_in; void* st_out;
     int64_t x_sb, x_sd, x_sl, o_sb, o_sd, o_sl;
-    int L, D, K, silu;
+    int L, D, K, silu, par_bf;
 };
 
 // VC adjacent channels as one vector (VC > 1 needs unit channel stride and
@@ -112,12 +113,25 @@ __global__ void __launch_bounds__(kConvThreads) conv_fwd_kernel(const ConvArgs a
         Vec<T, VC>::load(xp + (int64_t)t * a.x_sl, v[j]);
     }
     float w[K][VC], bias[VC];
+    if (sizeof(T) == 2 && VC == 4 && a.par_bf) {
+        // the four channels' K weights are K runs of 4 values
+        const uint16_t* wp = static_cast<const uint16_t*>(a.w) + (int64_t)c0 * K;
 #pragma unroll
-    for (int ci = 0; ci < VC; ++ci) {
+        for (int q = 0; q < K; ++q) {
+            const F4v f = ld4(wp + 4 * q);
 #pragma unroll
-        for (int k = 0; k < K; ++k) w[k][ci] = a.w[(int64_t)(c0 + ci) * K + k];
-        bias[ci] = a.bias ? a.bias[c0 + ci] : 0.f;
+            for (int e = 0; e < 4; ++e) w[(4 * q + e) % K][(4 * q + e) / K % VC] = f[e];
+        }
+    } else {
+#pragma unroll
+        for (int ci = 0; ci < VC; ++ci)
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                w[k][ci] = load_param(a.w, (int64_t)(c0 + ci) * K + k, sizeof(T) == 2 && a.par_bf);
     }
+#pragma unroll
+    for (int ci = 0; ci < VC; ++ci)
+        bias[ci] = a.bias ? load_param(a.bias, c0 + ci, sizeof(T) == 2 && a.par_bf) : 0.f;
     // padded positions below K-1 are the carried history or zeros; with runs
     // shorter than K-1 they reach past the first run (uniform per wavefront)
     if (t0 < K - 1) {
@@ -373,7 +387,8 @@ extern "C" int mtl_causal_conv1d_fwd(const mtl_conv_params* p, mtl_stream_t stre
     MTL_REQUIRE(p->batch <= 65535, "batch must be <= 65535");
     MTL_REQUIRE(p->seqlen < (int64_t(1) << 31) && p->dim < (int64_t(1) << 31), "size overflows int32");
     MTL_REQUIRE((p->seqlen + kTC - 1) / kTC <= 65535, "seqlen too long for one launch");
-    MTL_REQUIRE(p->dtype == MTL_F32 || p->dtype == MTL_BF16, "dtype must be MTL_F32 or MTL_BF16");
+    MTL_REQUIRE(p->dtype == MTL_F32 || p->dtype == MTL_BF16 || p->dtype == MTL_BF16_PARAMS,
+                "dtype must be MTL_F32, MTL_BF16 or MTL_BF16_PARAMS");
     MTL_REQUIRE(p->conv_state_in == nullptr || p->conv_state_in != p->conv_state_out,
                 "conv_state_out must not alias conv_state_in");
     if (p->batch == 0 || p->dim == 0) return MTL_OK;
@@ -398,6 +413,8 @@ extern "C" int mtl_causal_conv1d_fwd(const mtl_conv_params* p, mtl_stream_t stre
     a.x_sb = p->x_sb; a.x_sd = p->x_sd; a.x_sl = p->x_sl;
     a.o_sb = p->out_sb; a.o_sd = p->out_sd; a.o_sl = p->out_sl;
     a.L = (int)p->seqlen; a.D = (int)p->dim; a.K = p->width; a.silu = p->silu;
+    a.par_bf = p->dtype == MTL_BF16_PARAMS;
+    MTL_REQUIRE(!a.par_bf || reinterpret_cast<uintptr_t>(p->w) % 8 == 0, "bf16 weights must be 8-byte aligned");
     return p->dtype == MTL_F32 ? launch_conv<float>(a, p->batch, st) : launch_conv<uint16_t>(a, p->batch, st);
 }
 

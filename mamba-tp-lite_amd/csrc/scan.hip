@@ -40,7 +40,8 @@ namespace {
 
 struct ScanArgs {
     const void* u; const void* delta; const void* z; const void* B; const void* C; void* y;
-    const float* A; const float* Dv; const float* dbias; const float* h0; float* h_out;
+    const void* A; const void* Dv; const void* dbias;    // float, or bf16 with par_bf (bf16 activations only)
+    const float* h0; float* h_out;
     int64_t u_sb, u_sd, u_sl;
     int64_t d_sb, d_sd, d_sl;
     int64_t z_sb, z_sd, z_sl;
@@ -48,7 +49,7 @@ struct ScanArgs {
     int64_t C_sb, C_sn, C_sl;
     int64_t y_sb, y_sd, y_sl;
     int L, D, N;
-    int softplus, a_is_log;
+    int softplus, a_is_log, par_bf;
     // sequence in segments (scan_fwd_kernel's PASS 1 and 2): steps of a
     // segment, and per (segment, batch row, channel) the sum of dt (log2
     // units) and the states a segment reaches from zero
@@ -288,8 +289,9 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
     const uint32_t vo_z = has_z ? (uint32_t)(((int64_t)cl * a.z_sd + ot) * (int64_t)sizeof(T)) : vo_u;
     const uint32_t vo_y = (uint32_t)(((int64_t)cl * a.y_sd + ot) * (int64_t)sizeof(T));
 
-    const float bias_c = (a.dbias ? a.dbias[cl] : 0.f) * kLog2e;   // log2 units, as dt
-    const float D_c = a.Dv ? a.Dv[cl] : 0.f;
+    const bool pbf = sizeof(T) == 2 && a.par_bf;
+    const float bias_c = (a.dbias ? load_param(a.dbias, cl, pbf) : 0.f) * kLog2e;   // log2 units, as dt
+    const float D_c = a.Dv ? load_param(a.Dv, cl, pbf) : 0.f;
 
     // scan registers: states [wave*SPW, wave*SPW + SPW) of channel c0 + lane
     const bool lane_ok = c0 + lane < D;
@@ -301,7 +303,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
     for (int k = 0; k < SPW; ++k) {
         const int n = wave * SPW + k;
         const bool ok = lane_ok && n < N;
-        float av = ok ? a.A[(int64_t)(c0 + lane) * N + n] : 0.f;
+        float av = ok ? load_param(a.A, (int64_t)(c0 + lane) * N + n, pbf) : 0.f;
         if (ok && a.a_is_log) av = -expf(av);
         a2[k] = av;
         h[k / 4][k % 4] = (PASS != 1 && ok && a.h0) ? a.h0[((int64_t)b * D + c0 + lane) * N + n] : 0.f;
@@ -799,10 +801,11 @@ __global__ void __launch_bounds__(kLaneChannels * 64) scan_lanes_kernel(const Sc
     // them out uniformly.  States n >= N have A = 0 and B = C = 0: identity
     // maps that add nothing, so the state loop needs no branch and its
     // chains interleave.
-    const float bias_l2 = (a.dbias ? a.dbias[c] : 0.f) * kLog2e;
-    const float D_c = a.Dv ? a.Dv[c] : 0.f;
+    const bool pbf = sizeof(T) == 2 && a.par_bf;
+    const float bias_l2 = (a.dbias ? load_param(a.dbias, c, pbf) : 0.f) * kLog2e;
+    const float D_c = a.Dv ? load_param(a.Dv, c, pbf) : 0.f;
     const int nl = min(lane, N - 1);
-    float a_lane = a.A[(int64_t)c * N + nl];
+    float a_lane = load_param(a.A, (int64_t)c * N + nl, pbf);
     if (a.a_is_log) a_lane = -expf(a_lane);
     a_lane = lane < N ? a_lane : 0.f;
     float h_lane = a.h0 ? a.h0[((int64_t)b * D + c) * N + nl] : 0.f;
@@ -970,10 +973,11 @@ __global__ void __launch_bounds__(kLaneChannels * 64) scan_lanes_long_kernel(con
     Chunk cur, nxt;
     load_chunk(cur, 0);
 
-    const float bias_l2 = (a.dbias ? a.dbias[c] : 0.f) * kLog2e;
-    const float D_c = a.Dv ? a.Dv[c] : 0.f;
+    const bool pbf = sizeof(T) == 2 && a.par_bf;
+    const float bias_l2 = (a.dbias ? load_param(a.dbias, c, pbf) : 0.f) * kLog2e;
+    const float D_c = a.Dv ? load_param(a.Dv, c, pbf) : 0.f;
     const int nl = min(lane, N - 1);
-    float a_lane = a.A[(int64_t)c * N + nl];
+    float a_lane = load_param(a.A, (int64_t)c * N + nl, pbf);
     if (a.a_is_log) a_lane = -expf(a_lane);
     a_lane = lane < N ? a_lane : 0.f;
     float h_lane = a.h0 ? a.h0[((int64_t)b * D + c) * N + nl] : 0.f;
@@ -1181,7 +1185,8 @@ extern "C" int mtl_selective_scan_fwd_ws(const mtl_scan_params* p, void* ws, int
     MTL_REQUIRE(p->batch <= 65535, "batch must be <= 65535");
     MTL_REQUIRE(p->batch * ((p->dim + 63) / 64) < (int64_t(1) << 31), "batch * ceil(dim / 64) overflows int32");
     MTL_REQUIRE(p->seqlen < (int64_t(1) << 31) && p->dim < (int64_t(1) << 31), "size overflows int32");
-    MTL_REQUIRE(p->dtype == MTL_F32 || p->dtype == MTL_BF16, "dtype must be MTL_F32 or MTL_BF16");
+    MTL_REQUIRE(p->dtype == MTL_F32 || p->dtype == MTL_BF16 || p->dtype == MTL_BF16_PARAMS,
+                "dtype must be MTL_F32, MTL_BF16 or MTL_BF16_PARAMS");
     if (p->batch == 0 || p->dim == 0) return MTL_OK;
     MTL_REQUIRE(p->A != nullptr, "null A");
     // an empty sequence only carries h0 (or zeros) through to h_out; torch
@@ -1204,7 +1209,7 @@ extern "C" int mtl_selective_scan_fwd_ws(const mtl_scan_params* p, void* ws, int
     a.C_sb = p->C_sb; a.C_sn = p->C_sn; a.C_sl = p->C_sl;
     a.y_sb = p->y_sb; a.y_sd = p->y_sd; a.y_sl = p->y_sl;
     a.L = (int)p->seqlen; a.D = (int)p->dim; a.N = (int)p->dstate;
-    a.softplus = p->delta_softplus; a.a_is_log = p->a_is_log;
+    a.softplus = p->delta_softplus; a.a_is_log = p->a_is_log; a.par_bf = p->dtype == MTL_BF16_PARAMS;
     // B/C element offsets within a load tile and token-major channel offsets
     // are 32-bit byte offsets (non-negative strides, spans under 4 GiB)
     MTL_REQUIRE(p->B_sn >= 0 && p->B_sl >= 0 && p->C_sn >= 0 && p->C_sl >= 0, "negative B/C stride");

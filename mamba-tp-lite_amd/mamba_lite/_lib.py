@@ -19,6 +19,7 @@ ABI_VERSION = 3
 
 MTL_F32 = 0
 MTL_BF16 = 1
+MTL_BF16_PARAMS = 2     # bf16 activations and parameters (scan, causal conv)
 
 _i64 = ctypes.c_int64
 _i32 = ctypes.c_int32

@@ -399,9 +399,12 @@ class MambaMixer(nn.Module):
             z = z_flat.view(b, l, Dm).transpose(1, 2)
         else:
             u_store = torch.empty(b, l, Dm, device=x.device, dtype=x.dtype)
-            u, conv_state = ops.causal_conv1d(xs, self._conv_w(), _f32(self.conv1d.bias), conv_state=conv_in_state,
-                                              silu=True, out=u_store.transpose(1, 2),
-                                              final_state=out.conv_state if out is not None else None)
+            cw, cb = self.conv1d.weight, self.conv1d.bias
+            pbf = x.dtype == torch.bfloat16 and ops.bf16_params_ok(cw, cb)     # read as they are, no float copies
+            u, conv_state = ops.causal_conv1d(xs, cw if pbf else self._conv_w(), cb if pbf else _f32(cb),
+                                              conv_state=conv_in_state, silu=True, out=u_store.transpose(1, 2),
+                                              final_state=out.conv_state if out is not None else None,
+                                              bf16_params=pbf)
         w_x = self.x_proj.weight
         u2 = _skinny_rows(u_store, w_x, skinny)
         dt = None
@@ -435,9 +438,12 @@ class MambaMixer(nn.Module):
             h0 = cache.ssm_state.float().contiguous()
         y_store = torch.empty(b, l, Dm, device=x.device, dtype=x.dtype)
         # h_out may be h0: each state is read and written by the same thread
-        _, h = ops.selective_scan(u, dt.transpose(1, 2), _f32(self.A_log), B, C, D=_f32(self.D), z=z,
-                                  delta_bias=_f32(self.dt_proj.bias), h0=h0, delta_softplus=True, a_is_log=True,
-                                  y=y_store.transpose(1, 2), h_out=out.ssm_state if out is not None else None)
+        par = (self.A_log, self.D, self.dt_proj.bias)
+        pbf = x.dtype == torch.bfloat16 and ops.bf16_params_ok(*par)
+        A_log, Dv, dt_bias = par if pbf else map(_f32, par)
+        _, h = ops.selective_scan(u, dt.transpose(1, 2), A_log, B, C, D=Dv, z=z, delta_bias=dt_bias, h0=h0,
+                                  delta_softplus=True, a_is_log=True, y=y_store.transpose(1, 2),
+                                  h_out=out.ssm_state if out is not None else None, bf16_params=pbf)
         h = h if out is not None else h.to(_state_dtype(x.dtype))
         if parts_ok:
             w_out = self.out_proj.weight

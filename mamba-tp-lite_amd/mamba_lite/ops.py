@@ -82,20 +82,32 @@ def _same_device(ref: torch.Tensor, *ts):
             raise RuntimeError(f"all operands must be on {ref.device}, got {t.device}")
 
 
-def _f32_vec(t, n, name):
+def _f32_vec(t, n, name, dtype=torch.float32):
     if t is None:
         return None
-    if t.dtype != torch.float32 or t.dim() != 1 or t.shape[0] != n or not t.is_contiguous():
-        raise ValueError(f"{name} must be a contiguous float32 vector of length {n}, got "
+    if t.dtype != dtype or t.dim() != 1 or t.shape[0] != n or not t.is_contiguous():
+        raise ValueError(f"{name} must be a contiguous {str(dtype)[6:]} vector of length {n}, got "
                          f"{tuple(t.shape)} {t.dtype}")
     return t
 
 
-def _f32_mat(t, shape, name):
-    if t.dtype != torch.float32 or t.shape != shape or not t.is_contiguous():
-        raise ValueError(f"{name} must be contiguous float32 {tuple(shape)}, got {tuple(t.shape)} {t.dtype}"
+def _f32_mat(t, shape, name, dtype=torch.float32):
+    if t.dtype != dtype or t.shape != shape or not t.is_contiguous():
+        raise ValueError(f"{name} must be contiguous {str(dtype)[6:]} {tuple(shape)}, got {tuple(t.shape)} {t.dtype}"
                          f"{'' if t.is_contiguous() else ' (non-contiguous)'}")
     return t
+
+
+def _param_code(code: int, bf16_params: bool) -> int:
+    """The entry point's dtype when a call's parameters are bf16 like its activations."""
+    if bf16_params and code != _lib.MTL_BF16:
+        raise TypeError("bf16 parameters go with bfloat16 activations")
+    return _lib.MTL_BF16_PARAMS if bf16_params else code
+
+
+def bf16_params_ok(*ts) -> bool:
+    """Whether every (non-None) parameter can be handed over as bf16: contiguous, 16-byte aligned bfloat16."""
+    return all(t is None or (t.dtype == torch.bfloat16 and t.is_contiguous()) for t in ts) and aligned16(*ts)
 
 
 def _bdl_layout_ok(*ts):
@@ -115,30 +127,33 @@ SCAN_ALGOS = {"auto": 0, "tiled": 1, "chunked": 2}
 
 
 def selective_scan(u, delta, A, B, C, D=None, z=None, delta_bias=None, h0=None, delta_softplus=True,
-                   a_is_log=False, y=None, h_out=None, return_last_state=True, algo="auto"):
+                   a_is_log=False, y=None, h_out=None, return_last_state=True, algo="auto", bf16_params=False):
     """Fused selective scan (mtl_selective_scan_fwd); see include/mtl.h.
 
     Returns (y [b,D,l] in the activation dtype, h_last [b,D,N] fp32) -- the
     pair MambaMixer.prefill gets from its scan loop (model.py:226-241).
-    `y` / `h_out` may be preallocated (y with the same layout rules as u)."""
+    `y` / `h_out` may be preallocated (y with the same layout rules as u).
+    bf16_params: A, D and delta_bias are bfloat16 (with bfloat16 activations)
+    and read as they are; otherwise they are float32."""
+    pdt = torch.bfloat16 if bf16_params else torch.float32
     if u.dim() != 3:
         raise ValueError(f"u must be [b, D, l], got {tuple(u.shape)}")
     b, Dm, L = u.shape
     if A.dim() != 2 or A.shape[0] != Dm:
         raise ValueError(f"A must be [D={Dm}, N], got {tuple(A.shape)}")
     N = A.shape[1]
-    _f32_mat(A, (Dm, N), "A")
+    _f32_mat(A, (Dm, N), "A", pdt)
     for name, t in (("delta", delta), ("z", z)):
         if t is not None and tuple(t.shape) != (b, Dm, L):
             raise ValueError(f"{name} must be {(b, Dm, L)}, got {tuple(t.shape)}")
     for name, t in (("B", B), ("C", C)):
         if tuple(t.shape) != (b, N, L):
             raise ValueError(f"{name} must be {(b, N, L)}, got {tuple(t.shape)}")
-    _f32_vec(D, Dm, "D")
-    _f32_vec(delta_bias, Dm, "delta_bias")
+    _f32_vec(D, Dm, "D", pdt)
+    _f32_vec(delta_bias, Dm, "delta_bias", pdt)
     if h0 is not None:
         _f32_mat(h0, (b, Dm, N), "h0")
-    code = _act_code(u, delta, z, B, C)
+    code = _param_code(_act_code(u, delta, z, B, C), bf16_params)
     _same_device(u, delta, z, B, C, A, D, delta_bias, h0, y, h_out)
     if not _bdl_layout_ok(u, delta, z, y):
         u, delta = u.contiguous(), delta.contiguous()
@@ -183,10 +198,12 @@ def selective_scan(u, delta, A, B, C, D=None, z=None, delta_bias=None, h0=None, 
 
 # --------------------------------------------------------------------------- conv
 def causal_conv1d(x, weight, bias=None, conv_state=None, silu=True, out=None, final_state=None,
-                  return_final_state=True):
+                  return_final_state=True, bf16_params=False):
     """Fused causal depthwise conv (+SiLU) over x [b,D,l] (mtl_causal_conv1d_fwd).
     weight: [D,K] or [D,1,K] fp32; conv_state: [b,D,K-1] incoming history.
+    bf16_params: weight and bias are bfloat16 (with bfloat16 activations).
     Returns (out [b,D,l], final conv state [b,D,K-1]) as model.py:206-212."""
+    pdt = torch.bfloat16 if bf16_params else torch.float32
     if x.dim() != 3:
         raise ValueError(f"x must be [b, D, l], got {tuple(x.shape)}")
     b, Dm, L = x.shape
@@ -194,9 +211,9 @@ def causal_conv1d(x, weight, bias=None, conv_state=None, silu=True, out=None, fi
     if w.shape[0] != Dm:
         raise ValueError(f"weight must be [D={Dm}, K], got {tuple(weight.shape)}")
     K = w.shape[1]
-    _f32_mat(w, (Dm, K), "weight")
-    _f32_vec(bias, Dm, "bias")
-    code = _act_code(x, out, conv_state, final_state)
+    _f32_mat(w, (Dm, K), "weight", pdt)
+    _f32_vec(bias, Dm, "bias", pdt)
+    code = _param_code(_act_code(x, out, conv_state, final_state), bf16_params)
     _same_device(x, w, bias, conv_state, out, final_state)
     if conv_state is not None and (tuple(conv_state.shape) != (b, Dm, K - 1) or not conv_state.is_contiguous()):
         raise ValueError(f"conv_state must be contiguous {(b, Dm, K - 1)}, got {tuple(conv_state.shape)}")

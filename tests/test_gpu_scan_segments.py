@@ -45,3 +45,25 @@ def test_segments_match_the_sequential_scan(b, D, L, N, dtype, cm):
 def test_outside_the_rule_nothing_changes():
     ws = _lib.load().mtl_selective_scan_ws_bytes
     assert ws(1, 1536, 16, 1024) == 0 and ws(32, 1536, 16, 1024) == 0 and ws(1, 4096, 16, 300) == 0
+
+
+@pytest.mark.parametrize("b,D,L", [(1, 70, 5), (2, 256, 100), (1, 4096, 500), (8, 1536, 64)])
+def test_bf16_parameters_equal_their_float_copies(b, D, L):
+    """A bf16 model's scan and conv read its parameters as stored: the bits
+    that float copies of them give, on every scan kernel (chunked, segmented,
+    tiled) and with 4-channel and single-channel conv threads."""
+    c = _case(b, D, L, 16, torch.bfloat16, False)
+    A, Dv, bias = (-c["A"]).log().bfloat16(), c["D"].bfloat16(), c["bias"].bfloat16()
+    for algo in ("auto", "tiled", "chunked"):
+        kw = dict(z=c["z"], a_is_log=True, algo=algo)
+        got = ops.selective_scan(c["u"], c["delta"], A, c["B"], c["C"], D=Dv, delta_bias=bias, bf16_params=True, **kw)
+        ref = ops.selective_scan(c["u"], c["delta"], A.float(), c["B"], c["C"], D=Dv.float(),
+                                 delta_bias=bias.float(), **kw)
+        assert all(torch.equal(p, q) for p, q in zip(got, ref))
+    for K in (1, 3, 4):
+        w, wb = torch.randn(D, 1, K, device="cuda").bfloat16(), torch.randn(D, device="cuda").bfloat16()
+        got = ops.causal_conv1d(c["u"], w, wb, bf16_params=True)
+        ref = ops.causal_conv1d(c["u"], w.float(), wb.float())
+        assert all(torch.equal(p, q) for p, q in zip(got, ref))
+    with pytest.raises(ValueError):
+        ops.selective_scan(c["u"], c["delta"], A, c["B"], c["C"])          # bf16 parameters only on request
