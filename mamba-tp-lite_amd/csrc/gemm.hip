@@ -32,12 +32,12 @@
 // by plain fp32 sums in the epilogue, so infinities and NaN come out as an
 // fp32 product gives them.
 //
-// Measured (us; library fp32 GEMM -> this product, plus the splits of X / W):
-//   32768 x 3072 x 768 (mamba-130m in_proj, 32 x 1024 tokens)   1246 -> 449 + 44 / 7
-//   32768 x 768 x 1536 (its out_proj)                            554 -> 215 + 95 / 7
-//   1024 x 8192 x 2048 (mamba-1.4b in_proj, 1024 tokens)         240 -> 100 + 8 / 34
-//   1024 x 2048 x 4096 (its out_proj)                            119 -> 69 + 14 / 20
-//   999 x 50280 x 768 (the tied lm_head)                         700 -> 283 + 7 / 71
+// Measured (us; library fp32 GEMM -> this product, plus the splits of X and W):
+//   32768 x 3072 x 768 (mamba-130m in_proj, 32 x 1024 tokens)   1246 -> 449 + 41
+//   32768 x 768 x 1536 (its out_proj)                            554 -> 215 + 73
+//   1024 x 8192 x 2048 (mamba-1.4b in_proj, 1024 tokens)         240 -> 94 + 34
+//   1024 x 2048 x 4096 (its out_proj)                            119 -> 66 + 21
+//   999 x 50280 x 768 (the tied lm_head)                         700 -> 224 + 52
 // at 250 to 392 TFLOP/s of fp32 product, 3 MFMAs each: 0.75 to 1.18 PFLOP/s of
 // the 1.47 that the library reaches on an 8192^3 f16 product.  The relative
 // error against 64 bits (2-norm) falls from 5.0e-7 to 3.1e-7 at K = 768,
@@ -63,10 +63,10 @@ constexpr int kExpNan = 1 << 21;
 // ------------------------------------------------------------------ splitting
 // One workgroup takes 16 rows: lane = (row of 16, 8-column block of 4), so a
 // wavefront reads whole 128-byte runs of 16 rows and writes 1 KB runs of two
-// panels; the wavefronts take 32-column units in turn.  Pass 1 finds each
-// row's largest |x| (bit patterns, so a NaN is the largest), pass 2 reads the
-// rows again (from L2) and writes the parts.  The mark of a row with
-// non-finite values is its largest bit pattern: above inf's it holds a NaN.
+// panels; the wavefronts take 32-column units in turn.  Each row's largest
+// |x| is found first (bit patterns, so a NaN is the largest), then the parts
+// are written.  The mark of a row with non-finite values is its largest bit
+// pattern: above inf's it holds a NaN.
 constexpr int kSplitRows = 16;
 
 __device__ __forceinline__ void load8(const float* p, int n, bool vec, float* v) {
@@ -97,6 +97,28 @@ __device__ __forceinline__ void split8(const float* v, float scale, H8& hi, H8& 
     }
 }
 
+// The 4 lanes of a row hold two panels' 64 bytes, two lanes a panel; they swap
+// parts so that a store instruction writes one panel of 16 rows, 1 KB without
+// gaps (hi and lo stored by their own lanes left every other 16 bytes to the
+// next instruction).
+__device__ __forceinline__ void store_panels(const H8& hi, const H8& lo, uint8_t* q0, uint8_t* q1, int blk) {
+    typedef int I4 __attribute__((ext_vector_type(4)));
+    const I4 h = __builtin_bit_cast(I4, hi), l = __builtin_bit_cast(I4, lo);
+    I4 a, b;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        // quad_perm [0, 0, 1, 1] and [2, 2, 3, 3]
+        const int h0 = __builtin_amdgcn_update_dpp(0, h[i], 0x50, 0xF, 0xF, false);
+        const int l0 = __builtin_amdgcn_update_dpp(0, l[i], 0x50, 0xF, 0xF, false);
+        const int h1 = __builtin_amdgcn_update_dpp(0, h[i], 0xFA, 0xF, 0xF, false);
+        const int l1 = __builtin_amdgcn_update_dpp(0, l[i], 0xFA, 0xF, 0xF, false);
+        a[i] = blk & 1 ? l0 : h0;
+        b[i] = blk & 1 ? l1 : h1;
+    }
+    *reinterpret_cast<I4*>(q0 + blk * 16) = a;
+    *reinterpret_cast<I4*>(q1 + blk * 16) = b;
+}
+
 struct SplitJob {
     const float* x;
     int64_t ld, rows;
@@ -105,28 +127,44 @@ struct SplitJob {
     int* exps;                             // [rows rounded up to 64]
 };
 
-template <int NT>
+// U: 32-column units a wavefront holds in registers from one pass over the
+// row, all loaded up front (8 wavefronts: K <= 256 U); 0: any K, the rows read
+// a second time.  HBM is the bound.  Against two passes with one load in
+// flight at a time (both operands of a product, us): in_proj + out_proj of 32768
+// tokens at d_model 768 153 -> 114 (5.5 TB/s at K = 1536), of 1024 tokens at
+// 2048 70 -> 55, the lm_head's 999 + 50280 rows of 768 74 -> 52.  16 units take
+// 160 VGPRs (3 wavefronts a SIMD), 32 would spill.  Beside the norm (below)
+// the weight's workgroups are few and keep two passes: 10.2 us either way at
+// 999 + 3072 x 768.
+template <int NT, int U>
 __device__ __forceinline__ void split_block(const SplitJob& j, int64_t block) {
-    const float* const x = j.x;
-    const int64_t ld = j.ld, rows = j.rows;
-    const int K = j.K;
-    const bool vec = j.vec;
-    uint8_t* const out = j.out;
-    int* const exps = j.exps;
-    constexpr int NW = NT / 64;
+    constexpr int NW = NT / 64, UR = U > 0 ? U : 1;
     __shared__ uint32_t s_max[NW][kSplitRows];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = lane >> 2, blk = lane & 3;
+    const int r = lane >> 2, blk = lane & 3, K = j.K;
+    const bool vec = j.vec;
     const int64_t row = block * kSplitRows + r;
-    const float* p = x + min(row, rows - 1) * ld;
+    const float* p = j.x + min(row, j.rows - 1) * j.ld;
     const int units = (K + 31) / 32;
+    float held[UR][8];
     uint32_t mx = 0;
-    for (int u = wave; u < units; u += NW) {
-        const int c = u * 32 + blk * 8;
-        float v[8];
-        load8(p + c, K - c, vec, v);
+    if constexpr (U > 0) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) mx = max(mx, abs_bits(v[j]));
+        for (int i = 0; i < U; ++i) {
+            const int c = min(wave + i * NW, units - 1) * 32 + blk * 8;      // a unit past the end: the last again
+            load8(p + c, K - c, vec, held[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) mx = max(mx, abs_bits(held[i][q]));
+    } else {
+        for (int u = wave; u < units; u += NW) {
+            const int c = u * 32 + blk * 8;
+            load8(p + c, K - c, vec, held[0]);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) mx = max(mx, abs_bits(held[0][q]));
+        }
     }
     mx = max(mx, dpp_mov_u<kDppXor1>(mx));
     mx = max(mx, dpp_mov_u<kDppXor2>(mx));
@@ -135,34 +173,39 @@ __device__ __forceinline__ void split_block(const SplitJob& j, int64_t block) {
 #pragma unroll
     for (int w = 0; w < NW; ++w) mx = max(mx, s_max[w][r]);
     const int e = split_exp(mx);
-    if (wave == 0 && blk == 0) exps[row] = row < rows ? e : 0;     // exps is padded to whole row blocks
-    // a marked row's parts are never used: any finite values do
+    if (wave == 0 && blk == 0) j.exps[row] = row < j.rows ? e : 0;     // exps is padded to whole row blocks
+    // a marked row's parts are never used: zeros do
     const float scale = e >= kExpSpecial ? 0.f : __uint_as_float((uint32_t)(e + 127) << 23);
     const int np = 2 * units;
-    for (int u = wave; u < units; u += NW) {
-        const int c = u * 32 + blk * 8, pan = 2 * u + (blk >> 1);
-        float v[8];
-        load8(p + c, K - c, vec, v);
+    uint8_t* const q = j.out + (row / kRowBlock * np) * (kRowBlock * kPanelBytes) + (row % kRowBlock) * kPanelBytes;
+    auto put = [&](float* v, int u) __attribute__((always_inline)) {
         if (e >= kExpSpecial) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = 0.f;
+            for (int i = 0; i < 8; ++i) v[i] = 0.f;
         }
         H8 hi, lo;
         split8(v, scale, hi, lo);
-        if (row < rows) {
-            uint8_t* q = out + (row / kRowBlock * np + pan) * (kRowBlock * kPanelBytes) +
-                         (row % kRowBlock) * kPanelBytes + (blk & 1) * 32;
-            *reinterpret_cast<H8*>(q) = hi;
-            *reinterpret_cast<H8*>(q + 16) = lo;
+        uint8_t* qu = q + (int64_t)(2 * u) * (kRowBlock * kPanelBytes);
+        if (row < j.rows) store_panels(hi, lo, qu, qu + kRowBlock * kPanelBytes, blk);   // whole quads of lanes
+    };
+    if constexpr (U > 0) {
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+            if (wave + i * NW < units) put(held[i], wave + i * NW);
+    } else {
+        for (int u = wave; u < units; u += NW) {
+            const int c = u * 32 + blk * 8;
+            load8(p + c, K - c, vec, held[0]);
+            put(held[0], u);
         }
     }
 }
 
 // workgroups [0, nb0) take the first matrix, the others the second
-template <int NT>
+template <int NT, int U>
 __global__ void __launch_bounds__(NT) split_rows_kernel(const SplitJob j0, const SplitJob j1, int nb0) {
     const bool second = (int)blockIdx.x >= nb0;
-    split_block<NT>(second ? j1 : j0, (int)blockIdx.x - (second ? nb0 : 0));
+    split_block<NT, U>(second ? j1 : j0, (int)blockIdx.x - (second ? nb0 : 0));
 }
 
 // The residual add and RMSNorm in front of an in_proj (model.py:306, 130-135)
@@ -184,7 +227,7 @@ template <int RU>                          // 512-column runs of a row
 __global__ void __launch_bounds__(kNsThreads) norm_split_kernel(const NormArgs n, const SplitJob jx, const SplitJob jw,
                                                                 int nbn) {
     if ((int)blockIdx.x >= nbn) {
-        split_block<kNsThreads>(jw, (int)blockIdx.x - nbn);
+        split_block<kNsThreads, 0>(jw, (int)blockIdx.x - nbn);
         return;
     }
     const int lane = threadIdx.x & 63;
@@ -529,7 +572,13 @@ int split_rows(const float* x, int64_t ldx, int64_t M, const float* w, int64_t l
     const SplitJob jx = split_job(x ? x : w, x ? ldx : ldw, x ? M : N, K, x ? xbuf : wbuf);
     const SplitJob jw = split_job(w ? w : x, w ? ldw : ldx, w ? N : M, K, w ? wbuf : xbuf);
     const int64_t bx = x ? pad_to(M, kRowBlock) / kSplitRows : 0, bw = w ? pad_to(N, kRowBlock) / kSplitRows : 0;
-    hipLaunchKernelGGL((split_rows_kernel<512>), dim3((unsigned)(bx + bw)), dim3(512), 0, st, jx, jw, (int)bx);
+    const dim3 grid((unsigned)(bx + bw)), nt(512);
+#define MTL_SPLIT(U) hipLaunchKernelGGL((split_rows_kernel<512, U>), grid, nt, 0, st, jx, jw, (int)bx)
+    if (K <= 1024) MTL_SPLIT(4);
+    else if (K <= 2048) MTL_SPLIT(8);
+    else if (K <= 4096) MTL_SPLIT(16);
+    else MTL_SPLIT(0);
+#undef MTL_SPLIT
     return check_launch("split_rows");
 }
 

@@ -40,6 +40,19 @@ def test_product_matches_float64(M, N, K):
     assert _err(ops.linear_f32(x, w, b), x, w, b) < tol
 
 
+@pytest.mark.parametrize("K", [992, 1024, 1025, 2047, 2056, 4096, 4100])
+def test_split_widths(K):
+    """Either side of each width up to which the split holds a row in
+    registers (1024, 2048, 4096; past it two passes), with a row whose last
+    column is infinite; the bound of the products above."""
+    x, w, _ = _inputs(130, 70, K)
+    x[77, -1] = math.inf
+    got, rows = ops.linear_f32(x, w), torch.arange(130, device="cuda") != 77
+    assert torch.equal(got[77], torch.sign(w[:, -1]) * math.inf)
+    tol = 3 * 2.0 ** -22 + 2.0 ** -24 * math.sqrt(3 * K / 16 + 4)
+    assert _err(got[rows], x[rows], w) < tol
+
+
 @pytest.mark.parametrize("M,N,K", [(1024, 2048, 4096), (4096, 3072, 768), (512, 4096, 2048)])
 def test_error_not_above_the_fp32_product(M, N, K):
     x, w, _ = _inputs(M, N, K)
