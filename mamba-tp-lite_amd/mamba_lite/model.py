@@ -7,11 +7,13 @@ Same public surface as mamba-tp-lite's mamba_lite/model.py:
 Parameter names and shapes match the reference, so its state dicts (and HF
 `state-spaces/mamba-*-hf` checkpoints through from_pretrained) load as is.
 
-What runs where: the prefill's in_proj / x_proj / dt_proj / out_proj and the
-lm_head are torch GEMMs (hipBLASLt / rocBLAS).  The decode step's projections
+What runs where: the large fp32 products of a prefill (in_proj, out_proj and
+the lm_head from about 900 rows, or fewer rows of wide weights) run on libmtl's
+split-f16 GEMM; its x_proj and dt_proj, smaller products and bfloat16 ones are
+torch GEMMs (hipBLASLt / rocBLAS).  The decode step's projections
 run on libmtl kernels: GEMVs fused with the norm and the residual at batch
 <= 4, matrix-core skinny GEMMs at <= 32 tokens (in_proj fused with the conv
-step and x_proj).  The causal conv + SiLU, the selective scan (with dt bias,
+step and x_proj), and the lm_head of up to 16 rows of a wide model.  The causal conv + SiLU, the selective scan (with dt bias,
 softplus, D skip and SiLU gate fused), the single-token conv and SSM updates
 and the residual + RMSNorm are libmtl HIP kernels as well.  The model runs on
 the GPU only.
@@ -139,8 +141,9 @@ SKINNY_OUT_SPLIT = 4
 # mtl_sum_parts adds, and, inside MambaLM.prefill, out_proj as
 # SKINNY_OUT_SPLIT parts that the residual add sums.  The tied lm_head stays
 # on the library GEMM (faster at 64 x 50280 x 768: 66 against 69 us).
-# Prefills of more tokens keep torch's GEMMs on torch's own backend choice:
-# the library never changes that process-wide setting.
+# Prefills of more tokens take mtl_linear_f32 where it is the faster one and
+# otherwise keep torch's GEMMs on torch's own backend choice: the library
+# never changes that process-wide setting.
 _SKINNY_PREFILL = True
 
 # A prompt of at most 64 tokens on an fp32 model runs its whole layer stack
@@ -161,6 +164,9 @@ SHORT_PREFILL_NATIVE = True
 # path's by float rounding.
 LONG_PREFILL_NATIVE = True
 LONG_PREFILL_MAX_ELEMS = 1 << 23
+# From here on the per-op path costs the host no more than the GPU, and a
+# stack with hooks, replaced forwards or autocast keeps it (_plain_stack).
+LONG_PREFILL_PLAIN_ELEMS = 1 << 21
 # Up to LONG_PREFILL_SKINNY_ROWS token rows, at widths up to
 # LONG_PREFILL_SKINNY_MAX_D_MODEL, the one-call long prefill runs its
 # projections on the library's skinny GEMM (64-row chunks) instead of
@@ -228,9 +234,21 @@ def _linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     return ops.linear_f32(x, w, bias) if ops.linear_f32_ok(x, w, bias) else F.linear(x, w, bias)
 
 
+def _plain_modules(mod) -> bool:
+    """No hook and no replaced forward on mod or a module in it, all of which a raw launch would skip."""
+    d = mod.__dict__
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d) and \
+        all(m is None or _plain_modules(m) for m in d["_modules"].values())
+
+
+def _no_global_hooks() -> bool:
+    m = torch.nn.modules.module
+    return not (m._global_forward_hooks or m._global_forward_pre_hooks)
+
+
 def _linear_mod(mod, x: torch.Tensor) -> torch.Tensor:
     """mod(x) of a projection; a plain nn.Linear without hooks may take ops.linear_f32."""
-    if type(mod) is nn.Linear and not mod._forward_hooks and not mod._forward_pre_hooks and \
+    if type(mod) is nn.Linear and _plain_modules(mod) and _no_global_hooks() and \
             ops.linear_f32_ok(x, mod.weight, mod.bias):
         return ops.linear_f32(x, mod.weight, mod.bias)
     return mod(x)
@@ -663,6 +681,11 @@ class MambaLM(nn.Module):
         self._short_plan = (key, arr)
         return arr
 
+    def _plain_stack(self) -> bool:
+        """Whether the blocks are nothing but their launches: no hooks or
+        replaced forwards on a module, no autocast, transform or tracing."""
+        return ops.plain_call() and _no_global_hooks() and _plain_modules(self.layers)
+
     def _native_prefill_kind(self, b, l):
         """'short' (mtl_prefill_short), 'long' (mtl_prefill_long) or None for
         a prompt of b x l tokens of this model's shape."""
@@ -686,6 +709,8 @@ class MambaLM(nn.Module):
         D, N, K = cfg.d_inner, cfg.d_state, cfg.d_conv
         kind = self._native_prefill_kind(b, l)
         if kind is None or self.embedding.weight.dtype != torch.float32:
+            return None
+        if b * l * D > LONG_PREFILL_PLAIN_ELEMS and not self._plain_stack():
             return None
         for c in (cache, out_cache):
             if c is not None and not all(
@@ -834,7 +859,7 @@ class MambaLM(nn.Module):
         nl = len(self.layers)
         act = x.dtype
         if x.dim() != 2 or act not in (torch.float32, torch.bfloat16) or not x.is_cuda or not x.is_contiguous() or \
-                x.data_ptr() % 16 or len(cache.layers) != nl:
+                x.data_ptr() % 16 or len(cache.layers) != nl or act == torch.bfloat16 and not self._plain_stack():
             return None
         b, dm = x.shape
         D, N, K, R = cfg.d_inner, cfg.d_state, cfg.d_conv, cfg.dt_rank

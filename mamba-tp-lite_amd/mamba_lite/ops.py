@@ -914,10 +914,16 @@ def linear_f32_ok(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
     return _plain_forward(x, W) if bias is None else _plain_forward(x, W, bias)
 
 
+def plain_call() -> bool:
+    """No autocast, functorch or forward-mode transform, tracing or dispatch mode that a raw launch would bypass."""
+    return not torch.is_autocast_enabled("cuda") and torch.autograd.forward_ad._current_level < 0 and \
+        torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0 and \
+        not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+
+
 def _plain_forward(*ts) -> bool:
-    """Nothing of torch's between these tensors and a raw launch: no autograd, autocast or tensor subclass."""
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts) and \
-        not torch.is_autocast_enabled("cuda") and \
+    """Nothing of torch's between these tensors and a raw launch: no autograd, transform or tensor subclass."""
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts) and plain_call() and \
         not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
 
 

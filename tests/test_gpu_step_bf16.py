@@ -67,3 +67,24 @@ def test_bf16_one_call_step_matches_oracle_and_per_op(dm, expand, b, d_conv, bia
         st.capture()
         for g in got:
             assert torch.equal(st.replay(ids), g)
+
+
+@pytest.mark.parametrize("dtype,b,l", [(torch.bfloat16, 3, 1), (torch.float32, 2, 1024)])
+def test_a_hooked_stack_keeps_the_per_op_path(dtype, b, l):
+    """The bf16 step and an fp32 prompt of more than 2^21 token-channels run op by op where a module has a hook or
+    autocast is on, and in one call otherwise."""
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=640, n_layer=2, vocab_size=300)).eval().to(dtype)
+    cache = MambaCache.allocate(lm.cfg, b, torch.device("cuda"), dtype)
+    ids, x = torch.zeros(b, l, dtype=torch.long, device="cuda"), torch.zeros(b, 640, dtype=dtype, device="cuda")
+
+    def one_call():
+        with torch.no_grad():
+            return (lm._batched_step_layers(x, cache) if l == 1 else lm._prefill_native(ids, None, None)) is not None
+    assert one_call()
+    handle = lm.layers[1].mixer.out_proj.register_forward_hook(lambda *_: None)
+    assert not one_call()
+    handle.remove()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not one_call()
+    assert one_call()
