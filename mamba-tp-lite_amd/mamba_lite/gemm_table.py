@@ -1,7 +1,9 @@
 """Tuned GEMM solutions for the projection shapes of the prefill workloads.
 
-The projections (in_proj, x_proj, dt_proj, out_proj, the tied lm_head) are
-torch fp32 GEMMs on hipBLASLt / rocBLAS.  `gemm_table_gfx950.csv` is a torch
+The projections that mtl_linear_f32 does not take (x_proj, dt_proj, smaller
+in_proj / out_proj / lm_head products) are torch fp32 GEMMs on hipBLASLt /
+rocBLAS.  The figures below are from before that product, when every
+projection was one.  `gemm_table_gfx950.csv` is a torch
 TunableOp results table: for each prefill projection and lm_head shape of the
 mamba-130m model at batch 32 x 1024 tokens (and the lm_head of its 64-token
 prompt) and of the mamba-1.4b model at 1 x 1024 and 32 x 1024 tokens, it
