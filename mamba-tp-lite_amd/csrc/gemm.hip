@@ -483,8 +483,10 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
     // D[i][j] of a tile: column j = lane % 32 (an output column n), row
     // 8 (q / 4) + 4 (lane / 32) + q % 4 in register q (an output row m).  The
     // stores go through buffer resources that end at this tile's last row of
-    // y; a lane past the last column gets an offset past the end, so neither
-    // needs a branch.
+    // y.  A lane past the last column, or in the last tile past the last row,
+    // gets a VGPR offset past the end, so neither needs a branch; the SGPR
+    // offset, which the range check need not cover, holds a row of y's only.
+    const bool whole = m0 + BM <= a.M;
     const int mw = m0 + wm * WM, mpad = (a.M + kRowBlock - 1) / kRowBlock * kRowBlock;
     int en[TJ];
     float bn[TJ];
@@ -518,7 +520,9 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
             for (int q = 0; q < 16; ++q) {
                 const int ml = wm * WM + 32 * i + 8 * (q >> 2) + (q & 3);
                 const float v = __builtin_amdgcn_ldexpf(acc[i][j][q], -(em[q] + en[j])) + bn[j];
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ry, (int)vo, (int)(ml * ldy * 4), 0);
+                const uint32_t vq = whole || m0 + ml + 4 * g2 < a.M ? vo : 0xfffffff0u;
+                const int so = whole || m0 + ml < a.M ? (int)(ml * ldy * 4) : 0;
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ry, (int)vq, so, 0);
             }
         }
     }

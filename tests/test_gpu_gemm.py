@@ -1,12 +1,13 @@
 """mtl_linear_f32: the fp32 product on split f16 operands against the float64
 product, at tile edges and remainders, and its handling of extreme rows."""
+import ctypes
 import math
 
 import pytest
 import torch
 import torch.nn.functional as F
 
-from mamba_lite import ops
+from mamba_lite import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -69,6 +70,31 @@ def test_split_output_and_strided_weight():
     assert torch.equal(ops.linear_f32(x, sub, b), ops.linear_f32(x, sub.contiguous(), b))
     with pytest.raises(ValueError):
         ops.linear_f32(x, w, b, n_split=50)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 40, 32), (65, 129, 33), (257, 96, 100), (100, 1000, 48), (1793, 2049, 32),
+                                   (1000, 3001, 32), (4100, 8200, 32), (16500, 1100, 32)])
+def test_nothing_is_written_outside_the_outputs(M, N, K):
+    """y0 and y1 inside a larger filled buffer, 256 rows before and behind each and columns past N in every row
+    (the 64 x 64 tiles, the 128 x 128 and the 256 x 128 ones): what lies around them stays."""
+    x, w, b = _inputs(M, N, K)
+    lib = _lib.load()
+    for n0 in (N, 32):
+        widths = [n0, N - n0] if n0 < N else [N]
+        bufs = [torch.full((M + 512, n + 3), 7.25, device="cuda") for n in widths]
+        ws = torch.empty(lib.mtl_linear_f32_ws_bytes(M, N, K), dtype=torch.uint8, device="cuda")
+        a = _lib.LinearF32Args()
+        a.x, a.W, a.bias, a.ws, a.ws_bytes = x.data_ptr(), w.data_ptr(), b.data_ptr(), ws.data_ptr(), ws.numel()
+        a.ldx, a.ldw, a.M, a.N, a.K, a.n_split = K, K, M, N, K, n0
+        a.y0, a.ldy0 = bufs[0][256:].data_ptr(), n0 + 3
+        if n0 < N:
+            a.y1, a.ldy1 = bufs[1][256:].data_ptr(), N - n0 + 3
+        _lib.check(lib.mtl_linear_f32(ctypes.byref(a), torch.cuda.current_stream().cuda_stream), "linear_f32")
+        y = ops.linear_f32(x, w, b)
+        for buf, ref in zip(bufs, y.split(widths, 1)):
+            assert torch.equal(buf[256:256 + M, :ref.shape[1]], ref)
+            assert bool((buf[:256] == 7.25).all()) and bool((buf[256 + M:] == 7.25).all())
+            assert bool((buf[:, ref.shape[1]:] == 7.25).all())
 
 
 def test_rows_of_very_different_magnitude():
