@@ -66,7 +66,8 @@ int mtl_abi_version(void);
  * channel-major (sl == 1) or token-major (sd == 1) is fast, any other
  * stride pattern is rejected.  B, C: [b, N, l] with strides (sb, sn, sl).
  * h0 (nullable) and h_out (nullable): contiguous fp32 [b, D, N]; h_out may
- * be h0 (a state is read before it is overwritten, by the same thread).
+ * be h0 (each state is read before it is overwritten: by the same thread, or
+ * in segments, mtl_selective_scan_fwd_ws, from a copy in the workspace).
  * Two kernels compute this.  The tiled one (algo 1) walks the steps of a
  * sequence in turn with the state in registers: its time is the sequence
  * length times one step's latency, which is the right trade when the grid

@@ -56,6 +56,7 @@ struct ScanArgs {
     int seg_len;
     float* seg_dt;           // [segments, batch, D]
     float* seg_h;            // [segments, batch, D, N]
+    float* seg_h0;           // pass 1's copy of h0 [batch, D, N] where h_out overlaps it, else null
 };
 
 // E contiguous activations <-> floats (E a multiple of 4; 16-byte (fp32) or
@@ -185,7 +186,9 @@ template <> struct Buf4<uint16_t> {
 // Pass 1 runs each segment from zero states and leaves the states it reaches
 // and its sum of dt (the product of its decays is exp(A sum dt)); z, C and y
 // are left out.  Pass 2 folds the earlier segments' summaries, in order, into
-// its first states and runs the segment in full.
+// its first states and runs the segment in full.  Every segment of pass 2
+// starts from h0 while the last one writes h_out, so where the two overlap
+// pass 1 copies h0 to the workspace and pass 2 reads the copy.
 template <typename T, int NW, int SPW, int TT, bool CM, bool VEC, bool GEN, int PASS>
 __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const ScanArgs args) {
     ScanArgs a = args;
@@ -307,6 +310,10 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
         if (ok && a.a_is_log) av = -expf(av);
         a2[k] = av;
         h[k / 4][k % 4] = (PASS != 1 && ok && a.h0) ? a.h0[((int64_t)b * D + c0 + lane) * N + n] : 0.f;
+        if constexpr (PASS == 1) {
+            const int64_t i = ((int64_t)b * D + c0 + lane) * N + n;
+            if (a.seg_h0 && blockIdx.z == 0 && ok) a.seg_h0[i] = a.h0[i];
+        }
     }
     [[maybe_unused]] float dt_sum = 0.f;
     if constexpr (PASS == 2) {
@@ -682,8 +689,10 @@ void launch_scan(const ScanArgs& a, int64_t batch, hipStream_t st) {
         dim3 g1(grid.x, grid.y, (unsigned)(nseg - 1)), g2(grid.x, grid.y, (unsigned)nseg);
         if (a.softplus) hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, false, 1>), g1, dim3(NW * 64), 0, st, a);
         else hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, true, 1>), g1, dim3(NW * 64), 0, st, a);
-        if (plain) hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, false, 2>), g2, dim3(NW * 64), 0, st, a);
-        else hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, true, 2>), g2, dim3(NW * 64), 0, st, a);
+        ScanArgs a2 = a;
+        if (a.seg_h0) a2.h0 = a.seg_h0;
+        if (plain) hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, false, 2>), g2, dim3(NW * 64), 0, st, a2);
+        else hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, true, 2>), g2, dim3(NW * 64), 0, st, a2);
     } else if (plain) {
         hipLaunchKernelGGL((scan_fwd_kernel<T, NW, SPW, TT, CM, VEC, false, 0>), grid, dim3(NW * 64), 0, st, a);
     } else {
@@ -1169,7 +1178,8 @@ static int scan_segment_len(int64_t batch, int64_t dim, int64_t seqlen) {
 extern "C" int64_t mtl_selective_scan_ws_bytes(int64_t batch, int64_t dim, int64_t dstate, int64_t seqlen) {
     if (batch < 1 || dim < 1 || dstate < 1 || seqlen < 1) return 0;
     const int64_t len = scan_segment_len(batch, dim, seqlen);
-    return len ? (seqlen + len - 1) / len * batch * dim * (dstate + 1) * (int64_t)sizeof(float) : 0;
+    // a sum of dt and dstate states per segment, and the copy of h0
+    return len ? ((seqlen + len - 1) / len * (dstate + 1) + dstate) * batch * dim * (int64_t)sizeof(float) : 0;
 }
 
 extern "C" int mtl_selective_scan_fwd(const mtl_scan_params* p, mtl_stream_t stream) {
@@ -1240,6 +1250,9 @@ extern "C" int mtl_selective_scan_fwd_ws(const mtl_scan_params* p, void* ws, int
         a.seg_len = seg_len;
         a.seg_dt = static_cast<float*>(ws);
         a.seg_h = a.seg_dt + rows;
+        const int64_t states = p->batch * p->dim * p->dstate;
+        const uintptr_t h0 = reinterpret_cast<uintptr_t>(p->h0), ho = reinterpret_cast<uintptr_t>(p->h_out);
+        if (h0 && ho && h0 < ho + 4 * states && ho < h0 + 4 * states) a.seg_h0 = a.seg_h + rows * p->dstate;
     } else if (p->algo == 2 || (p->algo == 0 && p->batch * ((p->dim + 63) / 64) < kChunkedBelowWorkgroups &&
                                 p->seqlen > kChunkedMinSteps)) {
         MTL_REQUIRE(p->batch * ((p->dim + kLaneChannels - 1) / kLaneChannels) < (int64_t(1) << 31), "grid too large");

@@ -455,7 +455,7 @@ class MambaMixer(nn.Module):
         if cache is not None:
             h0 = cache.ssm_state.float().contiguous()
         y_store = torch.empty(b, l, Dm, device=x.device, dtype=x.dtype)
-        # h_out may be h0: each state is read and written by the same thread
+        # h_out may be h0 (mtl_selective_scan_fwd reads each state before it is overwritten)
         par = (self.A_log, self.D, self.dt_proj.bias)
         pbf = x.dtype == torch.bfloat16 and ops.bf16_params_ok(*par)
         A_log, Dv, dt_bias = par if pbf else map(_f32, par)

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from mamba_lite import _lib, ops
+from mamba_lite.model import MambaCache, MambaConfig, MambaLM
 
 pytestmark = pytest.mark.gpu
 
@@ -40,6 +41,40 @@ def test_segments_match_the_sequential_scan(b, D, L, N, dtype, cm):
         y, h = ops.selective_scan(c["u"], d, c["A"], c["B"], c["C"], **kw)
         yr, hr = ops.selective_scan(c["u"], d, c["A"], c["B"], c["C"], algo="tiled", **kw)
         assert rel(y, yr) < tol and rel(h, hr) < 1e-6
+
+
+@pytest.mark.parametrize("b,D,L,N", SHAPES)
+@pytest.mark.parametrize("dtype,cm", [(torch.float32, True), (torch.bfloat16, False)])
+def test_final_states_over_the_initial_ones(b, D, L, N, dtype, cm):
+    """h_out may be h0: every segment starts from h0 while the last one writes h_out, so the bits have to be those of
+    separate buffers."""
+    c = _case(b, D, L, N, dtype, cm)
+    run = lambda h0, **kw: ops.selective_scan(c["u"], c["delta"], c["A"], c["B"], c["C"], D=c["D"], z=c["z"],
+                                              delta_bias=c["bias"], h0=h0, **kw)
+    y, h = run(c["h0"])
+    kept = c["h0"].clone()
+    y2, h2 = run(kept, h_out=kept)
+    assert h2 is kept and torch.equal(h, h2) and torch.equal(y, y2)
+
+
+@pytest.mark.parametrize("d_model,b,l", [(768, 3, 333), (768, 7, 400), (2048, 1, 420), (768, 10, 700)])
+def test_a_prompt_that_continues_its_cache_in_place(d_model, b, l):
+    """MambaLM.prefill with out_cache = cache, in one call and op by op (10 x 700), at segmented sizes."""
+    torch.manual_seed(b)
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=d_model, n_layer=2, vocab_size=300)).eval()
+        ids = torch.randint(0, 300, (b, l))
+    assert _lib.load().mtl_selective_scan_ws_bytes(b, 2 * d_model, 16, l) > 0
+    cache = MambaCache.allocate(lm.cfg, b, "cuda", torch.float32)
+    for lc in cache.layers:
+        lc.conv_state.normal_(0, 0.6)
+        lc.ssm_state.normal_()
+    with torch.no_grad():
+        logits, new = lm.prefill(ids, cache)
+        logits2, got = lm.prefill(ids, cache, out_cache=cache)
+    assert got is cache and torch.equal(logits, logits2)
+    for p, q in zip(new.layers, cache.layers):
+        assert torch.equal(p.ssm_state, q.ssm_state) and torch.equal(p.conv_state, q.conv_state)
 
 
 def test_outside_the_rule_nothing_changes():
