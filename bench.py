@@ -42,21 +42,19 @@ HBM_PEAK_GBPS = 8000.0
 # VALU roofline of the scans: a wave64 VALU instruction holds one of the 1024
 # SIMDs for 4 cycles, a transcendental (half rate on gfx950) for 8; at the
 # 2.4 GHz peak engine clock.  Instruction counts per launch from rocprofv3
-# (SQ_INSTS_VALU, which counts MFMAs too, SQ_INSTS_VALU_TRANS_F32 and
-# SQ_INSTS_MFMA), recorded in profiles/; the scan's 4x4x1 MFMA holds its SIMD
-# for 8 cycles as well (SQ_VALU_MFMA_BUSY_CYCLES).
+# (SQ_INSTS_VALU, SQ_INSTS_VALU_TRANS_F32), recorded in profiles/.
 SIMDS, CLOCK_HZ = 1024, 2.4e9
-SCAN_VALU = {"fp32_b32_d1536_l1024": (70.8e6, 15.7e6, 3.15e6), "bf16_b32_d2048_l2048": (198.9e6, 42.0e6, 8.39e6)}
+SCAN_VALU = {"fp32_b32_d1536_l1024": (80.2e6, 15.7e6), "bf16_b32_d2048_l2048": (223.5e6, 42.0e6)}
 
 
 def valu_roofline(key, us):
     """VALU-bound time of a scan launch (every SIMD issuing every cycle) and
     the fraction of it the measured launch time reaches."""
-    valu, trans, mfma = SCAN_VALU[key]
-    floor_us = (valu + trans + mfma) * 4 / SIMDS / CLOCK_HZ * 1e6
+    valu, trans = SCAN_VALU[key]
+    floor_us = (valu + trans) * 4 / SIMDS / CLOCK_HZ * 1e6
     return {"bound": "valu", "floor_us": floor_us, "measured_us": us, "frac": floor_us / us,
-            "sq_insts_valu": valu, "sq_insts_valu_trans_f32": trans, "sq_insts_mfma": mfma,
-            "how": "(SQ_INSTS_VALU + SQ_INSTS_VALU_TRANS_F32 + SQ_INSTS_MFMA) x 4 cycles / 1024 SIMDs at 2.4 GHz"}
+            "sq_insts_valu": valu, "sq_insts_valu_trans_f32": trans,
+            "how": "(SQ_INSTS_VALU + SQ_INSTS_VALU_TRANS_F32) x 4 cycles / 1024 SIMDs at 2.4 GHz"}
 
 # isolated selective-scan workload
 SCAN_B, SCAN_D, SCAN_L, SCAN_N = 32, 1536, 1024, 16
@@ -626,9 +624,9 @@ def main():
                          "traffic": traffic_from_profiles("scan_fp32_b32_d1536_l1024"),
                          "kernel": "scan_fwd_kernel<float, NW=4, SPW=4, TT=16, channel-major>",
                          "algorithmic_bytes": SCAN_BYTES,
-                         "limiter": "VALU issue and the access pattern together: 90 VALU instructions per 64 "
-                                    "(channel, step) pairs, 68 of them the 16-state recurrence, 4 on the matrix cores "
-                                    "(rocprofv3 counters; 146 us of issue at 100% and the 2.4 GHz peak "
+                         "limiter": "VALU issue and the access pattern together: 102 VALU instructions per 64 "
+                                    "(channel, step) pairs, 80 of them the 16-state recurrence, 76% VALU busy "
+                                    "(rocprofv3 counters; 156 us of VALU issue at 100% and the 2.4 GHz peak "
                                     "clock, scan_valu_roofline); the same channel-major "
                                     "u/delta/z/y stream with no arithmetic takes 173 us (4.65 TB/s)"},
         })

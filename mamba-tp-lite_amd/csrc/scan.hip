@@ -19,15 +19,12 @@
 //   * Each wavefront writes its partial y_t (sum over its states) to LDS;
 //     the loader threads add the 4 partials in a fixed order (deterministic),
 //     apply (y + D*u) * silu(z) and store y coalesced.
-// Per (channel, t, state) the inner loop costs one v_exp_f32, three VALU ops
-// (dt * A, the decay of h, the C fma) and a quarter of a matrix instruction:
-// the injection of dt u B is, for 64 channels and a wavefront's 4 states, 16
-// rank-1 products of 4 channels by 4 states, which v_mfma_f32_4x4x1 adds to
-// the decayed states in place of 4 multiplies and 4 fused adds.  It issues
-// alone on the SIMD for its 8 cycles, so the gain is that of 4 VALU
-// instructions for 2: [32, 2048, 2048] bf16 with its conv 544 -> 534 us, fp32
-// [32, 1536, 1024] 208.2 -> 206.2 us, the error against float64 unchanged
-// (2.0e-7 / 2.1e-7).  dt is staged in log2 units (dt * log2 e, which
+// Per (channel, t, state) the inner loop costs one v_exp_f32 and four VALU
+// ops (mul, mul, fma, fma).  The injection of dt u B as a rank-1 product on
+// v_mfma_f32_4x4x1 issues alone on the SIMD, gave 1-2% ([32, 2048, 2048] bf16
+// with its conv 544 -> 534 us) and rounds the decayed state once more per
+// step (error against float64 2.06e-7 -> 2.16e-7): not taken.
+// dt is staged in log2 units (dt * log2 e, which
 // softplus_l2_f returns directly), so exp(dt * A) is exp2(dt_l2 * A); the
 // injection dt * u * B then takes its ln 2 from B, scaled where B is staged.
 
@@ -298,10 +295,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
 
     // scan registers: states [wave*SPW, wave*SPW + SPW) of channel c0 + lane
     const bool lane_ok = c0 + lane < D;
-    // (state k in h[k / 4][k % 4])
-    constexpr bool MF = SPW % 4 == 0;
-    F4v h[(SPW + 3) / 4];
-    float a2[SPW];
+    float h[SPW], a2[SPW];
 #pragma unroll
     for (int k = 0; k < SPW; ++k) {
         const int n = wave * SPW + k;
@@ -309,7 +303,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
         float av = ok ? load_param(a.A, (int64_t)(c0 + lane) * N + n, pbf) : 0.f;
         if (ok && a.a_is_log) av = -expf(av);
         a2[k] = av;
-        h[k / 4][k % 4] = (PASS != 1 && ok && a.h0) ? a.h0[((int64_t)b * D + c0 + lane) * N + n] : 0.f;
+        h[k] = (PASS != 1 && ok && a.h0) ? a.h0[((int64_t)b * D + c0 + lane) * N + n] : 0.f;
         if constexpr (PASS == 1) {
             const int64_t i = ((int64_t)b * D + c0 + lane) * N + n;
             if (a.seg_h0 && blockIdx.z == 0 && ok) a.seg_h0[i] = a.h0[i];
@@ -326,7 +320,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
             for (int k = 0; k < SPW; ++k) {
                 const int n = wave * SPW + k;
                 const float e = a.seg_h[row * N + min(n, N - 1)];
-                h[k / 4][k % 4] = fmaf(__builtin_amdgcn_exp2f(sd * a2[k]), h[k / 4][k % 4], n < N ? e : 0.f);
+                h[k] = fmaf(__builtin_amdgcn_exp2f(sd * a2[k]), h[k], n < N ? e : 0.f);
             }
         }
     }
@@ -481,17 +475,13 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
         // the B / C broadcasts of step st are read two steps before their use
         // (at 8 states per wavefront the registers for that would spill)
         constexpr int PRE = SPW <= 4 ? 2 : 0;
-        constexpr int NB = MF ? SPW / 4 : SPW;         // B registers of a step
-        float bq[TT][NB], cq[TT][SPW];
-        auto read_b = [&](int st, int k) __attribute__((always_inline)) {
-            return s_B[kc * TT + st][wave * SPW + (MF ? 4 * k + (lane & 3) : k)];
-        };
+        float bq[TT][SPW], cq[TT][SPW];
         auto read_bc = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
-            for (int k = 0; k < NB; ++k) bq[st][k] = read_b(st, k);
-#pragma unroll
-            for (int k = 0; k < SPW; ++k)
+            for (int k = 0; k < SPW; ++k) {
+                bq[st][k] = s_B[kc * TT + st][wave * SPW + k];
                 if constexpr (PASS != 1) cq[st][k] = s_C[kc * TT + st][wave * SPW + k];
+            }
         };
 #pragma unroll
         for (int st = 0; st < PRE; ++st) read_bc(st);
@@ -508,26 +498,12 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
                 if (PRE > 0 && st + PRE < TT) read_bc(st + PRE);
                 if constexpr (PASS == 1) dt_sum += dts[q];
                 float acc = 0.f;
-                auto ck = [&](int k) __attribute__((always_inline)) {
-                    return PRE > 0 ? cq[st][k] : s_C[kc * TT + st][wave * SPW + k];
-                };
-                if constexpr (MF) {
 #pragma unroll
-                    for (int k = 0; k < SPW; ++k) h[k / 4][k % 4] *= __builtin_amdgcn_exp2f(dts[q] * a2[k]);
-#pragma unroll
-                    for (int g = 0; g < SPW / 4; ++g)
-                        h[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(PRE > 0 ? bq[st][g] : read_b(st, g), dxs[q], h[g],
-                                                                  0, 0, 0);
-#pragma unroll
-                    for (int k = 0; k < SPW; ++k)
-                        if constexpr (PASS != 1) acc = fmaf(h[k / 4][k % 4], ck(k), acc);
-                } else {
-#pragma unroll
-                    for (int k = 0; k < SPW; ++k) {
-                        const float bk = PRE > 0 ? bq[st][k] : read_b(st, k);
-                        h[k / 4][k % 4] = fmaf(__builtin_amdgcn_exp2f(dts[q] * a2[k]), h[k / 4][k % 4], dxs[q] * bk);
-                        if constexpr (PASS != 1) acc = fmaf(h[k / 4][k % 4], ck(k), acc);
-                    }
+                for (int k = 0; k < SPW; ++k) {
+                    const float bk = PRE > 0 ? bq[st][k] : s_B[kc * TT + st][wave * SPW + k];
+                    h[k] = fmaf(__builtin_amdgcn_exp2f(dts[q] * a2[k]), h[k], dxs[q] * bk);
+                    if constexpr (PASS != 1)
+                        acc = fmaf(h[k], PRE > 0 ? cq[st][k] : s_C[kc * TT + st][wave * SPW + k], acc);
                 }
                 yq[q] = acc;
             }
@@ -674,7 +650,7 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
 #pragma unroll
         for (int k = 0; k < SPW; ++k) {
             const int n = wave * SPW + k;
-            if (lane_ok && n < N) ho[((int64_t)b * D + c0 + lane) * N + n] = h[k / 4][k % 4];
+            if (lane_ok && n < N) ho[((int64_t)b * D + c0 + lane) * N + n] = h[k];
         }
     }
 }

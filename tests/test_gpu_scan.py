@@ -382,3 +382,32 @@ def test_chunked_matches_tiled_and_continues(dtype, b, L, k):
     yb, hb = _run(cut(c, slice(k, L)), "tm", h0=ha, dtype=dtype, algo="chunked")
     assert_rel(np.concatenate([ya, yb], -1), y2, tol, "continued y")
     assert_rel(hb, h2, 1e-4, "continued h")
+
+
+@pytest.mark.parametrize("cm", [True, False])
+@pytest.mark.parametrize("N", [4, 16, 32])
+def test_tiled_states_are_the_fused_recurrence(cm, N):
+    """Each step of the tiled kernel rounds a state once: h = fma(decay, h, dt u B), bit for bit.  The decay of a
+    constant dt is read from the kernel itself (one step from h0 = 1 with u = 0); the fused product and sum are
+    formed in float64, where the product of two floats is exact."""
+    b, D, L = 2, 70, 301
+    rng = np.random.default_rng(N)
+    f32 = np.float32
+    delta = np.exp(rng.uniform(np.log(1e-3), np.log(0.1), (b, D, 1))).astype(f32)
+    u, B = rng.standard_normal((b, D, L)).astype(f32), rng.standard_normal((b, N, L)).astype(f32)
+    A = _t(-np.tile(np.arange(1, N + 1, dtype=f32), (D, 1)))
+    h0 = rng.standard_normal((b, D, N)).astype(f32)
+
+    def run(steps, u_, start):
+        lay = (lambda t: t) if cm else (lambda t: t.transpose(1, 2).contiguous().transpose(1, 2))
+        d = lay(_t(np.repeat(delta, steps, 2)))
+        return ops.selective_scan(lay(_t(u_)), d, A, _t(B[..., :steps]), _t(B[..., :steps]), h0=_t(start),
+                                  delta_softplus=False, algo="tiled")[1].cpu().numpy()
+
+    decay = run(1, np.zeros((b, D, 1), f32), np.ones((b, D, N), f32)).astype(np.float64)
+    dt_l2, Bs = delta * f32(np.log2(np.e)), B * f32(np.log(2))      # staged in log2 units, ln 2 on B
+    h = h0
+    for t in range(L):
+        inj = (dt_l2[..., 0] * u[..., t])[..., None] * Bs[:, None, :, t]
+        h = (decay * h + inj).astype(f32)
+    assert np.array_equal(run(L, u, h0), h)
