@@ -28,9 +28,12 @@
 // and a split row takes exactly the bytes of its fp32 values.
 //
 // A row that holds an infinity or NaN cannot be split; its exponent is
-// marked, and the outputs that touch it are computed from the fp32 operands
-// by plain fp32 sums in the epilogue, so infinities and NaN come out as an
-// fp32 product gives them.
+// marked, and the epilogue computes the outputs that touch it from the fp32
+// operands on the fp32 matrix instructions, so infinities and NaN come out as
+// an fp32 product gives them.  Measured, us, no row / one row of x / every row
+// marked (library fp32 product): 4096 x 3072 x 768 72 / 128 / 362 (162), 1024 x
+// 8192 x 2048 121 / 249 / 572 (265), 32768 x 3072 x 768 424 / 483 / 2610 (1107);
+// a lane's own sum over K per output took hundreds of products' time.
 //
 // Measured (us; library fp32 GEMM -> this product, plus the splits of X and W):
 //   32768 x 3072 x 768 (mamba-130m in_proj, 32 x 1024 tokens)   1246 -> 449 + 41
@@ -57,16 +60,14 @@ typedef float F16v __attribute__((ext_vector_type(16)));
 constexpr int kPanel = 16;                 // columns of a panel
 constexpr int kPanelBytes = 64;            // bytes of a row in it
 constexpr int kRowBlock = 64;              // rows of a block
-constexpr int kExpSpecial = 1 << 20;       // exponent mark of a row with infinities (kExpNan: with a NaN)
-constexpr int kExpNan = 1 << 21;
+constexpr int kExpSpecial = 1 << 20;       // exponent mark of a row that cannot be split
 
 // ------------------------------------------------------------------ splitting
 // One workgroup takes 16 rows: lane = (row of 16, 8-column block of 4), so a
 // wavefront reads whole 128-byte runs of 16 rows and writes 1 KB runs of two
 // panels; the wavefronts take 32-column units in turn.  Each row's largest
 // |x| is found first (bit patterns, so a NaN is the largest), then the parts
-// are written.  The mark of a row with non-finite values is its largest bit
-// pattern: above inf's it holds a NaN.
+// are written.
 constexpr int kSplitRows = 16;
 
 __device__ __forceinline__ void load8(const float* p, int n, bool vec, float* v) {
@@ -82,7 +83,7 @@ __device__ __forceinline__ void load8(const float* p, int n, bool vec, float* v)
 
 // the power of two of a row whose largest magnitude has the bits `mx`
 __device__ __forceinline__ int split_exp(uint32_t mx) {
-    if (mx >= 0x7f800000u) return mx > 0x7f800000u ? kExpNan : kExpSpecial;
+    if (mx >= 0x7f800000u) return kExpSpecial;
     // (a zero or subnormal row takes the largest scale, 2^126)
     return min(14 - ((int)(mx >> 23) - 127), 126);
 }
@@ -309,7 +310,16 @@ struct GemmArgs {
     int64_t ldx, ldw;
     int M, N, K, n_split;
     int tm, tn;                            // tiles along M and N
+    bool vec;                              // 16-byte aligned fp32 rows
 };
+
+// 4 consecutive columns of an fp32 row, zeros past the n there are
+__device__ __forceinline__ F4v load4(const float* p, int n) {
+    F4v v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = j < n ? p[j] : 0.f;
+    return v;
+}
 
 // Mapping: a workgroup of 4 wavefronts takes a BM x BN tile of Y, each
 // wavefront WM x WN of it as 32 x 32 MFMA tiles; the K loop walks stages of PK
@@ -488,6 +498,13 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
     // offset, which the range check need not cover, holds a row of y's only.
     const bool whole = m0 + BM <= a.M;
     const int mw = m0 + wm * WM, mpad = (a.M + kRowBlock - 1) / kRowBlock * kRowBlock;
+    auto row_exps = [&](int mt, int* em) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int4 v = *reinterpret_cast<const int4*>(a.ex + min(mt + 8 * q + 4 * g2, mpad - 4));
+            em[4 * q] = v.x; em[4 * q + 1] = v.y; em[4 * q + 2] = v.z; em[4 * q + 3] = v.w;
+        }
+    };
     int en[TJ];
     float bn[TJ];
     bool special = false;
@@ -501,12 +518,9 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
 #pragma unroll
     for (int i = 0; i < TI; ++i) {
         int em[16];
+        row_exps(mw + 32 * i, em);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int4 v = *reinterpret_cast<const int4*>(a.ex + min(mw + 32 * i + 8 * q + 4 * g2, mpad - 4));
-            em[4 * q] = v.x; em[4 * q + 1] = v.y; em[4 * q + 2] = v.z; em[4 * q + 3] = v.w;
-            special |= max(max(v.x, v.y), max(v.z, v.w)) >= kExpSpecial;
-        }
+        for (int q = 0; q < 16; ++q) special |= em[q] >= kExpSpecial;
 #pragma unroll
         for (int j = 0; j < TJ; ++j) {
             const int nt = n0 + wn * WN + 32 * j;            // n_split is a multiple of 32 (host-checked)
@@ -526,21 +540,60 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
             }
         }
     }
-    // outputs of rows that could not be split, over the values stored above by the same lanes
+    // outputs of rows that could not be split, over the values stored above by
+    // the same lanes: the 32 x 32 tiles that hold any, from the fp32 operands.
+    // Lane half g2 takes 4 consecutive columns of its row; MFMA q of a group
+    // of 8 columns sums columns q and q + 4.
     if (__any(special)) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        for (int j = 0; j < TJ; ++j) {
-            const int n = n0 + wn * WN + 32 * j + r32;
-            for (int mi = 0; mi < 16 * TI; ++mi) {
-                const int q = mi & 15, m = mw + (mi >> 4) * 32 + 8 * (q >> 2) + 4 * g2 + (q & 3);
-                if (m >= a.M || n >= a.N || (a.ex[m] < kExpSpecial && a.ew[n] < kExpSpecial)) continue;
-                const float* x = a.x32 + m * a.ldx;
-                const float* w = a.w32 + n * a.ldw;
-                float v = 0.f;
-                for (int k = 0; k < a.K; ++k) v = fmaf(x[k], w[k], v);
-                if (a.bias) v += a.bias[n];
-                if (n < a.n_split) a.y0[m * a.ldy0 + n] = v;
-                else a.y1[m * a.ldy1 + n - a.n_split] = v;
+        for (int t = 0; t < TI * TJ; ++t) {
+            const int mt = mw + 32 * (t / TJ), n = n0 + wn * WN + 32 * (t % TJ) + r32;
+            const int m = min(mt + r32, a.M - 1), nc = min(n, a.N - 1);
+            const bool ns_ = a.ew[nc] >= kExpSpecial;
+            if (!__any(ns_ || a.ex[m] >= kExpSpecial)) continue;
+            const float* x = a.x32 + m * a.ldx + 4 * g2;
+            const float* w = a.w32 + nc * a.ldw + 4 * g2;
+            F16v c;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) c[q] = 0.f;
+            constexpr int KG = 4;                            // groups of 8 columns loaded at a time
+            struct Cols { F4v x[KG], w[KG]; } cur, nxt;
+            auto load = [&](Cols& d, int k) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < KG; ++u) { d.x[u] = ld4(x + k + 8 * u); d.w[u] = ld4(w + k + 8 * u); }
+            };
+            auto mma = [&](const Cols& d) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < KG; ++u)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        c = __builtin_amdgcn_mfma_f32_32x32x2f32(d.x[u][q], d.w[u][q], c, 0, 0, 0);
+            };
+            const int whole_k = a.vec ? a.K & -(8 * KG) : 0;
+            if (whole_k) load(cur, 0);
+            for (int k = 0; k < whole_k; k += 8 * KG, cur = nxt) {
+                load(nxt, min(k + 8 * KG, whole_k - 8 * KG));
+                __builtin_amdgcn_sched_barrier(0);
+                mma(cur);
+            }
+            for (int k = whole_k; k < a.K; k += 8 * KG) {    // the last columns, or all of unaligned rows
+#pragma unroll
+                for (int u = 0; u < KG; ++u) {
+                    const int left = a.K - k - 8 * u - 4 * g2;
+                    cur.x[u] = load4(x + k + 8 * u, left);
+                    cur.w[u] = load4(w + k + 8 * u, left);
+                }
+                mma(cur);
+            }
+            const float bias = a.bias ? a.bias[nc] : 0.f;
+            int em[16];
+            row_exps(mt, em);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int mq = mt + 8 * (q >> 2) + 4 * g2 + (q & 3);
+                if (mq >= a.M || n >= a.N || (!ns_ && em[q] < kExpSpecial)) continue;
+                if (n < a.n_split) a.y0[mq * a.ldy0 + n] = c[q] + bias;
+                else a.y1[mq * a.ldy1 + n - a.n_split] = c[q] + bias;
             }
         }
     }
@@ -624,6 +677,7 @@ int gemm_split(const SplitGemm& g, hipStream_t st) {
     a.bias = g.bias;
     a.x32 = g.x; a.ldx = g.ldx; a.w32 = g.w; a.ldw = g.ldw;
     a.M = (int)g.M; a.N = (int)g.N; a.K = (int)g.K;
+    a.vec = x.vec && w.vec;
     // Tile by the number of tiles each gives (us at M x N x K; 256 x 128, 128 x
     // 128, 64 x 64): 32768 x 3072 x 768 449 / 499 / 739, 512 x 50280 x 768 147 /
     // 158 / 234 (786 large tiles); 768 x 8192 x 2048 100 / 90 / 103, 512 x 8192 x
