@@ -294,9 +294,16 @@ int mtl_quant_dequant_sum_fp16(const float* const* parts, int32_t nparts, int64_
  *   Y[m][n] = sum_k x[m][k] W[n][k] (+ bias[n]),  nn.Linear on M token rows
  * (model.py:197, 240, 339).  Every operand is split into two f16 parts under a
  * power of two per row and each product takes three MFMAs with fp32
- * accumulation: the error against exact arithmetic is below that of an fp32
- * matrix product (csrc/gemm.hip).  Infinities and NaN come out as an fp32
- * product gives them.
+ * accumulation.  The parts hold 22 significand bits of a value down to 2^-17 of
+ * its row's largest and 2^-40 of that largest below it, so beside the fp32
+ * sum's rounding y[m][n] may be off by
+ *   2^-22 sum_k |x W| + 2^-40 (max|x[m]| sum_k |W[n]| + max|W[n]| sum_k |x[m]|).
+ * Rows (of x or W) for which that could exceed an fp32 product's own error are
+ * not split: more than 1/16 of the nonzero values under 2^-20 of the largest,
+ * or fewer than 32 nonzero values, or an infinity or NaN.  Outputs that touch
+ * one are summed by fp32 matrix instructions, infinities and NaN come out as
+ * an fp32 product gives them.  Of Gaussian operands the error is 0.6 to 0.7 of
+ * an fp32 matrix product's (csrc/gemm.hip).
  *   x: [M, K], row stride ldx; W: [N, K], row stride ldw; unit column stride.
  *   y0: [M, N], row stride ldy0 < 2^21; with y1 (not NULL), columns [0,
  *       n_split) go to y0 and the others to y1 (n_split a multiple of 32).

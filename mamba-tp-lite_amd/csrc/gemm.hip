@@ -27,8 +27,18 @@
 // contiguous 4 KB runs, a tile's whole operand lies in one stretch of memory,
 // and a split row takes exactly the bytes of its fp32 values.
 //
-// A row that holds an infinity or NaN cannot be split; its exponent is
-// marked, and the epilogue computes the outputs that touch it from the fp32
+// Three kinds of rows are not split (split_ok):
+//   * a row that holds an infinity or NaN;
+//   * a row of great spread, more than 1/16 of whose nonzero values lie under
+//     2^-20 of its largest: those keep under 20 bits, and where the other
+//     operand is zero or small at the large ones the product shows it (K 768,
+//     one value 2^20 times the rest against a zero weight: 7.9e-7 split, 5.0e-7
+//     fp32; at 2^17 and below 2.4e-7 split).  Gaussian rows have 1e-5 of their
+//     values there, gated y rows up to a few percent;
+//   * a row of fewer than 32 nonzero values, whose fp32 sums round so little
+//     that 22 bits per operand would be the larger error (a row that selects
+//     one column is exact in fp32).
+// The exponent of such a row is marked, and the epilogue computes the outputs that touch it from the fp32
 // operands on the fp32 matrix instructions, so infinities and NaN come out as
 // an fp32 product gives them.  Measured, us, no row / one row of x / every row
 // marked (library fp32 product): 4096 x 3072 x 768 72 / 128 / 362 (162), 1024 x
@@ -47,6 +57,8 @@
 // 8.1e-7 to 5.0e-7 at 2048 and 1.15e-6 to 7.1e-7 at 4096.  With the
 // conversion inside the product's loop (fp32 tiles in LDS, no split pass) the
 // 1024 x 8192 x 2048 product took 147 us in place of 100 + 42.
+
+#include <type_traits>
 
 #include "common.h"
 #include "gemm.h"
@@ -79,6 +91,24 @@ __device__ __forceinline__ void load8(const float* p, int n, bool vec, float* v)
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = j < n ? p[j] : 0.f;
     }
+}
+
+// Whether a row's split holds it as well as fp32 does, from its largest
+// magnitude's bits and its counts over `cols` values: those that are not zero,
+// and those under 2^-20 of the largest.
+struct RowCount {
+    float below;                           // 2^-20 of the largest (0 where that is no normal number: none is small)
+    int nonzero = 0, small = 0;
+    __device__ __forceinline__ explicit RowCount(uint32_t mx)
+        : below(mx >= (21u << 23) ? __uint_as_float(mx - (20u << 23)) : 0.f) {}
+    __device__ __forceinline__ void add(float v) {
+        nonzero += v != 0.f;
+        small += fabsf(v) < below;         // (zeros too)
+    }
+};
+__device__ __forceinline__ bool split_ok(int nonzero, int small, int cols) {
+    small -= small ? cols - nonzero : 0;   // without the zeros (all or none of them were counted)
+    return (int64_t)small * 16 <= nonzero && (nonzero >= 32 || nonzero == 0);
 }
 
 // the power of two of a row whose largest magnitude has the bits `mx`
@@ -141,6 +171,7 @@ template <int NT, int U>
 __device__ __forceinline__ void split_block(const SplitJob& j, int64_t block) {
     constexpr int NW = NT / 64, UR = U > 0 ? U : 1;
     __shared__ uint32_t s_max[NW][kSplitRows];
+    __shared__ int2 s_cnt[NW][kSplitRows];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane >> 2, blk = lane & 3, K = j.K;
     const bool vec = j.vec;
@@ -174,12 +205,14 @@ __device__ __forceinline__ void split_block(const SplitJob& j, int64_t block) {
 #pragma unroll
     for (int w = 0; w < NW; ++w) mx = max(mx, s_max[w][r]);
     const int e = split_exp(mx);
-    if (wave == 0 && blk == 0) j.exps[row] = row < j.rows ? e : 0;     // exps is padded to whole row blocks
+    RowCount cnt(mx);
     // a marked row's parts are never used: zeros do
     const float scale = e >= kExpSpecial ? 0.f : __uint_as_float((uint32_t)(e + 127) << 23);
     const int np = 2 * units;
     uint8_t* const q = j.out + (row / kRowBlock * np) * (kRowBlock * kPanelBytes) + (row % kRowBlock) * kPanelBytes;
     auto put = [&](float* v, int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) cnt.add(v[i]);
         if (e >= kExpSpecial) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = 0.f;
@@ -199,6 +232,20 @@ __device__ __forceinline__ void split_block(const SplitJob& j, int64_t block) {
             load8(p + c, K - c, vec, held[0]);
             put(held[0], u);
         }
+    }
+    auto quad_sum = [](int v) __attribute__((always_inline)) {
+        v += (int)dpp_mov_u<kDppXor1>((uint32_t)v);
+        return v + (int)dpp_mov_u<kDppXor2>((uint32_t)v);
+    };
+    const int2 c4 = make_int2(quad_sum(cnt.nonzero), quad_sum(cnt.small));
+    if (blk == 0) s_cnt[wave][r] = c4;
+    // (a barrier for the LDS writes only: __syncthreads would wait for the stores)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (wave == 0 && blk == 0) {                   // exps is padded to whole row blocks
+        int2 c = c4;
+#pragma unroll
+        for (int w = 1; w < NW; ++w) { c.x += s_cnt[w][r].x; c.y += s_cnt[w][r].y; }
+        j.exps[row] = row >= j.rows ? 0 : split_ok(c.x, c.y, 32 * units) ? e : kExpSpecial;
     }
 }
 
@@ -281,8 +328,17 @@ __global__ void __launch_bounds__(kNsThreads) norm_split_kernel(const NormArgs n
         p[0] = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
         p[1] = make_float4(v[u][4], v[u][5], v[u][6], v[u][7]);
     }
-    const int e = split_exp(group_umax<64>(mx));
-    if (lane == 0) jx.exps[row] = e;
+    mx = group_umax<64>(mx);
+    const int e = split_exp(mx);
+    RowCount cnt(mx);
+#pragma unroll
+    for (int u = 0; u < RU; ++u)
+        if (u * 512 + lane * 8 < cols) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) cnt.add(v[u][j]);
+        }
+    const bool ok = split_ok((int)group_sum<64>((float)cnt.nonzero), (int)group_sum<64>((float)cnt.small), cols);
+    if (lane == 0) jx.exps[row] = ok ? e : kExpSpecial;
     if (e >= kExpSpecial) return;          // a marked row's parts are never used
     const float scale = __uint_as_float((uint32_t)(e + 127) << 23);
     const int np = cols / kPanel;
@@ -365,8 +421,7 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
     const int n0 = __builtin_amdgcn_readfirstlane(in_g / gm * BN);
 
     // copy lane: row 16 g + lane / 4 of the stage; position lane % 4 of a row
-    // takes 16-byte chunk (lane % 4) ^ ((row >> 1) & 3), so 8 consecutive rows'
-    // reads of one chunk hit distinct banks
+    // takes 16-byte chunk (lane % 4) ^ ((row >> 2) & 3) (above)
     const int np = (a.K + 31) / 32 * 2;                    // panels (K padded to 32)
     const uint8_t* base[NI];
 #pragma unroll
@@ -403,7 +458,7 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
 
     const int r32 = lane & 31, g2 = lane >> 5;
     // byte offsets of this lane's hi chunk in rows 32 i + r32 of a tile (the
-    // swizzle depends on r32 only, as 32 i is a multiple of 8)
+    // swizzle, of a period of 16 rows, depends on r32 only)
     const int sw = (r32 >> 2) & 3;
     const uint32_t o_hi = r32 * kPanelBytes + ((2 * g2) ^ sw) * 16, o_lo = r32 * kPanelBytes + ((2 * g2 + 1) ^ sw) * 16;
     struct Frag { H8 xh[TI], xl[TI], wh[TJ], wl[TJ]; };
@@ -496,7 +551,6 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
     // y.  A lane past the last column, or in the last tile past the last row,
     // gets a VGPR offset past the end, so neither needs a branch; the SGPR
     // offset, which the range check need not cover, holds a row of y's only.
-    const bool whole = m0 + BM <= a.M;
     const int mw = m0 + wm * WM, mpad = (a.M + kRowBlock - 1) / kRowBlock * kRowBlock;
     auto row_exps = [&](int mt, int* em) __attribute__((always_inline)) {
 #pragma unroll
@@ -515,31 +569,37 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
         bn[j] = a.bias ? a.bias[nc] : 0.f;
         special |= en[j] >= kExpSpecial;
     }
+    auto store = [&](auto all_rows) __attribute__((always_inline)) {
+        constexpr bool ALL = decltype(all_rows)::value;
 #pragma unroll
-    for (int i = 0; i < TI; ++i) {
-        int em[16];
-        row_exps(mw + 32 * i, em);
+        for (int i = 0; i < TI; ++i) {
+            int em[16], top = 0;
+            row_exps(mw + 32 * i, em);
 #pragma unroll
-        for (int q = 0; q < 16; ++q) special |= em[q] >= kExpSpecial;
+            for (int q = 0; q < 16; ++q) top = max(top, em[q]);
+            special |= top >= kExpSpecial;
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-            const int nt = n0 + wn * WN + 32 * j;            // n_split is a multiple of 32 (host-checked)
-            const bool first = nt < a.n_split;
-            const int64_t ldy = first ? a.ldy0 : a.ldy1;
-            const int n = nt + r32, col = first ? n : n - a.n_split;
-            float* yt = (first ? a.y0 : a.y1) + (int64_t)m0 * ldy;
-            const auto ry = __builtin_amdgcn_make_buffer_rsrc(yt, (short)0, (int)(min(BM, a.M - m0) * ldy * 4), 0x00020000);
-            const uint32_t vo = n < a.N ? (uint32_t)(col + 4 * g2 * ldy) * 4u : 0xfffffff0u;
+            for (int j = 0; j < TJ; ++j) {
+                const int nt = n0 + wn * WN + 32 * j;        // n_split is a multiple of 32 (host-checked)
+                const bool first = nt < a.n_split;
+                const int64_t ldy = first ? a.ldy0 : a.ldy1;
+                const int n = nt + r32, col = first ? n : n - a.n_split;
+                float* yt = (first ? a.y0 : a.y1) + (int64_t)m0 * ldy;
+                const auto ry = __builtin_amdgcn_make_buffer_rsrc(yt, (short)0, (int)(min(BM, a.M - m0) * ldy * 4), 0x00020000);
+                const uint32_t vo = n < a.N ? (uint32_t)(col + 4 * g2 * ldy) * 4u : 0xfffffff0u;
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int ml = wm * WM + 32 * i + 8 * (q >> 2) + (q & 3);
-                const float v = __builtin_amdgcn_ldexpf(acc[i][j][q], -(em[q] + en[j])) + bn[j];
-                const uint32_t vq = whole || m0 + ml + 4 * g2 < a.M ? vo : 0xfffffff0u;
-                const int so = whole || m0 + ml < a.M ? (int)(ml * ldy * 4) : 0;
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ry, (int)vq, so, 0);
+                for (int q = 0; q < 16; ++q) {
+                    const int ml = wm * WM + 32 * i + 8 * (q >> 2) + (q & 3);
+                    const float v = __builtin_amdgcn_ldexpf(acc[i][j][q], -(em[q] + en[j])) + bn[j];
+                    const uint32_t vq = ALL || m0 + ml + 4 * g2 < a.M ? vo : 0xfffffff0u;
+                    const int so = ALL || m0 + ml < a.M ? (int)(ml * ldy * 4) : 0;
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ry, (int)vq, so, 0);
+                }
             }
         }
-    }
+    };
+    if (m0 + BM <= a.M) store(std::true_type{});
+    else store(std::false_type{});
     // outputs of rows that could not be split, over the values stored above by
     // the same lanes: the 32 x 32 tiles that hold any, from the fp32 operands.
     // Lane half g2 takes 4 consecutive columns of its row; MFMA q of a group
@@ -553,9 +613,9 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
             if (!__any(ns_ || a.ex[m] >= kExpSpecial)) continue;
             const float* x = a.x32 + m * a.ldx + 4 * g2;
             const float* w = a.w32 + nc * a.ldw + 4 * g2;
-            F16v c;
+            F16v c, c2;                                      // two chains
 #pragma unroll
-            for (int q = 0; q < 16; ++q) c[q] = 0.f;
+            for (int q = 0; q < 16; ++q) c[q] = c2[q] = 0.f;
             constexpr int KG = 4;                            // groups of 8 columns loaded at a time
             struct Cols { F4v x[KG], w[KG]; } cur, nxt;
             auto load = [&](Cols& d, int k) __attribute__((always_inline)) {
@@ -566,8 +626,10 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
 #pragma unroll
                 for (int u = 0; u < KG; ++u)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
+                    for (int q = 0; q < 4; q += 2) {
                         c = __builtin_amdgcn_mfma_f32_32x32x2f32(d.x[u][q], d.w[u][q], c, 0, 0, 0);
+                        c2 = __builtin_amdgcn_mfma_f32_32x32x2f32(d.x[u][q + 1], d.w[u][q + 1], c2, 0, 0, 0);
+                    }
             };
             const int whole_k = a.vec ? a.K & -(8 * KG) : 0;
             if (whole_k) load(cur, 0);
@@ -585,6 +647,7 @@ __global__ void __launch_bounds__(BM / WM * (BN / WN) * 64, OCC) gemm_split_kern
                 }
                 mma(cur);
             }
+            c += c2;
             const float bias = a.bias ? a.bias[nc] : 0.f;
             int em[16];
             row_exps(mt, em);

@@ -60,6 +60,29 @@ def test_error_not_above_the_fp32_product(M, N, K):
     assert _err(ops.linear_f32(x, w), x, w) <= _err(F.linear(x, w), x, w)
 
 
+@pytest.mark.parametrize("M,N,K", [(999, 3072, 768), (600, 4096, 2500), (512, 2048, 4500), (1000, 8200, 1030)])
+@pytest.mark.parametrize("power", [12, 17, 18, 20, 23, 30])
+def test_spread_rows_keep_the_fp32_error(M, N, K, power):
+    """One value 2^power times the rest of its row against a zero in the other operand: what is left of the row
+    counts.  In every third row of x, and in every third row of W."""
+    x, w, _ = _inputs(M, N, K)
+    x[::3, 5] *= 2.0 ** power
+    w[::3, 9] *= 2.0 ** power
+    x[:, 9] = w[:, 5] = 0
+    assert _err(ops.linear_f32(x, w), x, w) <= _err(F.linear(x, w), x, w)
+
+
+@pytest.mark.parametrize("K", [32, 768, 2500, 4500])
+def test_selecting_rows_are_exact(K):
+    """A row of W (or x) that picks one column gives that column's bits, as an fp32 product does."""
+    x, _, _ = _inputs(200, 1, K)
+    x[::7] = 0
+    pick = torch.randint(0, K, (300,), generator=torch.Generator().manual_seed(K)).cuda()
+    w = F.one_hot(pick, K).float()
+    assert torch.equal(ops.linear_f32(x, w), x[:, pick])
+    assert torch.equal(ops.linear_f32(w, x), x[:, pick].t())
+
+
 def test_split_output_and_strided_weight():
     x, w, b = _inputs(300, 192, 80)
     y0, y1 = ops.linear_f32(x, w, b, n_split=96)
@@ -99,7 +122,7 @@ def test_nothing_is_written_outside_the_outputs(M, N, K):
 
 def test_rows_of_very_different_magnitude():
     """Each row's split is relative to its own largest value: rows 1e-30 to 1e30 keep their relative error, and
-    values far below their row's largest keep an absolute one of 2^-38 of it."""
+    rows whose values spread from 1 to 1e-12 are not split."""
     x, w, _ = _inputs(128, 96, 256)
     s = torch.logspace(-30, 30, 128, device="cuda")[:, None]
     a, b = ops.linear_f32(x * s, w).double() / s.double(), ops.linear_f32(x, w).double()
@@ -185,3 +208,25 @@ def test_one_call_prefill_with_split_projections(d_model, b, l, kw, monkeypatch)
     assert rel(got, ref) < 1e-5
     for a, r in zip(cache.layers, rcache.layers):
         assert rel(a.ssm_state, r.ssm_state) < 1e-5 and rel(a.conv_state, r.conv_state) < 1e-5
+
+
+@pytest.mark.parametrize("d_model", [512, 768, 2048])
+def test_one_call_prefill_with_spread_norm_rows(d_model, monkeypatch):
+    """A norm weight of 2^27 on a column that the in_proj ignores: the rows that the norm writes are not split, and
+    the one call agrees with the per-op path on fp32 products (1e-5, as above; split, the rows would keep 2^-13)."""
+    import mamba_lite.model as mm
+    from mamba_lite.model import MambaConfig, MambaLM
+    torch.manual_seed(d_model)
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=d_model, n_layer=2, vocab_size=300)).eval()
+        ids = torch.randint(0, 300, (1, 2600))
+    with torch.no_grad():
+        for blk in lm.layers:
+            blk.norm.weight[3] = 2.0 ** 27
+            blk.mixer.in_proj.weight[:, 3] = 0
+        assert ops.linear_f32_pays(2600, 4 * d_model, d_model)
+        got, _ = lm.prefill(ids)
+        monkeypatch.setattr(mm, "LONG_PREFILL_NATIVE", False)
+        monkeypatch.setattr(ops, "linear_f32_ok", lambda *a, **k: False)
+        ref, _ = lm.prefill(ids)
+    assert float((got.double() - ref.double()).norm() / ref.double().norm()) < 1e-5
