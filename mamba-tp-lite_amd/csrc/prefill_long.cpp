@@ -28,7 +28,9 @@
 //
 // An in_proj or out_proj with enough rows runs as the split-f16 product of
 // gemm.hip (split_pays), its operands split in blas_ws; the norm before such
-// an in_proj writes the split too (norm_split).
+// an in_proj writes the split too (norm_split) at the widths that takes, and is
+// followed by a split of its own at others (2560 columns, 1024 tokens: 494
+// us per layer, with the library's fp32 in_proj 700).
 //
 // The other GEMMs are hipBLASLt matmuls, fp32 in and out, fp32 compute.  For each
 // shape the heuristic's first algorithm is looked up once per device and
@@ -207,9 +209,9 @@ extern "C" int mtl_prefill_long(const mtl_prefill_long_args* a, const mtl_prefil
     // call may use it between that norm and the in_proj.
     const int64_t xb = (split_bytes(rows, M) + 1023) / 1024 * 1024, in_bytes = xb + split_bytes(2 * D, M);
     const int64_t yb = (split_bytes(rows, D) + 1023) / 1024 * 1024, out_bytes = yb + split_bytes(M, D);
-    bool split_in = !skinny && split_pays(rows, 2 * D, M) && in_bytes <= a->blas_ws_bytes && al16(a->blas_ws) &&
-                    norm_split_ok(a->h, a->out, nullptr, a->xn, M);
-    for (int32_t i = 0; split_in && i < a->n_layers; ++i) split_in = al16(layers[i].norm_w);
+    const bool split_in = !skinny && split_pays(rows, 2 * D, M) && in_bytes <= a->blas_ws_bytes && al16(a->blas_ws);
+    bool norm_splits = split_in && norm_split_ok(a->h, a->out, nullptr, a->xn, M);
+    for (int32_t i = 0; norm_splits && i < a->n_layers; ++i) norm_splits = al16(layers[i].norm_w);
     const bool split_out = !skinny && split_pays(rows, M, D) && out_bytes <= a->blas_ws_bytes && al16(a->blas_ws);
     uint8_t* sws = static_cast<uint8_t*>(a->blas_ws);
     float* x_parts = static_cast<float*>(a->blas_ws);                 // [xs, rows, J]
@@ -226,10 +228,11 @@ extern "C" int mtl_prefill_long(const mtl_prefill_long_args* a, const mtl_prefil
     // norm i's output feeds layer i's in_proj
     auto norm = [&](int32_t i, const float* y) {
         const mtl_prefill_layer& L = layers[i];
-        if (split_in)
+        if (norm_splits)
             return norm_split(a->h, y, y ? a->h : nullptr, L.norm_w, L.eps, a->xn, rows, M, L.W_in, M, 2 * D, sws,
                               sws + xb, st);
-        return mtl_add_rmsnorm(a->h, y, y ? a->h : nullptr, L.norm_w, a->xn, rows, M, L.eps, stream);
+        const int rc = mtl_add_rmsnorm(a->h, y, y ? a->h : nullptr, L.norm_w, a->xn, rows, M, L.eps, stream);
+        return rc || !split_in ? rc : split_rows(a->xn, M, rows, L.W_in, M, 2 * D, M, sws, sws + xb, st);
     };
     int rc = norm(0, nullptr);
     if (rc) return rc;

@@ -189,7 +189,7 @@ def test_route_keeps_autograd_and_autocast():
 def test_one_call_prefill_with_split_projections(d_model, b, l, kw, monkeypatch):
     """A one-call prefill whose in_proj (and, from 1909 rows at d_model 768,
     out_proj) run split, the in_proj's operand written by the norm before it
-    (d_model 1000 is no multiple of 32: library GEMM there), against the
+    (d_model 1000 is no multiple of 32: a split of its own there), against the
     per-op path: the two differ by fp32 rounding only (1e-5, the bound the
     long prefill's other forms are held to)."""
     import mamba_lite.model as mm
@@ -230,3 +230,21 @@ def test_one_call_prefill_with_spread_norm_rows(d_model, monkeypatch):
         monkeypatch.setattr(ops, "linear_f32_ok", lambda *a, **k: False)
         ref, _ = lm.prefill(ids)
     assert float((got.double() - ref.double()).norm() / ref.double().norm()) < 1e-5
+
+
+@pytest.mark.parametrize("d_model,l", [(2560, 1024), (1000, 1100)])
+def test_one_call_in_proj_is_split_past_the_norms_widths(d_model, l):
+    """Where the norm does not write the split (more than 2048 columns, or no multiple of 32), the in_proj of the one
+    call is the split product all the same: the conv state it leaves has that product's bits."""
+    from mamba_lite.model import MambaConfig, MambaLM
+    torch.manual_seed(d_model)
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=d_model, n_layer=1, vocab_size=300)).eval()
+        ids = torch.randint(0, 300, (1, l))
+    assert lm._native_prefill_kind(1, l) == "long"
+    mx, D = lm.layers[0].mixer, 2 * d_model
+    with torch.no_grad():
+        _, cache = lm.prefill(ids)
+        xn = ops.add_rmsnorm(lm.embedding(ids), lm.layers[0].norm.weight, lm.layers[0].norm.eps)
+        xz = ops.linear_f32(xn, mx.in_proj.weight, mx.in_proj.bias)
+    assert torch.equal(cache.layers[0].conv_state, xz[:, -3:, :D].transpose(1, 2))
