@@ -716,14 +716,14 @@ int mtl_decode_step(const mtl_decode_step_args* args, const mtl_decode_layer* la
  *               and conv_w [d_inner, d_conv]; W_x is not read.  Each layer's
  *               conv_state [b, d_inner, d_conv - 1] and ssm_state
  *               [b, d_inner, d_state] are updated in place.
- *   dtype       MTL_BF16: normed_out, norm_f, inp, xn, xc, z, y, every layer
- *               weight and the conv_states hold bf16 values; h, xpart, x_dbl,
- *               parts, sq and the ssm_states stay fp32.  d_model is then at
- *               least 512 and d_inner a multiple of 256, at least 1024.
  * d_model a multiple of 128 (at least 256), d_inner a multiple of 512,
  * d_state <= 16, dt_rank <= 256 with dt_rank + 2 d_state <= 288, d_conv
  * 2..4.  Every layer's pointers, its eps (>= 0, not NaN), the sizes and the
  * alignments the entry points take are checked before the first launch.
+ * mtl_decode_step_batched_bf16: the same with normed_out, norm_f, inp, xn, xc,
+ * z, y, every layer weight and the conv_states holding bf16 values (behind the
+ * same pointers); h, xpart, x_dbl, parts, sq and the ssm_states stay fp32.
+ * d_model is then at least 512 and d_inner a multiple of 256, at least 1024.
  * ---------------------------------------------------------------------- */
 typedef struct {
     float* h;
@@ -744,11 +744,13 @@ typedef struct {
     int32_t batch;
     int32_t d_model, d_inner, d_state, dt_rank, d_conv;
     int32_t fold;              /* 1: residual add + norm folded into the projections */
-    int32_t dtype;             /* MTL_F32 or MTL_BF16 */
+    int32_t reserved;
 } mtl_decode_step_batched_args;
 
 int mtl_decode_step_batched(const mtl_decode_step_batched_args* args, const mtl_decode_layer* layers,
                             mtl_stream_t stream);
+int mtl_decode_step_batched_bf16(const mtl_decode_step_batched_args* args, const mtl_decode_layer* layers,
+                                 mtl_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * mtl_decode_step_persist: the same step -- MambaLM.step (model.py:343-353)

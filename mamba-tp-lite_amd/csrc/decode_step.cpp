@@ -177,10 +177,8 @@ int step_layers(const mtl_decode_step_batched_args* a, const mtl_decode_layer* l
     return MTL_OK;
 }
 
-}  // namespace
-
-extern "C" int mtl_decode_step_batched(const mtl_decode_step_batched_args* a, const mtl_decode_layer* layers,
-                                       mtl_stream_t stream) {
+int step_batched(const mtl_decode_step_batched_args* a, const mtl_decode_layer* layers, bool bf16,
+                 mtl_stream_t stream) {
     using namespace mtl;
     clear_error();
     MTL_REQUIRE(a && layers, "null args or layers");
@@ -190,10 +188,8 @@ extern "C" int mtl_decode_step_batched(const mtl_decode_step_batched_args* a, co
     MTL_REQUIRE(b >= 1 && b <= 32, "batch must be in [1, 32]");
     MTL_REQUIRE(nl >= 1, "n_layers must be >= 1");
     MTL_REQUIRE(M >= 256 && M % 128 == 0 && M <= 65536, "d_model must be a multiple of 128 in [256, 65536]");
-    MTL_REQUIRE((D >= 512 && D % 512 == 0 && D <= 65536) || a->dtype == MTL_BF16,
-                "d_inner must be a multiple of 512 in [512, 65536]");
-    MTL_REQUIRE(a->dtype == MTL_F32 || a->dtype == MTL_BF16, "dtype must be MTL_F32 or MTL_BF16");
-    MTL_REQUIRE(a->dtype == MTL_F32 || (M >= 512 && D >= 1024 && D % 256 == 0 && D <= 65536),
+    MTL_REQUIRE(bf16 || (D >= 512 && D % 512 == 0 && D <= 65536), "d_inner must be a multiple of 512 in [512, 65536]");
+    MTL_REQUIRE(!bf16 || (M >= 512 && D >= 1024 && D % 256 == 0 && D <= 65536),
                 "bf16: d_model must be at least 512 and d_inner a multiple of 256 in [1024, 65536]");
     MTL_REQUIRE(N >= 1 && N <= 16 && R >= 1 && R <= 256, "d_state must be in [1, 16] and dt_rank in [1, 256]");
     MTL_REQUIRE(J <= 288, "dt_rank + 2 d_state must be at most 288");
@@ -225,6 +221,18 @@ extern "C" int mtl_decode_step_batched(const mtl_decode_step_batched_args* a, co
                          "16-byte aligned");
         MTL_REQUIRE(L.eps >= 0.f, at + "eps must be >= 0 (not NaN)");
     }
-    return a->dtype == MTL_BF16 ? step_layers<uint16_t>(a, layers, cpp, rpb_o, rpb_r, stream)
-                                : step_layers<float>(a, layers, cpp, rpb_o, rpb_r, stream);
+    return bf16 ? step_layers<uint16_t>(a, layers, cpp, rpb_o, rpb_r, stream)
+                : step_layers<float>(a, layers, cpp, rpb_o, rpb_r, stream);
+}
+
+}  // namespace
+
+extern "C" int mtl_decode_step_batched(const mtl_decode_step_batched_args* a, const mtl_decode_layer* layers,
+                                       mtl_stream_t stream) {
+    return step_batched(a, layers, false, stream);
+}
+
+extern "C" int mtl_decode_step_batched_bf16(const mtl_decode_step_batched_args* a, const mtl_decode_layer* layers,
+                                            mtl_stream_t stream) {
+    return step_batched(a, layers, true, stream);
 }

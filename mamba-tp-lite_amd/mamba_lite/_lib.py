@@ -121,7 +121,7 @@ class DecodeStepBatchedArgs(ctypes.Structure):
         ("h", _vp), ("normed_out", _vp), ("norm_f", _vp), ("inp", _vp), ("xn", _vp), ("xc", _vp), ("z", _vp),
         ("y", _vp), ("xpart", _vp), ("x_dbl", _vp), ("parts", _vp), ("sq", _vp), ("counters", _vp),
         ("eps_f", ctypes.c_float), ("n_layers", _i32), ("batch", _i32), ("d_model", _i32), ("d_inner", _i32),
-        ("d_state", _i32), ("dt_rank", _i32), ("d_conv", _i32), ("fold", _i32), ("dtype", _i32),
+        ("d_state", _i32), ("dt_rank", _i32), ("d_conv", _i32), ("fold", _i32), ("reserved", _i32),
     ]
 
 
@@ -145,6 +145,8 @@ SIGNATURES = {
     "mtl_decode_step": (ctypes.c_int, [ctypes.POINTER(DecodeStepArgs), ctypes.POINTER(DecodeLayer), _vp]),
     "mtl_decode_step_batched": (ctypes.c_int, [ctypes.POINTER(DecodeStepBatchedArgs), ctypes.POINTER(DecodeLayer),
                                                _vp]),
+    "mtl_decode_step_batched_bf16": (ctypes.c_int, [ctypes.POINTER(DecodeStepBatchedArgs),
+                                                    ctypes.POINTER(DecodeLayer), _vp]),
     "mtl_decode_persist_workspace_bytes": (ctypes.c_size_t, [_i32, _i32, _i32, _i32]),
     "mtl_decode_persist_grid": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "mtl_decode_step_persist": (ctypes.c_int, [ctypes.POINTER(DecodeStepArgs), ctypes.POINTER(DecodeLayer), _vp, _vp,

@@ -681,7 +681,7 @@ def decode_step(layers, ids, emb, norm_f, eps_f, logits, xc, gz, y, xs, xpart, c
 
 
 def decode_step_batched(layers, h, norm_f, eps_f, cfg, fold, dtype=torch.float32):
-    """mtl_decode_step_batched: a batched step of every layer in one call.
+    """mtl_decode_step_batched (_bf16): a batched step of every layer in one call.
     `layers` is a ctypes array of _lib.DecodeLayer (weights with W_xT, and
     this call's cache pointers); h [b, d_model] float32 holds the step's
     embedding rows and is left holding the final residual stream.  Returns
@@ -712,9 +712,11 @@ def decode_step_batched(layers, h, norm_f, eps_f, cfg, fold, dtype=torch.float32
     a.counters = counters.data_ptr() if fold else None
     a.eps_f, a.n_layers, a.batch = float(eps_f), nl, b
     a.d_model, a.d_inner, a.d_state, a.dt_rank, a.d_conv = M, D, cfg.d_state, cfg.dt_rank, cfg.d_conv
-    a.fold, a.dtype = int(bool(fold)), _ACT_DTYPES[dtype]
+    a.fold = int(bool(fold))
+    lib = _lib.load()
+    entry = lib.mtl_decode_step_batched_bf16 if dtype == torch.bfloat16 else lib.mtl_decode_step_batched
     with _dev_guard(h):
-        _lib.check(_lib.load().mtl_decode_step_batched(ctypes.byref(a), layers, _stream(h)), "decode_step_batched")
+        _lib.check(entry(ctypes.byref(a), layers, _stream(h)), "decode_step_batched")
     return ws.view(dtype)[:b * M].view(b, M)     # normed_out: the workspace's first slice
 
 

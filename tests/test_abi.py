@@ -177,6 +177,13 @@ def test_invalid_arguments_are_rejected_without_a_gpu():
     ("mtl_decode_step_batched", dict(fold=1, misaligned_norm=True), b"layer 1: W_in, b_in, conv_state"),
     ("mtl_decode_step_batched", dict(fold=1, d_model=2176), b"at most 128"),
     ("mtl_decode_step_batched", dict(inp_is_h=True), b"must not alias h"),
+    # the field that is reserved is not read, whatever it holds: fp32's rules, in their order
+    ("mtl_decode_step_batched", dict(reserved=7, layer1_eps=-1.0), b"layer 1: eps must be >= 0"),
+    ("mtl_decode_step_batched", dict(reserved=1, layer1_eps=-1.0), b"layer 1: eps must be >= 0"),
+    ("mtl_decode_step_batched", dict(reserved=1, d_inner=1280, d_model=512), b"d_inner must be a multiple of 512"),
+    ("mtl_decode_step_batched_bf16", dict(d_model=384, d_inner=1024), b"bf16: d_model must be at least 512"),
+    ("mtl_decode_step_batched_bf16", dict(d_model=512, d_inner=512), b"bf16: d_model must be at least 512"),
+    ("mtl_decode_step_batched_bf16", dict(d_model=512, d_inner=1280, layer1_eps=-1.0), b"layer 1: eps must be >= 0"),
     ("mtl_decode_step_batched", dict(layer1_eps=-1.0), b"layer 1: eps must be >= 0"),
     # a NaN eps would pass a "not below zero" test and then fail in the folded
     # in_proj of layer 1, after layer 0 has stepped its caches
@@ -356,12 +363,13 @@ def test_entry_points_validate_sizes_on_the_host(case):
                 L.W_xT = None
         rc = lib.mtl_decode_step_persist(ctypes.byref(args), layers, ctypes.c_void_p(256), ctypes.c_void_p(256),
                                          a["ws_bytes"], a["blocking"], None)
-    elif name == "mtl_decode_step_batched":
+    elif name in ("mtl_decode_step_batched", "mtl_decode_step_batched_bf16"):
         a = dict(batch=8, n_layers=2, d_model=256, d_inner=512, d_state=16, dt_rank=16, d_conv=4, fold=0,
                  null_ws=False, null_fold=False, xn_is_h=False, null_layer=False, misaligned_layer=False,
-                 misaligned_norm=False, inp_is_h=False, layer1_eps=None)
+                 misaligned_norm=False, inp_is_h=False, layer1_eps=None, reserved=0)
         a.update(over)
         args = _lib.DecodeStepBatchedArgs()
+        args.reserved = a["reserved"]
         for k, (f, *_) in enumerate(_lib.DecodeStepBatchedArgs._fields_[:13]):
             # distinct 16-byte aligned placeholders, never dereferenced
             setattr(args, f, 16 * (k + 1))
@@ -389,7 +397,7 @@ def test_entry_points_validate_sizes_on_the_host(case):
                 L.norm_w = 20
             if a["layer1_eps"] is not None and i == 1:
                 L.eps = a["layer1_eps"]
-        rc = lib.mtl_decode_step_batched(ctypes.byref(args), layers, None)
+        rc = getattr(lib, name)(ctypes.byref(args), layers, None)
     elif name == "mtl_in_proj_conv_xproj":
         a = dict(batch=8, d_model=256, d_inner=64, cpp=16, d_conv=4, J=40)
         a.update(over)
