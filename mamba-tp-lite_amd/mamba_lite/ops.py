@@ -916,9 +916,16 @@ def linear_f32_ok(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
     return _plain_forward(x, W) if bias is None else _plain_forward(x, W, bias)
 
 
+def _no_function_mode() -> bool:
+    """No TorchFunctionMode that would see F.linear (a default device only changes factory calls)."""
+    return all(type(torch._C._get_function_stack_at(i)) is torch.utils._device.DeviceContext
+               for i in range(torch._C._len_torch_function_stack()))
+
+
 def plain_call() -> bool:
-    """No autocast, functorch or forward-mode transform, tracing or dispatch mode that a raw launch would bypass."""
-    return not torch.is_autocast_enabled("cuda") and torch.autograd.forward_ad._current_level < 0 and \
+    """No autocast, functorch or forward-mode transform, tracing, function or dispatch mode that a raw launch would
+    bypass."""
+    return _no_function_mode() and not torch.is_autocast_enabled("cuda") and torch.autograd.forward_ad._current_level < 0 and \
         torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0 and \
         not torch.jit.is_tracing() and not torch.compiler.is_compiling()
 

@@ -407,3 +407,21 @@ def test_from_pretrained_loads_in_proj_bias_of_a_bias_snapshot(tmp_path):
     for k, v in sd.items():
         assert torch.equal(got[k], torch.from_numpy(v)), k
     assert lm.layers[1].mixer.in_proj.bias is not None and lm.layers[1].mixer.out_proj.bias is not None
+
+
+def test_a_torch_function_mode_is_no_plain_call():
+    """A mode that sees F.linear keeps the raw routes off; a default device, which changes factory calls only, does
+    not."""
+    import torch
+    from mamba_lite import ops
+
+    class Seen(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert ops.plain_call()
+    with torch.device("cpu"):
+        assert ops.plain_call()
+        with Seen():
+            assert not ops.plain_call()
+    assert ops.plain_call()
