@@ -746,8 +746,11 @@ class MambaLM(nn.Module):
             normed = ops.prefill_short(h, arr, self.norm_f.weight, self.norm_f.eps, D, N, cfg.dt_rank, K)
         else:
             skinny = LONG_PREFILL_SKINNY_ROWS if cfg.d_model <= LONG_PREFILL_SKINNY_MAX_D_MODEL else 0
-            normed = ops.prefill_long(h, arr, self.norm_f.weight, self.norm_f.eps, D, N, cfg.dt_rank, K,
-                                      skinny_rows=skinny)
+            try:
+                normed = ops.prefill_long(h, arr, self.norm_f.weight, self.norm_f.eps, D, N, cfg.dt_rank, K,
+                                          skinny_rows=skinny)
+            except torch.OutOfMemoryError:      # its workspace, before any launch: op by op takes less at a time
+                return None
         return self.lm_head(normed), (out_cache if out_cache is not None else MambaCache(new_layers))
 
     def step(self, input_ids: torch.Tensor, cache: MambaCache):

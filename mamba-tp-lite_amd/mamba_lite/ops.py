@@ -16,6 +16,7 @@ import contextlib
 import ctypes
 
 import torch
+import torch.nn.functional as F
 
 from . import _lib
 
@@ -190,7 +191,12 @@ def selective_scan(u, delta, A, B, C, D=None, z=None, delta_bias=None, h0=None, 
     p.algo = SCAN_ALGOS[algo]
     lib = _lib.load()
     nb = lib.mtl_selective_scan_ws_bytes(b, Dm, N, L) if p.algo == 0 else 0
-    ws = torch.empty(nb // 4, device=u.device, dtype=torch.float32) if nb else None
+    ws = None
+    if nb:
+        try:
+            ws = torch.empty(nb // 4, device=u.device, dtype=torch.float32)
+        except torch.OutOfMemoryError:
+            nb = 0                  # no room for the segments' summaries: the unsegmented scan
     with _dev_guard(u):
         _lib.check(lib.mtl_selective_scan_fwd_ws(ctypes.byref(p), _ptr(ws), nb, _stream(u)), "selective_scan_fwd")
     return y, h_out
@@ -631,18 +637,24 @@ def prefill_long(h, layers, norm_f, eps_f, d_inner, d_state, dt_rank, d_conv, sk
     lib = _lib.load()
     blas_ws = max([PREFILL_LONG_BLAS_WS] + [lib.mtl_linear_f32_ws_bytes(rows, n, k)
                                             for n, k in ((2 * d_inner, M), (M, d_inner)) if linear_f32_pays(rows, n, k)])
-    sizes = [rows * M, rows * 2 * d_inner, rows * d_inner, rows * J, rows * d_inner, rows * d_inner, rows * M,
-             -(-blas_ws // 4)]
     offs, n = [], 0
-    for sz in sizes:
+    for sz in (rows * M, rows * 2 * d_inner, rows * d_inner, rows * J, rows * d_inner, rows * d_inner, rows * M, rows * M):
         offs.append(n)
         n += -(-sz // 64) * 64
-    ws = torch.empty(n + rows * M, device=h.device, dtype=torch.float32)
-    normed = ws[n:].view(b, l, M)
+    alloc = lambda: torch.empty(n + -(-blas_ws // 4), device=h.device, dtype=torch.float32)
+    try:
+        ws = alloc()
+    except torch.OutOfMemoryError:
+        if blas_ws == PREFILL_LONG_BLAS_WS:
+            raise
+        blas_ws = PREFILL_LONG_BLAS_WS      # no room for the split operands: those products on the library
+        ws = alloc()
+    *offs, at_normed = offs
+    normed = ws[at_normed:at_normed + rows * M].view(b, l, M)
     base = ws.data_ptr()
     a = _lib.PrefillLongArgs()
     a.h = h.data_ptr()
-    a.xn, a.xz, a.u, a.x_dbl, a.dt, a.y, a.out, a.blas_ws = [base + 4 * o for o in offs]
+    a.xn, a.xz, a.u, a.x_dbl, a.dt, a.y, a.out, a.blas_ws = [base + 4 * o for o in (*offs, n)]
     a.blas_ws_bytes = blas_ws
     a.norm_f, a.normed_out, a.eps_f = norm_f.data_ptr(), normed.data_ptr(), float(eps_f)
     a.d_conv, a.n_layers, a.skinny_rows = d_conv, len(layers), int(skinny_rows)
@@ -980,10 +992,19 @@ def linear_f32(x, W, bias=None, n_split=None):
     a = _lib.LinearF32Args()
     a.M, a.N, a.K, a.ldx, a.ldw = M, N, K, K, W.stride(0)
     nb = lib.mtl_linear_f32_ws_bytes(M, N, K)
-    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=x.device)
     n0 = N if n_split is None else n_split
-    y0 = torch.empty(*lead, n0, dtype=torch.float32, device=x.device)
-    y1 = None if n_split is None else torch.empty(*lead, N - n0, dtype=torch.float32, device=x.device)
+    ws = y0 = y1 = None
+    try:
+        ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=x.device)
+        y0 = torch.empty(*lead, n0, dtype=torch.float32, device=x.device)
+        if n_split is not None:
+            y1 = torch.empty(*lead, N - n0, dtype=torch.float32, device=x.device)
+    except torch.OutOfMemoryError:
+        # no room for the split operands: the library's product needs none
+        del ws, y0, y1
+        if n_split is None:
+            return F.linear(x, W, bias)
+        return tuple(F.linear(x, W[s], None if bias is None else bias[s]) for s in (slice(n0), slice(n0, N)))
     a.x, a.W, a.bias, a.y0, a.y1 = _ptr(x), _ptr(W), _ptr(bias), _ptr(y0), _ptr(y1)
     a.ws, a.ws_bytes, a.ldy0, a.ldy1, a.n_split = _ptr(ws), nb, n0, N - n0, n0
     with _dev_guard(x):
