@@ -234,11 +234,12 @@ def _linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     return ops.linear_f32(x, w, bias) if ops.linear_f32_ok(x, w, bias) else F.linear(x, w, bias)
 
 
-def _plain_modules(mod) -> bool:
-    """No hook and no replaced forward on mod or a module in it, all of which a raw launch would skip."""
+def _plain_modules(mod, types) -> bool:
+    """mod and the modules in it are of `types` (no adapter, parametrization or other subclass), without hooks or a
+    replaced forward, all of which a raw launch would skip."""
     d = mod.__dict__
-    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d) and \
-        all(m is None or _plain_modules(m) for m in d["_modules"].values())
+    return type(mod) in types and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d) and \
+        all(m is None or _plain_modules(m, types) for m in d["_modules"].values())
 
 
 def _no_global_hooks() -> bool:
@@ -248,7 +249,7 @@ def _no_global_hooks() -> bool:
 
 def _linear_mod(mod, x: torch.Tensor) -> torch.Tensor:
     """mod(x) of a projection; a plain nn.Linear without hooks may take ops.linear_f32."""
-    if type(mod) is nn.Linear and _plain_modules(mod) and _no_global_hooks() and \
+    if _plain_modules(mod, (nn.Linear,)) and _no_global_hooks() and \
             ops.linear_f32_ok(x, mod.weight, mod.bias):
         return ops.linear_f32(x, mod.weight, mod.bias)
     return mod(x)
@@ -596,6 +597,10 @@ class MambaBlock(nn.Module):
         return x_t + self.mixer.step(self.norm(x_t), cache)
 
 
+# what a MambaLM's layers are made of, and nothing else of, where _plain_stack holds
+_STACK_MODULES = frozenset((nn.ModuleList, MambaBlock, MambaMixer, RMSNorm, nn.Linear, nn.Conv1d))
+
+
 class MambaLM(nn.Module):
     """Embedding -> n_layer MambaBlocks -> RMSNorm -> lm_head tied to the
     embedding (reference model.py:314-365).  Between blocks the residual add
@@ -682,9 +687,10 @@ class MambaLM(nn.Module):
         return arr
 
     def _plain_stack(self) -> bool:
-        """Whether the blocks are nothing but their launches: no hooks or
+        """Whether the blocks are nothing but their launches: no module of
+        another class in them (an adapter, a parametrization), no hooks or
         replaced forwards on a module, no autocast, transform or tracing."""
-        return ops.plain_call() and _no_global_hooks() and _plain_modules(self.layers)
+        return ops.plain_call() and _no_global_hooks() and _plain_modules(self.layers, _STACK_MODULES)
 
     def _native_prefill_kind(self, b, l):
         """'short' (mtl_prefill_short), 'long' (mtl_prefill_long) or None for

@@ -88,3 +88,57 @@ def test_a_hooked_stack_keeps_the_per_op_path(dtype, b, l):
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert not one_call()
     assert one_call()
+
+
+class _Negating(torch.nn.Linear):
+    def forward(self, x):
+        return -super().forward(x)
+
+
+class _Adapter(torch.nn.Module):
+    """A projection inside another module, which shows its weight and bias."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    weight = property(lambda self: self.inner.weight)
+    bias = property(lambda self: self.inner.bias)
+
+    def forward(self, x):
+        return -self.inner(x)
+
+
+class _Negated(torch.nn.Module):
+    def forward(self, w):
+        return -w
+
+
+@pytest.mark.parametrize("kind,dtype,b,l", [("subclass", torch.bfloat16, 3, 1), ("subclass", torch.float32, 2, 1024),
+                                            ("adapter", torch.float32, 2, 1024),
+                                            ("parametrization", torch.float32, 2, 1024)])
+def test_a_replaced_projection_is_called(kind, dtype, b, l):
+    """An out_proj of another class is called as a module, not read past, by the bf16 step and by an fp32 prompt of
+    more than 2^21 token-channels: here each negates what nn.Linear gives."""
+    torch.manual_seed(3)
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=640, n_layer=1, vocab_size=300)).eval().to(dtype)
+        ids = torch.randint(0, 300, (b, l))
+    mx = lm.layers[0].mixer
+
+    def logits():
+        with torch.no_grad():
+            cache = MambaCache.allocate(lm.cfg, b, "cuda", dtype)
+            return (lm.step(ids, cache) if l == 1 else lm.prefill(ids)[0]).double()
+
+    with torch.no_grad():
+        mx.out_proj.weight.mul_(-50)            # the block outweighs the embedding it is added to
+        want = logits()
+        mx.out_proj.weight.neg_()
+    if kind == "subclass":
+        mx.out_proj.__class__ = _Negating
+    elif kind == "adapter":
+        mx.out_proj = _Adapter(mx.out_proj)
+    else:
+        torch.nn.utils.parametrize.register_parametrization(mx.out_proj, "weight", _Negated())
+    assert float((logits() - want).norm() / want.norm()) < (1e-2 if dtype == torch.bfloat16 else 1e-5)
