@@ -878,6 +878,10 @@ class MambaLM(nn.Module):
         if not (1 <= b <= ops.IN_CONV_MAX_ROWS and fits and dm % 128 == 0 and N <= 16 and R <= 256 and 2 <= K <= 4 and R + 2 * N <= 288):
             return None
         dev = x.device
+        nf = self.norm_f.weight           # (not in the template: norm_f may be cast or replaced between steps)
+        if act != torch.float32 and (nf.dtype != act or nf.device != dev or not nf.is_contiguous() or
+                                     tuple(nf.shape) != (dm,)):
+            return None
         lt = self._layer_tensors() if lt is None else lt
         sig = (dev, dm, act, tuple(0 if t is None else t.data_ptr() for ts in lt for t in ts),
                tuple(ts[_LT_XPROJ]._version for ts in lt), self._norm_eps())
@@ -914,8 +918,6 @@ class MambaLM(nn.Module):
         ok = lambda t, shape: t.device == dev and t.dtype == act and t.is_contiguous() and tuple(t.shape) == shape
         opt = lambda t, shape: t is None or ok(t, shape)
         tmpl = (_lib.DecodeLayer * len(lt))()
-        if not ok(self.norm_f.weight, (dm,)) and act != torch.float32:
-            return None
         for i, (ts, L) in enumerate(zip(lt, tmpl)):
             if not (ok(ts[_LT_NORM], (dm,)) and ok(ts[_LT_W_IN], (2 * D, dm)) and opt(ts[_LT_B_IN], (2 * D,))
                     and ok(ts[_LT_CONV_W], (D, 1, K)) and opt(ts[_LT_CONV_B], (D,))

@@ -90,6 +90,26 @@ def test_a_hooked_stack_keeps_the_per_op_path(dtype, b, l):
     assert one_call()
 
 
+def test_a_norm_f_cast_between_steps():
+    """norm_f kept in float32 on a bf16 model, before the first step or after one: the per-op path, as if it had been
+    so from the start."""
+    torch.manual_seed(5)
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=640, n_layer=2, vocab_size=300)).eval().to(torch.bfloat16)
+    ids = torch.zeros(3, 1, dtype=torch.long, device="cuda")
+
+    def step():
+        with torch.no_grad():
+            return lm.step(ids, MambaCache.allocate(lm.cfg, 3, "cuda", torch.bfloat16)).double()
+
+    before = step()
+    lm.norm_f.float()
+    after = step()
+    lm._batched_tmpl = None
+    assert torch.equal(after, step())
+    assert float((after - before).norm() / before.norm()) < 1e-2
+
+
 class _Negating(torch.nn.Linear):
     def forward(self, x):
         return -super().forward(x)
