@@ -236,10 +236,10 @@ def _linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
 
 def _plain_modules(mod, types) -> bool:
     """mod and the modules in it are of `types` (no adapter, parametrization or other subclass), without hooks or a
-    replaced forward, all of which a raw launch would skip."""
+    replaced forward, and their parameters no tensor subclass, all of which a raw launch would skip."""
     d = mod.__dict__
     return type(mod) in types and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d) and \
-        all(m is None or _plain_modules(m, types) for m in d["_modules"].values())
+        all(p is None or type(p) in ops.PLAIN_TENSORS for p in d["_parameters"].values()) and all(m is None or _plain_modules(m, types) for m in d["_modules"].values())
 
 
 def _no_global_hooks() -> bool:

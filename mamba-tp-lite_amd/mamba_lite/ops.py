@@ -106,9 +106,15 @@ def _param_code(code: int, bf16_params: bool) -> int:
     return _lib.MTL_BF16_PARAMS if bf16_params else code
 
 
+# what holds its values where data_ptr() says, and means nothing else to torch
+PLAIN_TENSORS = frozenset((torch.Tensor, torch.nn.Parameter))
+
+
 def bf16_params_ok(*ts) -> bool:
-    """Whether every (non-None) parameter can be handed over as bf16: contiguous, 16-byte aligned bfloat16."""
-    return all(t is None or (t.dtype == torch.bfloat16 and t.is_contiguous()) for t in ts) and aligned16(*ts)
+    """Whether every (non-None) parameter can be handed over as bf16: a contiguous, 16-byte aligned bfloat16 tensor of
+    no subclass (whose values .float() would read)."""
+    return all(t is None or (type(t) in PLAIN_TENSORS and t.dtype == torch.bfloat16 and t.is_contiguous())
+               for t in ts) and aligned16(*ts)
 
 
 def _bdl_layout_ok(*ts):
@@ -944,7 +950,7 @@ def plain_call() -> bool:
 
 def _plain_forward(*ts) -> bool:
     """Nothing of torch's between these tensors and a raw launch: no autograd, transform or tensor subclass."""
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts) and plain_call() and \
+    return all(type(t) in PLAIN_TENSORS for t in ts) and plain_call() and \
         not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
 
 

@@ -162,3 +162,49 @@ def test_a_replaced_projection_is_called(kind, dtype, b, l):
     else:
         torch.nn.utils.parametrize.register_parametrization(mx.out_proj, "weight", _Negated())
     assert float((logits() - want).norm() / want.norm()) < (1e-2 if dtype == torch.bfloat16 else 1e-5)
+
+
+class _Halved(torch.Tensor):
+    """A weight whose values are half of those it holds, as a quantized weight's are not the ones in memory."""
+
+    @staticmethod
+    def __new__(cls, held):
+        return torch.Tensor._make_wrapper_subclass(cls, held.shape, strides=held.stride(), dtype=held.dtype,
+                                                   device=held.device)
+
+    def __init__(self, held):
+        self.held = held
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        real = lambda t: t.held * 0.5 if isinstance(t, cls) else t
+        if func is torch.ops.aten.detach.default:
+            return cls(args[0].held)
+        return func(*torch.utils._pytree.tree_map(real, args), **(kwargs or {}))
+
+
+@pytest.mark.parametrize("dtype,b,l", [(torch.bfloat16, 3, 1), (torch.float32, 2, 1024), (torch.bfloat16, 2, 40)])
+def test_a_subclass_weight_is_read_through_torch(dtype, b, l):
+    """An out_proj weight (a bf16 prompt: dt_proj's bias) of a tensor subclass keeps torch's product, or float copy, of
+    it: the bf16 step, an fp32 prompt of more than 2^21 token-channels, the bf16 scan's parameters."""
+    torch.manual_seed(3)
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=640, n_layer=1, vocab_size=300)).eval().to(dtype)
+        ids = torch.randint(0, 300, (b, l))
+    mx = lm.layers[0].mixer
+    mod, name = (mx.dt_proj, "bias") if l == 40 else (mx.out_proj, "weight")
+
+    def logits():
+        with torch.no_grad():
+            cache = MambaCache.allocate(lm.cfg, b, "cuda", dtype)
+            return (lm.step(ids, cache) if l == 1 else lm.prefill(ids)[0]).double()
+
+    with torch.no_grad():
+        mx.out_proj.weight.mul_(50)
+        mx.dt_proj.bias.normal_(0, 4)
+        held = getattr(mod, name).detach().clone()
+        setattr(mod, name, torch.nn.Parameter(held * 0.5))
+        want = logits()
+        setattr(mod, name, torch.nn.Parameter(_Halved(held), requires_grad=False))
+        assert type(getattr(mod, name)) is _Halved
+    assert float((logits() - want).norm() / want.norm()) < (1e-2 if dtype == torch.bfloat16 else 1e-5)
