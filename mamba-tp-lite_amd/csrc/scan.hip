@@ -320,7 +320,10 @@ __global__ void __launch_bounds__(NW * 64, CM ? 3 : 4) scan_fwd_kernel(const Sca
             for (int k = 0; k < SPW; ++k) {
                 const int n = wave * SPW + k;
                 const float e = a.seg_h[row * N + min(n, N - 1)];
-                h[k] = fmaf(__builtin_amdgcn_exp2f(sd * a2[k]), h[k], n < N ? e : 0.f);
+                // step by step a zero state stays zero and an infinite one infinite, also
+                // where the product of the decays is out of range
+                const bool keep = h[k] == 0.f || fabsf(h[k]) == INFINITY;
+                h[k] = fmaf(keep ? 1.f : __builtin_amdgcn_exp2f(sd * a2[k]), h[k], n < N ? e : 0.f);
             }
         }
     }

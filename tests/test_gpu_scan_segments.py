@@ -77,6 +77,27 @@ def test_a_prompt_that_continues_its_cache_in_place(d_model, b, l):
         assert torch.equal(p.ssm_state, q.ssm_state) and torch.equal(p.conv_state, q.conv_state)
 
 
+@pytest.mark.parametrize("b,D,L,N", SHAPES)
+@pytest.mark.parametrize("cm", [True, False])
+def test_zero_and_infinite_states_as_step_by_step(b, D, L, N, cm):
+    """The product of a segment's decays overflows (A > 0) or underflows (A = -16) where each step's is in range: a
+    state that is zero until the last steps stays zero, an infinite one stays infinite."""
+    c = _case(b, D, L, N, torch.float32, cm)
+    zero = torch.zeros_like(c["u"])
+    zero[..., -5:] = c["u"][..., -5:]
+    h0 = c["h0"].clone()
+    h0[:, ::2] = float("inf")
+    h0[:, 1::4] = 0
+    for A, u, start in ((2.0, zero, None), (2.0, zero, torch.zeros_like(h0)), (-16.0, c["u"], h0)):
+        run = lambda **kw: ops.selective_scan(u, torch.full_like(c["delta"], 1.0 if A > 0 else 0.2),
+                                              torch.full_like(c["A"], A), c["B"], c["C"], h0=start,
+                                              delta_softplus=False, **kw)
+        for got, ref in zip(run(), run(algo="tiled")):
+            assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+            ok = torch.isfinite(ref)
+            assert bool(ok.any()) and float((got[ok] - ref[ok]).norm()) <= 1e-6 * float(ref[ok].norm())
+
+
 def test_outside_the_rule_nothing_changes():
     ws = _lib.load().mtl_selective_scan_ws_bytes
     assert ws(1, 1536, 16, 1024) == 0 and ws(32, 1536, 16, 1024) == 0 and ws(1, 4096, 16, 300) == 0
