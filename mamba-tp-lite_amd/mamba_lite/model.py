@@ -597,6 +597,9 @@ class MambaBlock(nn.Module):
         return x_t + self.mixer.step(self.norm(x_t), cache)
 
 
+_CALL_PLANS = frozenset(("_short_plan", "_batched_tmpl", "_plan", "_step_tmpl", "_fused_memo", "_persist_tab",
+                         "_persist_ws"))
+
 # what a MambaLM's layers are made of, and nothing else of, where _plain_stack holds
 _STACK_MODULES = frozenset((nn.ModuleList, MambaBlock, MambaMixer, RMSNorm, nn.Linear, nn.Conv1d))
 
@@ -612,6 +615,11 @@ class MambaLM(nn.Module):
         self.embedding = nn.Embedding(cfg.vocab_size, cfg.d_model)
         self.layers = nn.ModuleList([MambaBlock(cfg, i) for i in range(cfg.n_layer)])
         self.norm_f = RMSNorm(cfg.d_model, eps=cfg.layer_norm_epsilon)
+
+    def __getstate__(self):
+        """Without the call plans: they hold addresses of this object's
+        tensors, and a copy or a reloaded model makes its own."""
+        return {k: v for k, v in self.__dict__.items() if k not in _CALL_PLANS}
 
     def lm_head(self, x: torch.Tensor) -> torch.Tensor:
         w = self.embedding.weight

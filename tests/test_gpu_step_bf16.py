@@ -2,6 +2,9 @@
 history in bf16; fp32 residual, SSM state and partial sums): MambaLM.step
 (model.py:343-353) at 1-32 rows against the float64 oracle and the per-op
 step, and captured."""
+import copy
+import io
+
 import numpy as np
 import pytest
 import torch
@@ -108,6 +111,32 @@ def test_a_norm_f_cast_between_steps():
     lm._batched_tmpl = None
     assert torch.equal(after, step())
     assert float((after - before).norm() / before.norm()) < 1e-2
+
+
+@pytest.mark.parametrize("dtype,b,l", [(torch.bfloat16, 3, 1), (torch.float32, 2, 1024), (torch.float32, 1, 1),
+                                       (torch.float32, 1, 20)])
+def test_a_model_is_copied_and_saved_after_its_calls(dtype, b, l):
+    """copy.deepcopy and torch.save of a model that has stepped or prefilled: its call plans stay behind, and the copy
+    gives the same bits from its own weights."""
+    torch.manual_seed(6)
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=640, n_layer=2, vocab_size=300)).eval().to(dtype)
+        ids = torch.randint(0, 300, (b, l))
+
+    def logits(m):
+        with torch.no_grad():
+            return m.step(ids, MambaCache.allocate(m.cfg, b, "cuda", dtype)) if l == 1 else m.prefill(ids)[0]
+
+    want = logits(lm)
+    twin = copy.deepcopy(lm)
+    buf = io.BytesIO()
+    torch.save(lm, buf)
+    buf.seek(0)
+    with torch.no_grad():
+        lm.layers[0].mixer.out_proj.weight.zero_()
+    assert torch.equal(logits(twin), want)
+    assert torch.equal(logits(torch.load(buf, weights_only=False)), want)
+    assert not torch.equal(logits(lm), want)
 
 
 class _Negating(torch.nn.Linear):
