@@ -891,6 +891,9 @@ class MambaLM(nn.Module):
                                      tuple(nf.shape) != (dm,)):
             return None
         lt = self._layer_tensors() if lt is None else lt
+        # (inference tensors have no version that W_xT could follow: bf16 steps need none op by op)
+        if act != torch.float32 and any(ts[_LT_XPROJ].is_inference() for ts in lt):
+            return None
         sig = (dev, dm, act, tuple(0 if t is None else t.data_ptr() for ts in lt for t in ts),
                tuple(ts[_LT_XPROJ]._version for ts in lt), self._norm_eps())
         cached = getattr(self, "_batched_tmpl", None)

@@ -139,6 +139,23 @@ def test_a_model_is_copied_and_saved_after_its_calls(dtype, b, l):
     assert not torch.equal(logits(lm), want)
 
 
+@pytest.mark.parametrize("l", [1, 40])
+def test_a_model_made_in_inference_mode(l):
+    """Its parameters are inference tensors, which have no version counter: it steps and prefills, and a
+    weight changed in place counts."""
+    torch.manual_seed(8)
+    with torch.inference_mode(), torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=640, n_layer=2, vocab_size=300)).eval().to(torch.bfloat16)
+    ids = torch.zeros(3, l, dtype=torch.long, device="cuda")
+    with torch.inference_mode():
+        cache = MambaCache.allocate(lm.cfg, 3, "cuda", torch.bfloat16)
+        got = lm.step(ids, cache) if l == 1 else lm.prefill(ids)[0]
+        assert bool(torch.isfinite(got).all())
+        lm.layers[0].mixer.x_proj.weight.mul_(3)
+        cache = MambaCache.allocate(lm.cfg, 3, "cuda", torch.bfloat16)
+        assert not torch.equal(lm.step(ids, cache) if l == 1 else lm.prefill(ids)[0], got)
+
+
 class _Negating(torch.nn.Linear):
     def forward(self, x):
         return -super().forward(x)
