@@ -250,38 +250,32 @@ def test_one_call_in_proj_is_split_past_the_norms_widths(d_model, l):
     assert torch.equal(cache.layers[0].conv_state, xz[:, -3:, :D].transpose(1, 2))
 
 
-class _Limit:
-    """At most `extra` bytes of the GPU past what is allocated now."""
+def _no_more_than(mp, most):
+    """torch.empty of more than `most` bytes is out of memory, as far as Python's calls go."""
+    real = torch.empty
 
-    def __init__(self, extra):
-        self.extra = extra
-
-    def __enter__(self):
-        torch.cuda.synchronize()
-        torch.cuda.empty_cache()
-        total = torch.cuda.get_device_properties(0).total_memory
-        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + self.extra) / total)
-
-    def __exit__(self, *_):
-        torch.cuda.set_per_process_memory_fraction(1.0)
+    def empty(*size, **kw):
+        t = real(*size, **{**kw, "device": "meta"})
+        if t.numel() * t.element_size() > most:
+            raise torch.OutOfMemoryError(f"{t.numel() * t.element_size()} bytes")
+        return real(*size, **kw)
+    mp.setattr(torch, "empty", empty)
 
 
-def test_without_room_for_the_split_operands_the_library_takes_the_product():
-    x, w, b = _inputs(8192, 2048, 4096)
-    ref = F.linear(x, w, b)                      # (the library's own workspace is there from here on)
-    with _Limit(96 << 20):                       # the output and some; the operands take 160 MB
-        with pytest.raises(torch.OutOfMemoryError):
-            torch.empty(160 << 20, dtype=torch.uint8, device="cuda")
-        got = ops.linear_f32(x, w, b)
-    assert torch.equal(got, ref)
-    with _Limit(96 << 20):
-        halves = ops.linear_f32(x, w, b, n_split=1024)
+def test_without_room_for_the_split_operands_the_library_takes_the_product(monkeypatch):
+    x, w, b = _inputs(1024, 2048, 4096)
+    ref = F.linear(x, w, b)
+    _no_more_than(monkeypatch, 16 << 20)         # the output's 8 MB; the operands take 48 MB
+    with pytest.raises(torch.OutOfMemoryError):
+        torch.empty(x.numel() + w.numel(), device="cuda")
+    assert torch.equal(ops.linear_f32(x, w, b), ref)
+    halves = ops.linear_f32(x, w, b, n_split=1024)
     assert float((torch.cat(halves, 1) - ref).norm() / ref.norm()) < 2e-6
 
 
 def test_without_room_for_its_workspace_a_prompt_runs_as_it_fits(monkeypatch):
-    """A prompt of over 2^21 token-channels within the memory that the per-op path takes on library products, and one
-    with room for the one call but not for the split operands."""
+    """A prompt of over 2^21 token-channels with no room for the one call's workspace runs op by op; with room for that
+    but not for the split operands, in one call on library products."""
     import mamba_lite.model as mm
     from mamba_lite.model import MambaConfig, MambaLM
     torch.manual_seed(4)
@@ -291,23 +285,30 @@ def test_without_room_for_its_workspace_a_prompt_runs_as_it_fits(monkeypatch):
     calls = []
     real = ops.prefill_long
     monkeypatch.setattr(ops, "prefill_long", lambda *a, **k: (calls.append(1), real(*a, **k), calls.append(2))[1])
+    rows, M, D = 5000, 768, 1536
+    one_call = 4 * rows * (4 * M + 5 * D + 80) + (33 << 20)
     with torch.no_grad():
-        full, _ = lm.prefill(ids)
-        assert calls == [1, 2]
         with monkeypatch.context() as mp:
             mp.setattr(mm, "LONG_PREFILL_NATIVE", False)
             mp.setattr(ops, "linear_f32_ok", lambda *a, **k: False)
-            lm.prefill(ids)
-            torch.cuda.reset_peak_memory_stats()
             ref, _ = lm.prefill(ids)
-            peak = torch.cuda.max_memory_allocated() - torch.cuda.memory_allocated()
-        rows, M, D = 5000, 768, 1536
-        one_call = 4 * rows * (4 * M + 5 * D + 80) + (32 << 20)
-        assert peak + (16 << 20) < one_call
-        for extra, path in ((peak + (16 << 20), [1]), (one_call + (40 << 20), [1, 2])):
+        for most, path in ((1 << 40, [1, 2]), (one_call, [1, 2]), (one_call - (40 << 20), [1])):
             calls.clear()
-            with _Limit(extra):
+            with monkeypatch.context() as mp:
+                _no_more_than(mp, most)
                 got, _ = lm.prefill(ids)
             assert calls == path
             assert float((got - ref).norm() / ref.norm()) < 1e-5
-    assert float((full - ref).norm() / ref.norm()) < 1e-5
+
+
+def test_without_room_for_the_summaries_a_scan_is_not_segmented(monkeypatch):
+    b, D, L, N = 1, 4096, 1024, 16
+    u, z = (torch.randn(b, D, L, device="cuda") for _ in range(2))
+    B, C = (torch.randn(b, N, L, device="cuda") for _ in range(2))
+    A = -torch.arange(1, N + 1, device="cuda", dtype=torch.float32).repeat(D, 1).contiguous()
+    y, h = torch.empty_like(u), torch.empty(b, D, N, device="cuda")
+    run = lambda **kw: ops.selective_scan(u, u, A, B, C, z=z, **kw)
+    ref = run(algo="chunked")
+    _no_more_than(monkeypatch, 1 << 10)
+    got = run(y=y, h_out=h)
+    assert all(torch.equal(p, q) for p, q in zip(got, ref))

@@ -29,7 +29,7 @@ BF16_SHAPES = [(512, 2, 1, 4, False), (640, 2, 3, 4, True), (896, 2, 16, 3, Fals
 def test_bf16_one_call_step_matches_oracle_and_per_op(dm, expand, b, d_conv, bias, monkeypatch):
     """A bfloat16 model's one-call step against the float64 oracle on the same
     bf16-rounded weights and caches (1e-2, the bf16 gate), and no further
-    from it than twice the per-op step; graph replays equal eager."""
+    from it than the per-op step; graph replays equal eager."""
     import mamba_lite.model as mm
     torch.manual_seed(dm + b)
     cfg = MambaConfig(d_model=dm, n_layer=2, vocab_size=200, d_state=16, d_conv=d_conv, expand=expand, bias=bias)
@@ -62,7 +62,7 @@ def test_bf16_one_call_step_matches_oracle_and_per_op(dm, expand, b, d_conv, bia
             ref = om.lm_step(W, ids.cpu().numpy(), oc, dtype=np.float64)
             assert_rel(f64(g), ref, 1e-2, "one call vs oracle")
             e_g, e_o = np.linalg.norm(f64(g) - ref), np.linalg.norm(f64(o) - ref)
-            assert e_g <= 2 * e_o, (e_g, e_o)
+            assert e_g <= 1.02 * e_o, (e_g, e_o)      # measured 0.989 to 1.004
         for a_, b_ in zip(one.layers, per_op.layers):
             assert_rel(f64(a_.ssm_state), f64(b_.ssm_state), 1e-2, "ssm_state")
             assert_rel(f64(a_.conv_state), f64(b_.conv_state), 2e-2, "conv_state")
