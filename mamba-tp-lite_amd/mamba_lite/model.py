@@ -249,8 +249,7 @@ def _no_global_hooks() -> bool:
 
 def _linear_mod(mod, x: torch.Tensor) -> torch.Tensor:
     """mod(x) of a projection; a plain nn.Linear without hooks may take ops.linear_f32."""
-    if _plain_modules(mod, (nn.Linear,)) and _no_global_hooks() and \
-            ops.linear_f32_ok(x, mod.weight, mod.bias):
+    if _plain_modules(mod, (nn.Linear,)) and _no_global_hooks() and ops.linear_f32_ok(x, mod.weight, mod.bias):
         return ops.linear_f32(x, mod.weight, mod.bias)
     return mod(x)
 
@@ -371,8 +370,9 @@ class MambaMixer(nn.Module):
         """prefill(); with parts_ok, out_proj of a short prefill may come back
         as _Parts (split-K partial products for the residual add to sum);
         skinny=False keeps every projection on torch's GEMMs."""
-        b, l, _ = x.shape
+        b, l, dm = x.shape
         Dm, N, R, K = self.cfg.d_inner, self.cfg.d_state, self.cfg.dt_rank, self.cfg.d_conv
+        bf16 = x.dtype == torch.bfloat16
         if out is not None:
             if tuple(out.conv_state.shape) != (b, Dm, K - 1) or out.conv_state.dtype != x.dtype or \
                     not out.conv_state.is_contiguous():
@@ -398,7 +398,8 @@ class MambaMixer(nn.Module):
                 z = F.linear(x, w_in[Dm:], b_in[Dm:] if b_in is not None else None).transpose(1, 2)
         else:
             xz = (ops.linear_skinny(x2, self.in_proj.weight, self.in_proj.bias).view(b, l, 2 * Dm) if x2 is not None
-                  else _linear_mod(self.in_proj, x))             # [b, l, 2D]
+                  else _linear_mod(self.in_proj, x) if ops.linear_f32_pays(b * l, 2 * Dm, dm)
+                  else self.in_proj(x))                          # [b, l, 2D]
             xs = xz[..., :Dm].transpose(1, 2)                    # [b, D, l] view, D-stride 1
             z = xz[..., Dm:].transpose(1, 2)
         conv_in_state = cache.conv_state if cache is not None else None
@@ -419,9 +420,10 @@ class MambaMixer(nn.Module):
         else:
             u_store = torch.empty(b, l, Dm, device=x.device, dtype=x.dtype)
             cw, cb = self.conv1d.weight, self.conv1d.bias
-            pbf = x.dtype == torch.bfloat16 and ops.bf16_params_ok(cw, cb)     # read as they are, no float copies
-            u, conv_state = ops.causal_conv1d(xs, cw if pbf else self._conv_w(), cb if pbf else _f32(cb),
-                                              conv_state=conv_in_state, silu=True, out=u_store.transpose(1, 2),
+            pbf = bf16 and ops.bf16_params_ok(cw, cb)            # read as they are, no float copies
+            cw, cb = (cw, cb) if pbf else (_f32(cw.reshape(cw.shape[0], cw.shape[-1])), _f32(cb))
+            u, conv_state = ops.causal_conv1d(xs, cw, cb, conv_state=conv_in_state, silu=True,
+                                              out=u_store.transpose(1, 2),
                                               final_state=out.conv_state if out is not None else None,
                                               bf16_params=pbf)
         w_x = self.x_proj.weight
@@ -458,7 +460,7 @@ class MambaMixer(nn.Module):
         y_store = torch.empty(b, l, Dm, device=x.device, dtype=x.dtype)
         # h_out may be h0 (mtl_selective_scan_fwd reads each state before it is overwritten)
         par = (self.A_log, self.D, self.dt_proj.bias)
-        pbf = x.dtype == torch.bfloat16 and ops.bf16_params_ok(*par)
+        pbf = bf16 and ops.bf16_params_ok(*par)
         A_log, Dv, dt_bias = par if pbf else map(_f32, par)
         _, h = ops.selective_scan(u, dt.transpose(1, 2), A_log, B, C, D=Dv, z=z, delta_bias=dt_bias, h0=h0,
                                   delta_softplus=True, a_is_log=True, y=y_store.transpose(1, 2),
@@ -470,7 +472,9 @@ class MambaMixer(nn.Module):
             if y2 is not None and Dm % (128 * SKINNY_OUT_SPLIT) == 0:
                 parts = ops.linear_skinny(y2, w_out, self.out_proj.bias, ksplit=SKINNY_OUT_SPLIT)
                 return _Parts(parts.view(SKINNY_OUT_SPLIT, b, l, -1)), conv_state, h
-        return _linear_mod(self.out_proj, y_store), conv_state, h
+        # (the sizes come first: a small eager call is bound by the host)
+        return (_linear_mod(self.out_proj, y_store) if ops.linear_f32_pays(b * l, dm, Dm)
+                else self.out_proj(y_store)), conv_state, h
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """No-cache forward (reference model.py:243-246)."""

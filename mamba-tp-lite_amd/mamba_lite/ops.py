@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 
 import torch
 import torch.nn.functional as F
@@ -133,6 +134,11 @@ def _bdl_layout_ok(*ts):
 SCAN_ALGOS = {"auto": 0, "tiled": 1, "chunked": 2}
 
 
+@functools.lru_cache(maxsize=4096)
+def _scan_ws_bytes(b, dim, dstate, seqlen):
+    return _lib.load().mtl_selective_scan_ws_bytes(b, dim, dstate, seqlen)
+
+
 def selective_scan(u, delta, A, B, C, D=None, z=None, delta_bias=None, h0=None, delta_softplus=True,
                    a_is_log=False, y=None, h_out=None, return_last_state=True, algo="auto", bf16_params=False):
     """Fused selective scan (mtl_selective_scan_fwd); see include/mtl.h.
@@ -196,7 +202,7 @@ def selective_scan(u, delta, A, B, C, D=None, z=None, delta_bias=None, h0=None, 
     p.dtype, p.delta_softplus, p.a_is_log = code, int(bool(delta_softplus)), int(bool(a_is_log))
     p.algo = SCAN_ALGOS[algo]
     lib = _lib.load()
-    nb = lib.mtl_selective_scan_ws_bytes(b, Dm, N, L) if p.algo == 0 else 0
+    nb = _scan_ws_bytes(b, Dm, N, L) if algo == "auto" else 0
     ws = None
     if nb:
         try:
@@ -913,6 +919,7 @@ def decode_gemv(v, W, out, bias=None, x_in=None):
     return out
 
 
+@functools.lru_cache(maxsize=4096)
 def linear_f32_pays(M: int, N: int, K: int) -> bool:
     """Where mtl_linear_f32 (the splits of x and W included) beats the library's fp32 GEMM."""
     return bool(_lib.load().mtl_linear_f32_pays(M, N, K))
@@ -926,7 +933,7 @@ def linear_f32_ok(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
             x.dim() < 2 or W.dim() != 2 or not x.is_contiguous() or W.stride(1) != 1 or x.shape[-1] != W.shape[1]:
         return False
     N, K = W.shape
-    if x.numel() == 0 or not linear_f32_pays(x.numel() // K, N, K) or N >= 1 << 21 or W.stride(0) < K:
+    if K == 0 or not linear_f32_pays(x.numel() // K, N, K) or N >= 1 << 21 or W.stride(0) < K:
         return False
     if bias is not None and (bias.dtype != torch.float32 or bias.device != x.device or not bias.is_contiguous() or
                              tuple(bias.shape) != (N,)):
