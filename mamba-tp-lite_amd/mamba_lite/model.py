@@ -880,7 +880,7 @@ class MambaLM(nn.Module):
         nl = len(self.layers)
         act = x.dtype
         if x.dim() != 2 or act not in (torch.float32, torch.bfloat16) or not x.is_cuda or not x.is_contiguous() or \
-                x.data_ptr() % 16 or len(cache.layers) != nl or act == torch.bfloat16 and not self._plain_stack():
+                x.data_ptr() % 16 or len(cache.layers) != nl:
             return None
         b, dm = x.shape
         D, N, K, R = cfg.d_inner, cfg.d_state, cfg.d_conv, cfg.dt_rank
@@ -888,6 +888,8 @@ class MambaLM(nn.Module):
         fits = dm >= 256 and D % (128 * SKINNY_OUT_SPLIT) == 0 if act == torch.float32 else \
             dm >= 512 and D >= 1024 and D % (64 * SKINNY_OUT_SPLIT) == 0
         if not (1 <= b <= ops.IN_CONV_MAX_ROWS and fits and dm % 128 == 0 and N <= 16 and R <= 256 and 2 <= K <= 4 and R + 2 * N <= 288):
+            return None
+        if act == torch.bfloat16 and not self._plain_stack():        # (after the sizes: it walks every module)
             return None
         dev = x.device
         nf = self.norm_f.weight           # (not in the template: norm_f may be cast or replaced between steps)

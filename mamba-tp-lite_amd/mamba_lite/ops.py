@@ -961,6 +961,11 @@ def _plain_forward(*ts) -> bool:
         not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
 
 
+@functools.lru_cache(maxsize=4096)
+def _lm_head_sizes(M, N, K, code) -> bool:
+    return bool(_lib.load().mtl_lm_head_ok(M, N, K, code))
+
+
 def lm_head_ok(x: torch.Tensor, W: torch.Tensor) -> bool:
     """Whether lm_head takes F.linear(x, W) in its place: a decode step's rows
     against a wide, contiguous vocabulary matrix of x's type."""
@@ -968,9 +973,8 @@ def lm_head_ok(x: torch.Tensor, W: torch.Tensor) -> bool:
             W.dim() != 2 or x.shape[-1] != W.shape[1] or not x.is_contiguous() or not W.is_contiguous():
         return False
     N, K = W.shape
-    M = x.numel() // K if K else 0
-    return M <= 16 and _plain_forward(x, W) and aligned16(x, W) and \
-        bool(_lib.load().mtl_lm_head_ok(M, N, K, _ACT_DTYPES[x.dtype]))
+    return K > 0 and _lm_head_sizes(x.numel() // K, N, K, _ACT_DTYPES[x.dtype]) and _plain_forward(x, W) and \
+        aligned16(x, W)
 
 
 def lm_head(x, W):

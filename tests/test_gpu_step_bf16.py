@@ -156,6 +156,17 @@ def test_a_model_made_in_inference_mode(l):
         assert not torch.equal(lm.step(ids, cache) if l == 1 else lm.prefill(ids)[0], got)
 
 
+def test_a_step_the_sizes_rule_out_walks_no_modules(monkeypatch):
+    """A bf16 step of a model too narrow for the one call is bound by the host: its modules are not looked through."""
+    with torch.device("cuda"):
+        lm = MambaLM(MambaConfig(d_model=256, n_layer=2, vocab_size=300)).eval().to(torch.bfloat16)
+    walked = []
+    monkeypatch.setattr(MambaLM, "_plain_stack", lambda self: walked.append(1))
+    with torch.no_grad():
+        lm.step(torch.zeros(3, 1, dtype=torch.long, device="cuda"), MambaCache.allocate(lm.cfg, 3, "cuda", torch.bfloat16))
+    assert not walked
+
+
 class _Negating(torch.nn.Linear):
     def forward(self, x):
         return -super().forward(x)
