@@ -164,9 +164,9 @@ struct SplitJob {
 // flight at a time (both operands of a product, us): in_proj + out_proj of 32768
 // tokens at d_model 768 153 -> 114 (5.5 TB/s at K = 1536), of 1024 tokens at
 // 2048 70 -> 55, the lm_head's 999 + 50280 rows of 768 74 -> 52.  16 units take
-// 160 VGPRs (3 wavefronts a SIMD), 32 would spill.  Beside the norm (below)
+// 167 VGPRs (3 wavefronts a SIMD), 32 would spill.  Beside the norm (below)
 // the weight's workgroups are few and keep two passes: 10.2 us either way at
-// 999 + 3072 x 768.
+// 999 + 3072 x 768, 11.0 since the rows' counts (split_ok) are taken.
 template <int NT, int U>
 __device__ __forceinline__ void split_block(const SplitJob& j, int64_t block) {
     constexpr int NW = NT / 64, UR = U > 0 ? U : 1;

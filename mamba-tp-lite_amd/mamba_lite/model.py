@@ -239,7 +239,8 @@ def _plain_modules(mod, types) -> bool:
     replaced forward, and their parameters no tensor subclass, all of which a raw launch would skip."""
     d = mod.__dict__
     return type(mod) in types and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d) and \
-        all(p is None or type(p) in ops.PLAIN_TENSORS for p in d["_parameters"].values()) and all(m is None or _plain_modules(m, types) for m in d["_modules"].values())
+        all(p is None or type(p) in ops.PLAIN_TENSORS for p in d["_parameters"].values()) and \
+        all(m is None or _plain_modules(m, types) for m in d["_modules"].values())
 
 
 def _no_global_hooks() -> bool:

@@ -650,7 +650,8 @@ def prefill_long(h, layers, norm_f, eps_f, d_inner, d_state, dt_rank, d_conv, sk
     blas_ws = max([PREFILL_LONG_BLAS_WS] + [lib.mtl_linear_f32_ws_bytes(rows, n, k)
                                             for n, k in ((2 * d_inner, M), (M, d_inner)) if linear_f32_pays(rows, n, k)])
     offs, n = [], 0
-    for sz in (rows * M, rows * 2 * d_inner, rows * d_inner, rows * J, rows * d_inner, rows * d_inner, rows * M, rows * M):
+    for sz in (rows * M, rows * 2 * d_inner, rows * d_inner, rows * J, rows * d_inner, rows * d_inner, rows * M,
+               rows * M):
         offs.append(n)
         n += -(-sz // 64) * 64
     alloc = lambda: torch.empty(n + -(-blas_ws // 4), device=h.device, dtype=torch.float32)
@@ -950,8 +951,8 @@ def _no_function_mode() -> bool:
 def plain_call() -> bool:
     """No autocast, functorch or forward-mode transform, tracing, function or dispatch mode that a raw launch would
     bypass."""
-    return _no_function_mode() and not torch.is_autocast_enabled("cuda") and torch.autograd.forward_ad._current_level < 0 and \
-        torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0 and \
+    return _no_function_mode() and not torch.is_autocast_enabled("cuda") and \
+        torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0 and \
         not torch.jit.is_tracing() and not torch.compiler.is_compiling()
 
 

@@ -1,7 +1,8 @@
-"""mtl_decode_step_batched on a bfloat16 model (weights, activations and conv
+"""mtl_decode_step_batched_bf16 on a bfloat16 model (weights, activations and conv
 history in bf16; fp32 residual, SSM state and partial sums): MambaLM.step
 (model.py:343-353) at 1-32 rows against the float64 oracle and the per-op
-step, and captured."""
+step, and captured; the models and states that keep it, and a long fp32
+prompt's one call, on the per-op path; models copied and saved after calls."""
 import copy
 import io
 
@@ -163,7 +164,8 @@ def test_a_step_the_sizes_rule_out_walks_no_modules(monkeypatch):
     walked = []
     monkeypatch.setattr(MambaLM, "_plain_stack", lambda self: walked.append(1))
     with torch.no_grad():
-        lm.step(torch.zeros(3, 1, dtype=torch.long, device="cuda"), MambaCache.allocate(lm.cfg, 3, "cuda", torch.bfloat16))
+        lm.step(torch.zeros(3, 1, dtype=torch.long, device="cuda"),
+                MambaCache.allocate(lm.cfg, 3, "cuda", torch.bfloat16))
     assert not walked
 
 
